@@ -98,23 +98,6 @@ __device__ __forceinline__ bf4 conv_in4(const ConvArgs& A, int n, int hh, int ww
   return *(const bf4*)(A.xb + (((size_t)n * A.H + hh) * A.W + ww) * A.cb + (c0 - A.ca));
 }
 
-// One input channel c of pixel p shifted by tap t (zero outside the grid).
-__device__ __forceinline__ float conv_in1(const ConvArgs& A, int p, int t, int c) {
-  const int HW = A.H * A.W, n = p / HW, rem = p % HW;
-  const int hh = rem / A.W + t / 3 - 1, ww = rem % A.W + t % 3 - 1;
-  if (hh < 0 || hh >= A.H || ww < 0 || ww >= A.W) return 0.0f;
-  if (A.mode == kPlain) return bf2f(A.xa[(((size_t)n * A.H + hh) * A.W + ww) * A.ca + c]);
-  if (A.mode == kPool) {
-    const size_t W2 = 2 * (size_t)A.W;
-    const size_t b = (((size_t)n * 2 * A.H + 2 * hh) * W2 + 2 * ww) * A.ca + c;
-    return bf2f(f2bf((bf2f(A.xa[b]) + bf2f(A.xa[b + A.ca]) + bf2f(A.xa[b + W2 * A.ca]) +
-                      bf2f(A.xa[b + (W2 + 1) * A.ca])) *
-                     0.25f));
-  }
-  if (c < A.ca) return bf2f(A.xa[(((size_t)n * (A.H / 2) + hh / 2) * (A.W / 2) + ww / 2) * A.ca + c]);
-  return bf2f(A.xb[(((size_t)n * A.H + hh) * A.W + ww) * A.cb + (c - A.ca)]);
-}
-
 // Forward (and input-gradient) 3x3 convolution: each wave computes NT output
 // tiles of 16 channels (from tile NT * blockIdx.y on; cout = 16 * NT *
 // gridDim.y) for 16 pixels, over CB = cin / 16 input-channel blocks, fully
@@ -176,9 +159,25 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A) {
 constexpr int kWgradParts = 256;
 
 // Weight gradient dW[t][o][i] = sum_p x(p + tap t)[i] dpre(p)[o]: GEMM with
-// M = output channels, N = input channels, K = pixels.  Block (gx, gy): pixel
-// chunks of 64 in the range of gx, 16 (tap, o-tile, i-tile) combinations of gy
-// (4 per wave).  Partials per gx, reduced by k_wgrad_reduce.
+// M = output channels, N = input channels, K = pixels.  Block (gx, gy, gz):
+// the pixel range of gx in steps of kWgPixels, the 16 input channels of gy,
+// the three taps of kernel row gz and every output tile (wave w takes the
+// (tap, o-tile) pairs w, w + 4, ...).  Partials per gx, reduced by
+// k_wgrad_reduce.
+//
+// The matrix cores want four consecutive pixels of one channel per lane, the
+// activations hold the channels of one pixel together.  A step is therefore
+// transposed once into LDS, as three shifted copies of its input channels and
+// the output gradients: a thread loads 4 pixels x 4 channels as 8-byte loads,
+// transposes them in registers and writes 8-byte rows, and the operands are
+// 8-byte LDS reads.  The row pitch (8 banks past a multiple of 64) spreads the
+// 16 rows x 4 pixel groups that a wave reads evenly over the banks.  What
+// bounds it is the latency of a step (load, two barriers, transposes), so a
+// step takes as many pixels as a block's range usually has (4 chunks of 64),
+// and the kernel rows go to different blocks.  Measured for a batch of 16
+// samples of 64 x 64: 7-14 us per layer instead of 85-98 us when the lanes
+// gathered their operands from global memory two bytes at a time (the sums are
+// the same, bit for bit); 64-pixel steps with all nine taps: 14-29 us.
 struct WgradArgs {
   ConvArgs X;            // the layer's input (mode, channels, resolution)
   const uint16_t* dp;    // dpre [N][H][W][cout]
@@ -186,63 +185,116 @@ struct WgradArgs {
   float* part;           // [gridDim.x][9][cout][cin]
 };
 
+constexpr int kWgPixels = 256;             // pixels per step: 4 per (thread / 4)
+constexpr int kWgPitch = kWgPixels + 16;   // LDS row of one channel, padded
+
+// rows v[pixel][channel] to t[channel][pixel], four of each
+__device__ __forceinline__ void transpose4(const bf4 (&v)[4], bf4 (&t)[4]) {
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) t[c][e] = v[e][c];
+}
+
+template <int MODE, int NM>
 __global__ void __launch_bounds__(256) k_wgrad(WgradArgs A) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ __align__(16) uint16_t s_x[3 * 16 * kWgPitch];
+  __shared__ __align__(16) uint16_t s_d[NM * 16 * kWgPitch];
+  constexpr int cout = 16 * NM, NC = (3 * NM + 3) / 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int kg = lane >> 4, col = lane & 15;
+  const int pq = tid >> 2, cq = tid & 3;  // this thread's pixel and channel quads
   const ConvArgs& X = A.X;
-  const int cin = X.mode == kUpCat ? X.ca + X.cb : X.ca;
-  const int nm = A.cout / 16, nn = cin / 16, ncombo = 9 * nm * nn;
-  const int cbase = (blockIdx.y * 4 + wave) * 4;
-  if (cbase >= ncombo) return;  // whole wave
-  int tap[4], m0[4], n0[4];
-  bool act[4];
+  const int cin = MODE == kUpCat ? X.ca + X.cb : X.ca;
+  const int n0 = blockIdx.y * 16, row = blockIdx.z, HW = X.H * X.W;
+  f4 acc[NC];
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int c = cbase + j;
-    act[j] = c < ncombo;
-    const int cc = act[j] ? c : 0;
-    tap[j] = cc / (nm * nn);
-    m0[j] = (cc / nn) % nm * 16;
-    n0[j] = cc % nn * 16;
-  }
-  f4 acc[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) acc[j] = (f4){0.f, 0.f, 0.f, 0.f};
-  const int total = X.N * X.H * X.W, chunks = (total + 63) / 64;
+  for (int j = 0; j < NC; j++) acc[j] = (f4){0.f, 0.f, 0.f, 0.f};
+  const int total = X.N * HW, chunks = (total + 63) / 64;
   const int per = (chunks + gridDim.x - 1) / gridDim.x;
-  const int ch0 = blockIdx.x * per, ch1 = min(chunks, ch0 + per);
-  for (int ch = ch0; ch < ch1; ch++)
-    for (int ks = 0; ks < 4; ks++) {
-      const int k0 = ch * 64 + ks * 16 + 4 * kg;
+  const int pend = min(total, ((int)blockIdx.x + 1) * per * 64);  // the range's end
+  for (int ps = blockIdx.x * per * 64; ps < pend; ps += kWgPixels) {
+    const int p0 = ps + 4 * pq;
+    bf4 x[3][4], d[NM][4], t[4];
+    int n = p0 / HW, h = p0 % HW / X.W, w = p0 % HW % X.W;
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if (!act[j]) continue;
-        bf4 a, b;
+    for (int e = 0; e < 4; e++) {
+      const int hh = h + row - 1;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int p = k0 + e;
-          const bool in = p < total;
-          a[e] = in ? (short)A.dp[(size_t)p * A.cout + m0[j] + col] : (short)0;
-          b[e] = in ? (short)f2bf(conv_in1(X, p, tap[j], n0[j] + col)) : (short)0;
+      for (int k = 0; k < 3; k++) {
+        const int ww = w + k - 1;
+        const bool in = p0 + e < pend && hh >= 0 && hh < X.H && ww >= 0 && ww < X.W;
+        x[k][e] = in ? conv_in4<MODE>(X, n, hh, ww, n0 + 4 * cq) : (bf4){0, 0, 0, 0};
+      }
+      const bool in = p0 + e < pend;
+#pragma unroll
+      for (int m = 0; m < NM; m++)
+        d[m][e] = in ? *(const bf4*)(A.dp + (size_t)(p0 + e) * cout + 16 * m + 4 * cq)
+                     : (bf4){0, 0, 0, 0};
+      if (++w == X.W) {  // the next pixel in order
+        w = 0;
+        if (++h == X.H) {
+          h = 0;
+          n++;
         }
+      }
+    }
+    __syncthreads();  // the previous step's operands have been read
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      transpose4(x[k], t);
+#pragma unroll
+      for (int c = 0; c < 4; c++) *(bf4*)(s_x + (k * 16 + 4 * cq + c) * kWgPitch + 4 * pq) = t[c];
+    }
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+      transpose4(d[m], t);
+#pragma unroll
+      for (int c = 0; c < 4; c++) *(bf4*)(s_d + (m * 16 + 4 * cq + c) * kWgPitch + 4 * pq) = t[c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+      const int c = wave + 4 * j;
+      if (c >= 3 * NM) break;
+      const int k = c / NM, m = c % NM;
+      for (int ks = 0; ks < kWgPixels / 16; ks++) {
+        const bf4 a = *(const bf4*)(s_d + (m * 16 + col) * kWgPitch + ks * 16 + 4 * kg);
+        const bf4 b = *(const bf4*)(s_x + (k * 16 + col) * kWgPitch + ks * 16 + 4 * kg);
         acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[j], 0, 0, 0);
       }
     }
-  float* out = A.part + (size_t)blockIdx.x * 9 * A.cout * cin;
+  }
+  float* out = A.part + (size_t)blockIdx.x * 9 * cout * cin;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    if (!act[j]) continue;
+  for (int j = 0; j < NC; j++) {
+    const int c = wave + 4 * j;
+    if (c >= 3 * NM) break;
+    const int tap = 3 * row + c / NM, m = c % NM;
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      out[((size_t)tap[j] * A.cout + m0[j] + 4 * kg + i) * cin + n0[j] + col] = acc[j][i];
+      out[((size_t)tap * cout + m * 16 + 4 * kg + i) * cin + n0 + col] = acc[j][i];
   }
 }
 
+// Sum of the ranges' partials in their order.  The chain of additions is
+// serial, the loads need not be: kWgReduceBatch of them are in flight at a
+// time (5 us for the 256 ranges of a full-resolution layer at batch 16; one by
+// one they took 58 us).
+constexpr int kWgReduceBatch = 32;
 __global__ void k_wgrad_reduce(const float* part, int nparts, int len, float* g) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= len) return;
   float s = 0.0f;
-  for (int k = 0; k < nparts; k++) s += part[(size_t)k * len + i];
+  int k = 0;
+  for (; k + kWgReduceBatch <= nparts; k += kWgReduceBatch) {
+    float v[kWgReduceBatch];
+#pragma unroll
+    for (int b = 0; b < kWgReduceBatch; b++) v[b] = part[(size_t)(k + b) * len + i];
+#pragma unroll
+    for (int b = 0; b < kWgReduceBatch; b++) s += v[b];
+  }
+  for (; k < nparts; k++) s += part[(size_t)k * len + i];
   g[i] = s;
 }
 
@@ -492,10 +544,16 @@ __global__ void k_nn_store(MgLevel L, int H, int W, float* out) {
   X(kUpCat, 1, 3) X(kPlain, 1, 3) X(kPlain, 1, 4) X(kPool, 1, 1) X(kPool, 1, 2)        \
   X(kPool, 1, 3) X(kUpCat, 1, 5) X(kUpCat, 1, 7)
 
-// split: one output tile per wave, the tiles along the grid's y (the
-// network application); otherwise every tile in each wave (training batches).
+// split: one output tile per wave, the tiles along the grid's y (the network
+// application, and the layers of a batch with at most kSplitPixels pixels);
+// otherwise every tile in each wave.  Measured at batch 16: the 64-channel
+// layers at 8 x 8 (1024 pixels) 22.6 -> 10 us, 48 channels at 16 x 16 9.1 -> 6 us,
+// 32 channels at 32 x 32 (16384 pixels) 8.4 -> 6.8 us; at 64 x 64 the layers
+// have one or three tiles and fill the chip either way.
+constexpr int kSplitPixels = 16384;
 int launch_conv(const ConvArgs& a, hipStream_t st, bool split = false) {
   const int total = a.N * a.H * a.W;
+  split = split || total <= kSplitPixels;
   const int ntile = a.cout / 16, cb = (a.mode == kUpCat ? a.ca + a.cb : a.ca) / 16;
   const int nt = split ? 1 : ntile;
   const dim3 g((total + 63) / 64, split ? ntile : 1), b(256);
@@ -537,24 +595,39 @@ int forward(const Net* net, const Acts& a, hipStream_t st, bool split = false) {
 
 int ceil_div(size_t a, size_t b) { return (int)((a + b - 1) / b); }
 
+template <int MODE>
+int launch_wgrad(const WgradArgs& w, dim3 g, hipStream_t st) {
+  switch (w.cout / 16) {
+    case 1: hipLaunchKernelGGL((k_wgrad<MODE, 1>), g, dim3(256), 0, st, w); return 0;
+    case 2: hipLaunchKernelGGL((k_wgrad<MODE, 2>), g, dim3(256), 0, st, w); return 0;
+    case 3: hipLaunchKernelGGL((k_wgrad<MODE, 3>), g, dim3(256), 0, st, w); return 0;
+    case 4: hipLaunchKernelGGL((k_wgrad<MODE, 4>), g, dim3(256), 0, st, w); return 0;
+  }
+  return -1;
+}
+
 // dW of layer l into net->g, from a.dpre[l].
-void wgrad(Net* net, const Acts& a, int l, hipStream_t st) {
+int wgrad(Net* net, const Acts& a, int l, hipStream_t st) {
   WgradArgs w;
   w.X = fwd_args(net, a, l);
   w.dp = a.dpre[l];
   w.cout = kNet[l].cout;
   w.part = net->wpart;
   const int cin = layer_cin(l), len = 9 * w.cout * cin;
-  const int ncombo = 9 * (w.cout / 16) * (cin / 16);
   const int total = a.N * (a.H >> kNet[l].level) * (a.W >> kNet[l].level);
   // pixel chunks of 64, at least 4 per block, at most kWgradParts blocks along x
   int gx = ceil_div(total, 64 * 4);
   const int cap = (int)(net->wpart_len / (size_t)len);
   gx = gx < 1 ? 1 : gx > kWgradParts ? kWgradParts : gx;
   if (gx > cap) gx = cap;
-  hipLaunchKernelGGL(k_wgrad, dim3(gx, ceil_div(ncombo, 16)), dim3(256), 0, st, w);
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(len, 256)), dim3(256), 0, st, net->wpart, gx,
+  const dim3 g(gx, cin / 16, 3);
+  if (w.X.mode == kPlain ? launch_wgrad<kPlain>(w, g, st)
+      : w.X.mode == kPool ? launch_wgrad<kPool>(w, g, st)
+                          : launch_wgrad<kUpCat>(w, g, st))
+    return -1;
+  hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(len, 64)), dim3(64), 0, st, net->wpart, gx,
                      len, net->g + net->off[l]);
+  return 0;
 }
 
 // Input gradient of layer l (l > 0): masked BF16 into dpre[l - 1] for plain
@@ -615,7 +688,7 @@ int backward(Net* net, const Acts& a, hipStream_t st) {
     offc += (size_t)a.N * (a.H >> lv) * (a.W >> lv) * layer_cin(l);
   }
   for (int l = kLayers - 1; l >= 0; l--) {
-    wgrad(net, a, l, st);
+    if (wgrad(net, a, l, st)) return -1;
     if (l == 0) break;
     const LayerDesc& L = kNet[l];
     if (L.mode == kPlain) {

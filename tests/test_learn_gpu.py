@@ -91,6 +91,31 @@ def test_application_launch_shape_equals_training_shape(H, W):
     assert np.abs(out1).max() > 0
 
 
+@pytest.mark.parametrize("B,H,W", [(2, 8, 8), (4, 24, 40), (8, 40, 24), (4, 64, 64)])
+def test_weight_gradient_of_a_batch_is_the_mean_of_its_samples(B, H, W):
+    """The weight-gradient kernel takes 4-pixel groups in steps of 256 pixels
+    over ranges of the batch: single samples and batches cut the same pixels
+    differently (groups that straddle rows and samples at the 1 x 1, 3 x 5 and
+    5 x 3 deepest levels, partial steps, several ranges at 64 x 64).  With a
+    power-of-two batch the pre-activation gradients scale exactly, so only the
+    FP32 summation order differs: n <= 2^14 products, sqrt(n) 2^-24 = 8e-6,
+    bound 4e-5."""
+    from fluidsim_amd.learn import LearnedPreconditioner
+
+    rng = np.random.default_rng(23)
+    net = LearnedPreconditioner(0, 8, 8, seed=9)
+    in5, rhat, op = _batch(rng, B, H, W)
+    loss, grad, out = net.loss_grad(in5, rhat, op)
+    one = [net.loss_grad(in5[b:b + 1], rhat[b:b + 1], op[b:b + 1]) for b in range(B)]
+    assert all(np.array_equal(out[b], one[b][2][0]) for b in range(B))
+    assert loss == pytest.approx(np.mean([o[0] for o in one]), rel=1e-6)
+    mean = np.mean([o[1].astype(np.float64) for o in one], axis=0)
+    off, n = U.offsets()
+    for l in range(15):
+        hi = off[l + 1] if l < 14 else n
+        assert rel_l2(grad[off[l]:hi], mean[off[l]:hi]) <= 4e-5, l
+
+
 def _harvested(nx=64, steps=24, seed=0):
     from fluidsim_amd import Discharge, configs
     from fluidsim_amd.learn import LearnedPreconditioner
