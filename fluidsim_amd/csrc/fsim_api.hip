@@ -954,13 +954,20 @@ int ensure_mg_graphs(fs_handle* h) {
   return 0;
 }
 
-// Multigrid-PCG with graphs can be issued ahead of the host: after the
-// controller's kernel (mode 1) the assembly, the set-up and the first chunk
-// with its finishing kernels are enqueued, the assembly skipping the whole
-// solve on the device unless the attempt is accepted; after the host has read
-// the scalars, mode 2 continues that solve.  Mode 0: a whole solve.
+// The Jacobi-PCG solve of a small system as one launch (k_pcg_small).
+bool small_jacobi(const fs_handle* h) {
+  return h->p.lapl_solver != 2 && !(h->p.lapl_solver == 1 && h->mg.size() > 1) &&
+         pcg_small_fits(h->G);
+}
+
+// Multigrid-PCG with graphs, and the one-launch Jacobi-PCG, can be issued
+// ahead of the host: after the controller's kernel (mode 1) the assembly, the
+// set-up and the first chunk with its finishing kernels (or the whole small
+// solve) are enqueued, the assembly skipping the solve on the device unless
+// the attempt is accepted; after the host has read the scalars, mode 2
+// continues that solve.  Mode 0: a whole solve.
 bool can_issue_ahead(const fs_handle* h) {
-  return h->p.use_graphs && h->p.lapl_solver == 1 && h->mg.size() > 1;
+  return small_jacobi(h) || (h->p.use_graphs && h->p.lapl_solver == 1 && h->mg.size() > 1);
 }
 
 int lapl_solve_impl(fs_handle* h, int* lerr, fs_solve_stats* stats, int mode = 0) {
@@ -1060,6 +1067,14 @@ int lapl_solve_impl(fs_handle* h, int* lerr, fs_solve_stats* stats, int mode = 0
       mg_it += mg_chunk;
       mg_chunk = chunk > 8 ? chunk / 4 : chunk;
       if (int e = end_chunk()) return e;
+    }
+  } else if (small_jacobi(h)) {
+    if (mode != 2) {
+      launch_pcg_small(pa, h->st);
+      HIP_OK(hipGetLastError());
+      time_mark(h, 6);
+      if (mode == 1) return 0;
+      if (sync_scalars(h)) return FS_E_HIP;
     }
   } else {
     PcgArgs ia = pcg_args(h, 0);

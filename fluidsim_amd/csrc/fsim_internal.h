@@ -336,6 +336,9 @@ void launch_lapl_assemble(const LaplArgs* a, const FsPhys* K, int nblocks, hipSt
 void launch_pcg_init(const PcgArgs& a, hipStream_t s);
 void launch_pcg_it(const PcgArgs& a, hipStream_t s);
 void launch_pcg_finish(const PcgArgs& a, hipStream_t s);
+// the Jacobi-PCG solve of a system that fits one workgroup
+bool pcg_small_fits(const Geo& G);
+void launch_pcg_small(const PcgArgs& a, hipStream_t s);
 void launch_mg_coarsen(const MgArgs& a, hipStream_t s);
 int mg_grid(const MgLevel& F);  // blocks (= partials) of a down/up launch
 void launch_mg_down(const MgArgs& a, hipStream_t s);

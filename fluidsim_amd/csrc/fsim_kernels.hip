@@ -33,6 +33,7 @@ constexpr int kNF = kNFX > kNFY ? kNFX : kNFY;
 // its face buffer s_f[4][kNF]
 static_assert(3 * (kSNT + kSNT / 4 + kSNT / 16 + kSNT / 64) <= 4 * kNF, "assembly LDS levels");
 constexpr int kNW = kNT / 64;
+constexpr int kPcgSmallPlane = 5120;  // LDS doubles of k_pcg_small's padded plane (two dimensions)
 constexpr int kSNW = kSNT / 64;
 
 // The stage kernel's tile: kTX x TY cells (TY = 4, 8 or 16, chosen per grid by
@@ -1413,6 +1414,196 @@ __device__ __forceinline__ void pcg_tres_body(const PcgArgs& A, int nb) {
 }
 
 __global__ void __launch_bounds__(kNT) k_pcg_tres(PcgArgs A, int nb) { pcg_tres_body<0>(A, nb); }
+
+// A whole Jacobi-PCG solve in one workgroup, for systems whose cells fit its
+// registers: k_pcg_init, the iterations of k_pcg_it, k_pcg_finish and
+// k_pcg_tres in one launch.  Such a system is bound by latency: as a launch per
+// iteration it costs 6-8 us each (3.4 us of kernel, the rest launch and host),
+// here an iteration is two barriers, an LDS exchange of u = r / d and three
+// wave reductions, about 1 us.  Measured: a pass of the 40-cell default
+// discharge (40 iterations) 430 -> 117 us.
+//
+// Every value is the one the launches compute, bit for bit: the same
+// expressions, and sums over the same tiles in the same order (a tile's
+// threads by wave trees and then its waves in order, the tiles by one wave's
+// tree).  The tiles are those of the launches, 64 x 8 cells with two cells per
+// thread of 256; in one dimension (kOneD) a tile has one row, so a wave takes
+// a tile of its own.  Thread t holds the cells of tiles (t / 256) + NTH / 256 q
+// (one dimension: t / 64 + NTH / 64 q), q < S.
+template <bool kOneD, int NTH, int S>
+__global__ void __launch_bounds__(NTH) k_pcg_small(PcgArgs A) {
+  constexpr int C = kOneD ? S : S * kPcgRows;  // cells per thread
+  constexpr int kTpb = kOneD ? 64 : kNT;       // threads per tile
+  constexpr int kTiles = NTH / kTpb * S;       // tiles the workgroup holds (at most 64)
+  constexpr int kWpt = kTpb / 64;              // waves per tile
+  constexpr int kPlane = kOneD ? kTX * kTiles + 2 : kPcgSmallPlane;
+  static_assert(kTiles <= 64, "one wave sums the tiles' partials");
+  __shared__ double s_u[kPlane];  // padded as the planes: (nx + 2) x (ny + 2)
+  __shared__ double s_w[kTiles * kWpt][3];
+  DevScalars* sc = A.sc;
+  // the assembly's gate (no solve), or its error (the host stops on it)
+  if (sc->done || sc->status < 0) return;
+  const Geo& G = A.G;
+  const int P = G.P, nt = A.nbx * A.nby, t = threadIdx.x;
+  const double tol = sc->tol;
+  const int maxit = sc->maxit;
+  double r[C], w[C], so[C], p[C], d[C], cl[C], cr[C], cb[C], ct[C], u[C];
+  // x and the volumes: in registers, or, for four cells in two dimensions,
+  // which would not fit 128 VGPRs, in this thread's own places in LDS
+  constexpr bool kOwnLds = !kOneD && S == 2;
+  __shared__ double s_own[kOwnLds ? 2 * C * NTH : 1];
+  double own[kOwnLds ? 1 : 2 * C];
+  auto x = [&](int c) -> double& { return kOwnLds ? s_own[c * NTH + t] : own[c]; };
+  auto vol = [&](int c) -> double& { return kOwnLds ? s_own[(C + c) * NTH + t] : own[C + c]; };
+  int k[C];  // index in s_u, 0 (a ghost) for a slot without a cell
+#pragma unroll
+  for (int c = 0; c < C; c++) {
+    const int tile = t / kTpb + NTH / kTpb * (kOneD ? c : c / kPcgRows);
+    const int ci = (tile % A.nbx) * kTX + t % kTX;
+    const int cj = kOneD ? 0
+                         : (tile / A.nbx) * kPcgTY + t % kTpb / kTX +
+                               (c % kPcgRows) * (kPcgTY / kPcgRows);
+    const bool in = tile < nt && ci < G.bx && cj < G.by;
+    const size_t m = in ? (size_t)(cj + 1) * P + (ci + 1) : 0;
+    k[c] = in ? (kOneD ? ci + 1 : (int)m) : 0;
+    r[c] = in ? A.r_old[m] : 0.0;
+    d[c] = in ? A.dg[m] : 1.0;
+    cl[c] = in ? A.cx[m - 1] : 0.0;
+    cr[c] = in ? A.cx[m] : 0.0;
+    cb[c] = in && !kOneD ? A.cy[m - P] : 0.0;
+    ct[c] = in && !kOneD ? A.cy[m] : 0.0;
+    vol(c) = in ? G.dlx[ci] * G.dly[cj] * (G.cyl ? G.r[cj + 1] : 1.0) : 1.0;
+    so[c] = p[c] = x(c) = 0.0;
+    u[c] = r[c] / d[c];
+  }
+  for (int q = t; q < kPlane; q += NTH) s_u[q] = 0.0;
+  __syncthreads();
+  // v at this thread's cells into LDS, then M v there
+  auto exchange = [&](auto v) {
+#pragma unroll
+    for (int c = 0; c < C; c++)
+      if (k[c]) s_u[k[c]] = v(c);
+    __syncthreads();
+  };
+  auto uc = [&](int c) { return u[c]; };
+  auto mul = [&](double v, int c) {
+    if (!k[c]) return 0.0;
+    double y = d[c] * v - cl[c] * s_u[k[c] - 1] - cr[c] * s_u[k[c] + 1];
+    if (!kOneD) y = y - cb[c] * s_u[k[c] - P] - ct[c] * s_u[k[c] + P];
+    return y;
+  };
+  // the sums over all cells of per-cell terms (f0, f1, f2)
+  auto total3 = [&](auto term, double (&tot)[3]) {
+#pragma unroll
+    for (int q = 0; q < S; q++) {
+      double acc[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int e = 0; e < C / S; e++) {
+        const int c = q * (C / S) + e;
+        if (!k[c]) continue;
+        double f[3];
+        term(c, f);
+        acc[0] += f[0];
+        acc[1] += f[1];
+        acc[2] += f[2];
+      }
+#pragma unroll
+      for (int v = 0; v < 3; v++)
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) acc[v] += __shfl_down(acc[v], off, 64);
+      const int slot = (t / kTpb + NTH / kTpb * q) * kWpt + t % kTpb / 64;
+      if ((t & 63) == 0)
+#pragma unroll
+        for (int v = 0; v < 3; v++) s_w[slot][v] = acc[v];
+    }
+    __syncthreads();
+    // partial b is that of the tile block b of a launch takes
+    const int b = t & 63, tb = b < nt ? xcd_tile(b, nt) : 0;
+#pragma unroll
+    for (int v = 0; v < 3; v++) {
+      double a = 0.0;
+      if (b < nt) {
+        a = s_w[tb * kWpt][v];
+        for (int q = 1; q < kWpt; q++) a += s_w[tb * kWpt + q][v];
+      }
+      // (the tree's wider steps only add zeros)
+#pragma unroll
+      for (int off = kTiles / 2; off > 0; off >>= 1) a += __shfl_down(a, off, 64);
+      tot[v] = __shfl(a, 0, 64);
+    }
+  };
+  exchange(uc);
+#pragma unroll
+  for (int c = 0; c < C; c++) w[c] = mul(u[c], c);
+  double tot[3];
+  auto terms = [&](int c, double (&f)[3]) {
+    const double rv = r[c] / vol(c);
+    f[0] = r[c] * u[c];
+    f[1] = w[c] * u[c];
+    f[2] = rv * rv;
+  };
+  total3(terms, tot);
+  const double bnorm2 = tot[2];
+  double gam_old = 1.0, alpha_old = 1.0, res = 0.0;
+  int done = 0, it = 0;
+  for (;; it++) {  // (ends: it reaches maxit at the latest)
+    const double gam = tot[0], del = tot[1], rho = tot[2];
+    res = bnorm2 > 0 ? sqrt(rho / bnorm2) : 0.0;
+    double alpha, beta;
+    if (it == 0) {
+      beta = 0.0;
+      alpha = gam / del;
+    } else {
+      beta = gam / gam_old;
+      alpha = gam / (del - beta * gam / alpha_old);
+    }
+    if (isnan(res)) it = maxit;  // nothing later changes a NaN
+    if ((it > 0 && res <= tol) || bnorm2 == 0.0) done = 1;
+    else if (it >= maxit) done = 2;
+    if (done) break;
+    gam_old = gam;
+    alpha_old = alpha;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      if (!k[c]) continue;
+      const double sn = w[c] + beta * so[c];
+      const double pc = u[c] + beta * p[c];
+      r[c] = r[c] - alpha * sn;
+      u[c] = r[c] / d[c];
+      p[c] = pc;
+      x(c) = x(c) + alpha * pc;
+      so[c] = sn;
+    }
+    exchange(uc);
+#pragma unroll
+    for (int c = 0; c < C; c++) w[c] = mul(u[c], c);
+    total3(terms, tot);
+  }
+  // the potential (once converged) and the true residual of x
+  exchange(x);
+  total3(
+      [&](int c, double (&f)[3]) {
+        const int tile = t / kTpb + NTH / kTpb * (kOneD ? c : c / kPcgRows);
+        const int ci = (tile % A.nbx) * kTX + t % kTX;
+        const int cj = kOneD ? 0
+                             : (tile / A.nbx) * kPcgTY + t % kTpb / kTX +
+                                   (c % kPcgRows) * (kPcgTY / kPcgRows);
+        const size_t m = (size_t)(cj + 1) * P + (ci + 1);
+        const double rr = (A.rhs0[m] - mul(x(c), c)) / vol(c);
+        f[0] = rr * rr;
+        f[1] = f[2] = 0.0;
+        A.x[m] = x(c);
+        if (done == 1) A.ph[m] = A.ph[m] + x(c);
+      },
+      tot);
+  if (t == 0) {
+    sc->bnorm2 = bnorm2;
+    sc->iters = it;
+    sc->resid = res;
+    sc->tres = bnorm2 > 0 ? sqrt(tot[0] / bnorm2) : sqrt(tot[0]);
+    sc->done = done;
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Aggregation multigrid V(2,2)-cycle used as the PCG preconditioner.
@@ -3157,6 +3348,29 @@ void launch_pcg_it(const PcgArgs& a, hipStream_t s) {
 void launch_pcg_finish(const PcgArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_pcg_finish, dim3(capped_grid(a.nbx * a.nby)), dim3(kNT), 0, s, a);
   hipLaunchKernelGGL(k_pcg_tres, dim3(1), dim3(kNT), 0, s, a, capped_grid(a.nbx * a.nby));
+}
+// The workgroup shapes of k_pcg_small: the smallest that holds the system's
+// tiles (one dimension: a wave per 64 cells; two: 256 threads per 64 x 8).
+bool pcg_small_fits(const Geo& G) {
+  if (G.by == 1) return G.bx <= 64 * 64;
+  const int nt = ((G.bx + kTX - 1) / kTX) * ((G.by + kPcgTY - 1) / kPcgTY);
+  return nt <= 8 && (G.bx + 2) * (G.by + 2) <= kPcgSmallPlane;
+}
+void launch_pcg_small(const PcgArgs& a, hipStream_t s) {
+  const int nt = a.nbx * a.nby;
+#define PCG_SMALL(ONED, NTH, S) \
+  hipLaunchKernelGGL((k_pcg_small<ONED, NTH, S>), dim3(1), dim3(NTH), 0, s, a)
+  if (a.G.by == 1) {
+    if (nt <= 1) PCG_SMALL(true, 64, 1);
+    else if (nt <= 4) PCG_SMALL(true, 256, 1);
+    else if (nt <= 16) PCG_SMALL(true, 1024, 1);
+    else PCG_SMALL(true, 1024, 4);
+  } else {
+    if (nt <= 1) PCG_SMALL(false, 256, 1);
+    else if (nt <= 4) PCG_SMALL(false, 1024, 1);
+    else PCG_SMALL(false, 1024, 2);
+  }
+#undef PCG_SMALL
 }
 static int cells_blocks(int n) { return (n + 255) / 256; }
 void launch_mg_coarsen(const MgArgs& a, hipStream_t s) {
