@@ -1704,141 +1704,229 @@ __device__ __forceinline__ void mg_coarsen_body(const MgArgs& A, int bid, int nb
 __global__ void __launch_bounds__(256) k_mg_coarsen(MgArgs A) { mg_coarsen_body<0>(A, blockIdx.x, gridDim.x); }
 
 constexpr int kGsTX = 32, kGsTY = 16;  // tile
-constexpr int kGsH = 4;                 // halo of the down kernels (four half-sweeps)
-static_assert((kGsTX / 2) * kGsTY == kNT, "one thread per horizontal cell pair");
+constexpr int kGsH = 4;                // halo of the down kernels (four half-sweeps)
+// The tile and its 4-cell halo as 20 x 12 aggregates of 2x2 cells, one per
+// thread.  Children c = a + 2b at (2I + a, 2J + b): colour (a + b) & 1 (tiles
+// start at even cells), i.e. 0 and 3 are red, 1 and 2 black.
+constexpr int kAgX = (kGsTX + 2 * kGsH) / 2, kAgY = (kGsTY + 2 * kGsH) / 2;
+static_assert(kAgX * kAgY <= kNT, "one thread per aggregate");
+constexpr int kGsW = kGsTX + 2 * kGsH, kGsR = kGsTY + 2 * kGsH;  // the staged cells
 
-// A level's equation on one tile plus a halo of H cells, staged in LDS:
-// right-hand side, diagonal and its inverse (the sweeps multiply by it),
-// right/upper couplings and the iterate.  Cells outside the level carry r = 0,
-// d = 1 and no couplings, so they stay zero.
-template <int H>
-struct GsTile {
-  static constexpr int W = kGsTX + 2 * H, R = kGsTY + 2 * H;
-  double x[R][W];
-  double r[R][W];
-  double d[R][W];
-  double dinv[R][W];
-  double cx[R][W];
-  double cy[R][W];
+// A thread holds its aggregate's equations in registers: right-hand side,
+// diagonal and inverse diagonal (the sweeps multiply by it), the couplings
+// (left of children 0 and 2, inside them, right of 1 and 3; below 0 and 1,
+// inside, above 2 and 3) and the iterate.  Only the iterate is also in LDS,
+// for the neighbours: half of each update's neighbours are the thread's own
+// registers.  (With every operand of a cell in LDS, a tile took 46 KB and an
+// update ten LDS reads: two or three workgroups per CU, bound by LDS and
+// latency.)  Cells outside the level have r = 0, d = 1 and no couplings, so
+// they stay zero.  Every half-sweep updates every cell; those of the outer
+// rings, whose own neighbours are missing, become invalid, one ring further
+// inwards per half-sweep, and never reach the tile.
+struct GsAgg {
+  double r[4], d[4], dinv[4], x[4];
+  double cl[2], ch[2], cr[2], cb[2], cv[2], ct[2];
 };
+// The iterates of the staged cells and one ring around them, by column parity
+// (even, odd), so that a wave's accesses have unit stride: cell (2I + a, y) of
+// the staged region is v[a][y + 1][I + 1].
+struct GsX {
+  double v[2][kGsR + 2][kAgX + 2];
+};
+
+// Where this thread's aggregate lies: (i, j) its child 0 in the level, in bit
+// c: child c inside the level, own: inside the tile.
+struct GsPos {
+  int I, J, i, j, in;
+  bool act, own;
+};
+
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // 8-byte aligned in memory
+__device__ __forceinline__ d2 gld2(const double* p, size_t i) {
+  return *(const __attribute__((address_space(1))) d2u*)(to_global(p) + i);
+}
+__device__ __forceinline__ void gst2(double* p, size_t i, double v0, double v1) {
+  d2 v = {v0, v1};
+  *(__attribute__((address_space(1))) d2u*)(to_global(p) + i) = v;
+}
 
 __device__ __forceinline__ int gs_tiles_x(const MgLevel& F) { return (F.nx + kGsTX - 1) / kGsTX; }
-
-// Stage r, d, cx, cy of the tile at (i0, j0) and its halo; with kUp also the
-// iterate x1 + oc * e_c(parent) of the up kernel.  In two parts: gs_load issues
-// every load of the tile into registers (cells outside the level load the
-// padded plane's first element and discard it), gs_store writes LDS, so the
-// staging costs one memory round trip and a kernel can issue other loads
-// between the two.
-template <int H, bool kUp>
-struct GsRegs {
-  static constexpr int NS = (GsTile<H>::R * GsTile<H>::W + kNT - 1) / kNT;
-  double r[NS], d[NS], cx[NS], cy[NS], x[NS], e[NS];
-  bool in[NS];
-};
-template <int H, bool kUp>
-__device__ __forceinline__ void gs_load(const MgLevel& F, int i0, int j0, const MgLevel& C,
-                                        GsRegs<H, kUp>& g) {
-  constexpr int W = GsTile<H>::W, R = GsTile<H>::R;
-#pragma unroll
-  for (int q = 0; q < g.NS; q++) {
-    const int k = threadIdx.x + kNT * q;
-    const int b = k / W, a = k % W;
-    const int i = i0 - H + a, j = j0 - H + b;
-    g.in[q] = k < R * W && i >= 0 && i < F.nx && j >= 0 && j < F.ny;
-    const size_t m = g.in[q] ? mg_at(F, i, j) : 0;
-    g.r[q] = gld(F.r, m);
-    g.d[q] = gld(F.d, m);
-    g.cx[q] = gld(F.cx, m);
-    g.cy[q] = gld(F.cy, m);
-    if (kUp) {
-      g.x[q] = gld(F.x1, m);
-      g.e[q] = gld(C.e, g.in[q] ? mg_at(C, i >> 1, j >> 1) : 0);
-    }
-  }
-}
-template <int H, bool kUp>
-__device__ __forceinline__ void gs_store(const GsRegs<H, kUp>& g, GsTile<H>& s, double oc) {
-  constexpr int W = GsTile<H>::W, R = GsTile<H>::R;
-#pragma unroll
-  for (int q = 0; q < g.NS; q++) {
-    const int k = threadIdx.x + kNT * q;
-    if (k < R * W) {
-      const int b = k / W, a = k % W;
-      const bool in = g.in[q];
-      const double dq = in ? g.d[q] : 1.0;
-      s.r[b][a] = in ? g.r[q] : 0.0;
-      s.d[b][a] = dq;
-      s.dinv[b][a] = 1.0 / dq;
-      s.cx[b][a] = in ? g.cx[q] : 0.0;
-      s.cy[b][a] = in ? g.cy[q] : 0.0;
-      if (kUp) s.x[b][a] = in ? g.x[q] + oc * g.e[q] : 0.0;
-    }
-  }
-}
-template <int H, bool kUp>
-__device__ __forceinline__ void gs_stage(const MgLevel& F, GsTile<H>& s, int i0, int j0,
-                                         const MgLevel& C, double oc) {
-  GsRegs<H, kUp> g;
-  gs_load<H, kUp>(F, i0, j0, C, g);
-  gs_store<H, kUp>(g, s, oc);
-}
-
-// One Gauss-Seidel half-sweep over the cells of colour c ((i + j) & 1 == c)
-// within h <= H - 1 cells of the tile at (i0, j0), entirely in LDS.  A thread
-// updates up to kGsHalfIt cells.  Batched (kBatch): cells of one colour do not
-// read each other, so every cell's operands are read before any new value is
-// written, and the LDS reads of all of a thread's cells are in flight
-// together; that holds their values in registers, which the ensemble's
-// kernels, whose grids fill the chip, cannot spare (three waves per SIMD need
-// at most 168 VGPRs), so they update one cell after the other.
-template <int H>
-constexpr int kGsHalfIt =
-    ((kGsTY + 2 * (H - 1)) * ((kGsTX + 2 * (H - 1)) / 2) + kNT - 1) / kNT;
-template <bool kBatch, int H>
-__device__ __forceinline__ void gs_half(GsTile<H>& s, int i0, int j0, int c, int h) {
-  #pragma clang fp contract(fast)  // smoother arithmetic: FMAs allowed
-  const int w2 = (kGsTX + 2 * h) / 2, rows = kGsTY + 2 * h, a0 = H - h;
-  if constexpr (!kBatch) {
-    for (int k = threadIdx.x; k < rows * w2; k += kNT) {
-      const int b = a0 + k / w2;
-      const int a = a0 + 2 * (k % w2) + ((c + i0 - H + a0 + j0 - H + b) & 1);
-      s.x[b][a] = (s.r[b][a] + s.cx[b][a - 1] * s.x[b][a - 1] + s.cx[b][a] * s.x[b][a + 1] +
-                   s.cy[b - 1][a] * s.x[b - 1][a] + s.cy[b][a] * s.x[b + 1][a]) *
-                  s.dinv[b][a];
-    }
-    return;
-  }
-  constexpr int NI = kGsHalfIt<H>;
-  double v[NI];
-  int at[NI];
-#pragma unroll
-  for (int q = 0; q < NI; q++) {
-    const int k = threadIdx.x + kNT * q;
-    at[q] = -1;
-    if (k < rows * w2) {
-      const int b = a0 + k / w2;
-      const int a = a0 + 2 * (k % w2) + ((c + i0 - H + a0 + j0 - H + b) & 1);
-      at[q] = b * GsTile<H>::W + a;
-      v[q] = (s.r[b][a] + s.cx[b][a - 1] * s.x[b][a - 1] + s.cx[b][a] * s.x[b][a + 1] +
-              s.cy[b - 1][a] * s.x[b - 1][a] + s.cy[b][a] * s.x[b + 1][a]) *
-             s.dinv[b][a];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < NI; q++)
-    if (at[q] >= 0) (&s.x[0][0])[at[q]] = v[q];
-}
-
-template <int H>
-__device__ __forceinline__ double gs_mx(const GsTile<H>& s, int b, int a) {
-  #pragma clang fp contract(fast)  // smoother arithmetic: FMAs allowed
-  return s.d[b][a] * s.x[b][a] - s.cx[b][a - 1] * s.x[b][a - 1] - s.cx[b][a] * s.x[b][a + 1] -
-         s.cy[b - 1][a] * s.x[b - 1][a] - s.cy[b][a] * s.x[b + 1][a];
-}
-
 __device__ __forceinline__ int gs_ntiles(const MgLevel& F) {
   return gs_tiles_x(F) * ((F.ny + kGsTY - 1) / kGsTY);
+}
+
+__device__ __forceinline__ GsPos gs_pos(const MgLevel& F, int i0, int j0) {
+  GsPos q;
+  const int t = threadIdx.x;
+  q.act = t < kAgX * kAgY;
+  q.I = q.act ? t % kAgX : 0;
+  q.J = q.act ? t / kAgX : 0;
+  q.i = i0 - kGsH + 2 * q.I;
+  q.j = j0 - kGsH + 2 * q.J;
+  // (levels start at even cells: child 0 is inside whenever another child is)
+  const bool ok = q.act && q.i >= 0 && q.i < F.nx && q.j >= 0 && q.j < F.ny;
+  const bool x1 = q.i + 1 < F.nx, y1 = q.j + 1 < F.ny;
+  q.in = ok ? 1 | (x1 ? 2 : 0) | (y1 ? 4 : 0) | (x1 && y1 ? 8 : 0) : 0;
+  q.own = ok && q.I >= kGsH / 2 && q.I < kAgX - kGsH / 2 && q.J >= kGsH / 2 && q.J < kAgY - kGsH / 2;
+  return q;
+}
+// The padded index of row b's pair of children, 0 (the plane's first elements,
+// loaded and discarded) for a row outside the level.
+__device__ __forceinline__ size_t gs_row(const MgLevel& F, const GsPos& q, int b) {
+  return q.in & (b ? 4 : 1) ? mg_at(F, q.i, q.j + b) : 0;
+}
+
+// The aggregate's loads (a row's two children as one 16-byte load; a row's
+// pair of an odd level reaches into the ghost column), issued together; gs_set
+// masks them and forms the inverse diagonal.
+struct GsRaw {
+  d2 r[2], d[2], cx[2], cy[2], cyb;
+  double cxl[2];
+};
+template <bool kR>
+__device__ __forceinline__ void gs_load(const MgLevel& F, const double* r, const GsPos& q,
+                                        GsRaw& g) {
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    const size_t m = gs_row(F, q, b);
+    if (kR) g.r[b] = gld2(r, m);
+    g.d[b] = gld2(F.d, m);
+    g.cx[b] = gld2(F.cx, m);
+    g.cy[b] = gld2(F.cy, m);
+    g.cxl[b] = gld((const double*)F.cx, m ? m - 1 : 0);
+  }
+  const size_t m = gs_row(F, q, 0);
+  g.cyb = gld2(F.cy, m ? m - F.P : 0);
+}
+__device__ __forceinline__ void gs_set(const GsRaw& g, int in, GsAgg& s) {
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+      const bool ok = in & (1 << (a + 2 * b));
+      const double dq = ok ? (a ? g.d[b].y : g.d[b].x) : 1.0;
+      s.d[a + 2 * b] = dq;
+      s.dinv[a + 2 * b] = 1.0 / dq;
+    }
+  s.cl[0] = in & 1 ? g.cxl[0] : 0.0;
+  s.cl[1] = in & 4 ? g.cxl[1] : 0.0;
+  s.ch[0] = in & 1 ? g.cx[0].x : 0.0;
+  s.ch[1] = in & 4 ? g.cx[1].x : 0.0;
+  s.cr[0] = in & 2 ? g.cx[0].y : 0.0;
+  s.cr[1] = in & 8 ? g.cx[1].y : 0.0;
+  s.cb[0] = in & 1 ? g.cyb.x : 0.0;
+  s.cb[1] = in & 2 ? g.cyb.y : 0.0;
+  s.cv[0] = in & 1 ? g.cy[0].x : 0.0;
+  s.cv[1] = in & 2 ? g.cy[0].y : 0.0;
+  s.ct[0] = in & 4 ? g.cy[1].x : 0.0;
+  s.ct[1] = in & 8 ? g.cy[1].y : 0.0;
+}
+__device__ __forceinline__ void gs_set_r(const d2 (&r)[2], int in, GsAgg& s) {
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+    s.r[c] = in & (1 << c) ? (c & 1 ? r[c >> 1].y : r[c >> 1].x) : 0.0;
+}
+
+// Writes one colour's children to LDS (red 0 and 3, black 1 and 2).
+template <int COL>
+__device__ __forceinline__ void gs_put(const GsAgg& g, GsX& s, const GsPos& q) {
+  if (!q.act) return;
+  const int y = 2 * q.J + 1, p = q.I + 1;
+  if (COL == 0) {
+    s.v[0][y][p] = g.x[0];
+    s.v[1][y + 1][p] = g.x[3];
+  } else {
+    s.v[1][y][p] = g.x[1];
+    s.v[0][y + 1][p] = g.x[2];
+  }
+}
+
+// One Gauss-Seidel half-sweep of colour COL (cells of one colour do not read
+// each other); the caller separates half-sweeps by barriers.
+template <int COL>
+__device__ __forceinline__ void gs_half(GsAgg& g, GsX& s, const GsPos& q) {
+  const int y = 2 * q.J + 1, p = q.I + 1;
+  // (r + left + right + below + above) / d, fused as written: the smoother's
+  // roundings are part of the results
+  auto gs = [](double r, double l, double xl, double c, double xr, double b, double xb, double t,
+               double xt, double dinv) {
+    return fma(t, xt, fma(b, xb, fma(c, xr, fma(l, xl, r)))) * dinv;
+  };
+  if (COL == 0) {
+    const double v0 = gs(g.r[0], g.cl[0], s.v[1][y][p - 1], g.ch[0], g.x[1], g.cb[0],
+                         s.v[0][y - 1][p], g.cv[0], g.x[2], g.dinv[0]);
+    const double v3 = gs(g.r[3], g.ch[1], g.x[2], g.cr[1], s.v[0][y + 1][p + 1], g.cv[1], g.x[1],
+                         g.ct[1], s.v[1][y + 2][p], g.dinv[3]);
+    g.x[0] = v0;
+    g.x[3] = v3;
+  } else {
+    const double v1 = gs(g.r[1], g.ch[0], g.x[0], g.cr[0], s.v[0][y][p + 1], g.cb[1],
+                         s.v[1][y - 1][p], g.cv[1], g.x[3], g.dinv[1]);
+    const double v2 = gs(g.r[2], g.cl[1], s.v[1][y + 1][p - 1], g.ch[1], g.x[3], g.cv[0], g.x[0],
+                         g.ct[0], s.v[0][y + 2][p], g.dinv[2]);
+    g.x[1] = v1;
+    g.x[2] = v2;
+  }
+  gs_put<COL>(g, s, q);
+}
+
+// M x at the aggregate's children (fused as written).
+__device__ __forceinline__ void gs_mx(const GsAgg& g, const GsX& s, const GsPos& q,
+                                      double (&mx)[4]) {
+  const int y = 2 * q.J + 1, p = q.I + 1;
+  auto m5 = [](double d, double x, double l, double xl, double c, double xr, double b, double xb,
+               double t, double xt) {
+    return fma(-t, xt, fma(-b, xb, fma(-c, xr, fma(d, x, -(l * xl)))));
+  };
+  mx[0] = m5(g.d[0], g.x[0], g.cl[0], s.v[1][y][p - 1], g.ch[0], g.x[1], g.cb[0],
+             s.v[0][y - 1][p], g.cv[0], g.x[2]);
+  mx[1] = m5(g.d[1], g.x[1], g.ch[0], g.x[0], g.cr[0], s.v[0][y][p + 1], g.cb[1],
+             s.v[1][y - 1][p], g.cv[1], g.x[3]);
+  mx[2] = m5(g.d[2], g.x[2], g.cl[1], s.v[1][y + 1][p - 1], g.ch[1], g.x[3], g.cv[0], g.x[0],
+             g.ct[0], s.v[0][y + 2][p]);
+  mx[3] = m5(g.d[3], g.x[3], g.ch[1], g.x[2], g.cr[1], s.v[0][y + 1][p + 1], g.cv[1], g.x[1],
+             g.ct[1], s.v[1][y + 2][p]);
+}
+
+// The ring around the staged cells (88 places in its two rows, 48 in its two
+// columns): `value(col, row)` of the region's cell (col, row), 0 for the
+// places no cell has.
+template <class V>
+__device__ __forceinline__ void gs_ring(GsX& s, V value) {
+  constexpr int kRows = 4 * (kAgX + 2), kAll = kRows + 2 * kGsR;
+  static_assert(kAll <= kNT, "one pass");
+  const int k = threadIdx.x;
+  if (k >= kAll) return;
+  int a, y, p;
+  if (k < kRows) {
+    a = k / (2 * (kAgX + 2));
+    y = k / (kAgX + 2) % 2 ? kGsR + 1 : 0;
+    p = k % (kAgX + 2);
+  } else {
+    a = (k - kRows) & 1 ? 0 : 1;
+    y = 1 + (k - kRows) / 2;
+    p = a ? 0 : kAgX + 1;
+  }
+  const int col = 2 * (p - 1) + a;
+  s.v[a][y][p] = col >= -1 && col <= kGsW ? value(col, y - 1) : 0.0;
+}
+
+// Writes the children of an own aggregate that lie inside the level.
+__device__ __forceinline__ void gs_store(double* p, const MgLevel& F, const GsPos& q,
+                                         const double (&v)[4]) {
+#pragma unroll
+  for (int b = 0; b < 2; b++) {
+    if (!(q.in & (b ? 4 : 1))) continue;
+    const size_t m = mg_at(F, q.i, q.j + b);
+    if (q.in & 2) gst2(p, m, v[2 * b], v[2 * b + 1]);
+    else gst(p, m, v[2 * b]);
+  }
+}
+// ... and one value per child into the tile's 32 x 16 table in LDS
+__device__ __forceinline__ void gs_table(double (&t)[kGsTY][kGsTX], const GsPos& q, int c,
+                                         double v) {
+  t[2 * q.J - kGsH + (c >> 1)][2 * q.I - kGsH + (c & 1)] = v;
 }
 
 // The solver state a convergence test reads, loaded at the start of the
@@ -1889,108 +1977,94 @@ __device__ __forceinline__ bool mg_check(DevScalars* sc, const CheckState& cs, d
   return stop;
 }
 
-// Level-0 CG vectors of the staged cells a thread holds in the down kernel,
-// and the volume of its own cells.
-constexpr int kGsSlots = (GsTile<kGsH>::R * GsTile<kGsH>::W + kNT - 1) / kNT;
-struct CgCells {
-  double r[kGsSlots], w[kGsSlots], s[kGsSlots], u[kGsSlots], p[kGsSlots], x[kGsSlots];
-  double vol[kGsSlots];
+// Loads of one tile for the level-0 CG update: the operator and the vectors of
+// the residual (CgRaw), and u, p, x of the tile's own cells (CgOwn).
+struct CgRaw {
+  GsRaw op;
+  d2 r[2], w[2], s[2], vx, vy, vr;
 };
-
-// Loads of one tile for the CG update: the operator into LDS, the vectors
-// into registers (u, p, x and the volume only for the tile's own cells).  As
-// gs_load / gs_store: cg_load issues every load (cells outside the level load
-// the padded planes' first element and discard it), cg_store writes LDS.
-struct CgRegs {
-  double d[kGsSlots], cx[kGsSlots], cy[kGsSlots], vx[kGsSlots], vy[kGsSlots], vr[kGsSlots];
-  bool in[kGsSlots], own[kGsSlots];
+struct CgOwn {
+  d2 u[2], p[2], x[2];
 };
-__device__ __forceinline__ void cg_load(const MgArgs& A, int i0, int j0, CgCells& c, CgRegs& g) {
-  constexpr int W = GsTile<kGsH>::W, R = GsTile<kGsH>::R;
+__device__ __forceinline__ void cg_load(const MgArgs& A, const GsPos& q, CgRaw& g) {
   const MgLevel& F = A.F;
   const Geo& G = A.G;
+  gs_load<false>(F, nullptr, q, g.op);
+  const d2 zero = {0.0, 0.0};
 #pragma unroll
-  for (int e = 0; e < kGsSlots; e++) {
-    const int k = threadIdx.x + kNT * e;
-    const int b = k / W, a = k % W;
-    const int i = i0 - kGsH + a, j = j0 - kGsH + b;
-    const bool in = k < R * W && i >= 0 && i < F.nx && j >= 0 && j < F.ny;
-    const bool own = in && a >= kGsH && a < kGsH + kGsTX && b >= kGsH && b < kGsH + kGsTY;
-    g.in[e] = in;
-    g.own[e] = own;
-    const size_t m = in ? mg_at(F, i, j) : 0;
-    const size_t mo = own ? m : 0;
-    g.d[e] = gld(F.d, m);
-    g.cx[e] = gld(F.cx, m);
-    g.cy[e] = gld(F.cy, m);
-    c.r[e] = gld((const double*)A.cg.r_old, m);
-    c.w[e] = gld((const double*)A.cg.w, m);
-    c.s[e] = A.cg.first ? 0.0 : gld((const double*)A.cg.s_old, m);
-    c.u[e] = gld((const double*)A.cg.u, mo);
-    c.p[e] = A.cg.first ? 0.0 : gld((const double*)A.cg.p, mo);
-    c.x[e] = gld((const double*)A.cg.x, mo);
-    g.vx[e] = gld(G.dlx, own ? i : 0);
-    g.vy[e] = gld(G.dly, own ? j : 0);
-    g.vr[e] = G.cyl ? gld(G.r, own ? j + 1 : 0) : 1.0;
+  for (int b = 0; b < 2; b++) {
+    const size_t m = gs_row(F, q, b);
+    g.r[b] = gld2(A.cg.r_old, m);
+    g.w[b] = gld2(A.cg.w, m);
+    g.s[b] = A.cg.first ? zero : gld2(A.cg.s_old, m);
   }
+  const int i = q.own ? q.i : 0, j = q.own ? q.j : 0;
+  const int i1 = q.own && (q.in & 2) ? i + 1 : i, j1 = q.own && (q.in & 4) ? j + 1 : j;
+  g.vx = {gld(G.dlx, i), gld(G.dlx, i1)};
+  g.vy = {gld(G.dly, j), gld(G.dly, j1)};
+  g.vr = {1.0, 1.0};
+  if (G.cyl) g.vr = {gld(G.r, j + 1), gld(G.r, j1 + 1)};
 }
-__device__ __forceinline__ void cg_store(const CgRegs& g, GsTile<kGsH>& s, CgCells& c) {
-  constexpr int W = GsTile<kGsH>::W, R = GsTile<kGsH>::R;
+__device__ __forceinline__ void cg_load_own(const MgArgs& A, const GsPos& q, CgOwn& g) {
+  const d2 zero = {0.0, 0.0};
 #pragma unroll
-  for (int e = 0; e < kGsSlots; e++) {
-    const int k = threadIdx.x + kNT * e;
-    if (!g.in[e]) c.r[e] = c.w[e] = c.s[e] = 0.0;
-    if (!g.own[e]) c.u[e] = c.p[e] = c.x[e] = 0.0;
-    c.vol[e] = g.vx[e] * g.vy[e] * g.vr[e];
-    if (k < R * W) {
-      const int b = k / W, a = k % W;
-      const double dq = g.in[e] ? g.d[e] : 1.0;
-      s.d[b][a] = dq;
-      s.dinv[b][a] = 1.0 / dq;
-      s.cx[b][a] = g.in[e] ? g.cx[e] : 0.0;
-      s.cy[b][a] = g.in[e] ? g.cy[e] : 0.0;
-    }
+  for (int b = 0; b < 2; b++) {
+    const size_t mo = q.own ? gs_row(A.F, q, b) : 0;
+    g.u[b] = gld2(A.cg.u, mo);
+    g.p[b] = A.cg.first ? zero : gld2(A.cg.p, mo);
+    g.x[b] = gld2(A.cg.x, mo);
   }
-}
-__device__ __forceinline__ void cg_stage(const MgArgs& A, GsTile<kGsH>& s, int i0, int j0,
-                                         CgCells& c) {
-  CgRegs g;
-  cg_load(A, i0, j0, c, g);
-  cg_store(g, s, c);
 }
 
-// The CG update of the staged cells: the new residual goes to LDS (halo cells
-// recompute their owners' values exactly); the tile's own cells also write
-// p, s, x, r and add |r/V|^2 to acc.
-__device__ __forceinline__ void cg_update(const MgArgs& A, GsTile<kGsH>& s, int i0, int j0,
-                                          const CgCells& c, double alpha, double beta,
-                                          double& acc) {
-  constexpr int W = GsTile<kGsH>::W, R = GsTile<kGsH>::R;
-  const MgLevel& F = A.F;
+// The CG update of the staged cells: the new residual is the aggregate's
+// right-hand side (halo cells recompute their owners' values exactly); own
+// aggregates also write s and r, and (r/V)^2 to the table ...
+__device__ __forceinline__ void cg_update(const MgArgs& A, const GsPos& q, const CgRaw& g,
+                                          double alpha, double beta, GsAgg& s,
+                                          double (&tab)[kGsTY][kGsTX]) {
+  double sn[4];
 #pragma unroll
-  for (int e = 0; e < kGsSlots; e++) {
-    const int k = threadIdx.x + kNT * e;
-    if (k < R * W) {
-      const int b = k / W, a = k % W;
-      const int i = i0 - kGsH + a, j = j0 - kGsH + b;
-      double r = 0.0;
-      if (i >= 0 && i < F.nx && j >= 0 && j < F.ny) {
-        const double sn = A.cg.first ? c.w[e] : c.w[e] + beta * c.s[e];
-        r = c.r[e] - alpha * sn;
-        if (a >= kGsH && a < kGsH + kGsTX && b >= kGsH && b < kGsH + kGsTY) {
-          const size_t m = mg_at(F, i, j);
-          const double pn = A.cg.first ? c.u[e] : c.u[e] + beta * c.p[e];
-          A.cg.p[m] = pn;
-          A.cg.s_new[m] = sn;
-          A.cg.x[m] = c.x[e] + alpha * pn;
-          F.r[m] = r;
-          const double rn = r / c.vol[e];
-          acc += rn * rn;
-        }
-      }
-      s.r[b][a] = r;
+  for (int c = 0; c < 4; c++) {
+    const int b = c >> 1;
+    const bool hi = c & 1;
+    const double w = hi ? g.w[b].y : g.w[b].x, so = hi ? g.s[b].y : g.s[b].x;
+    const double ro = hi ? g.r[b].y : g.r[b].x;
+    sn[c] = A.cg.first ? w : w + beta * so;
+    s.r[c] = q.in & (1 << c) ? ro - alpha * sn[c] : 0.0;
+    if (q.own) {
+      const double vol = (hi ? g.vx.y : g.vx.x) * (b ? g.vy.y : g.vy.x) * (b ? g.vr.y : g.vr.x);
+      const double rn = s.r[c] / vol;
+      gs_table(tab, q, c, rn * rn);
     }
   }
+  if (q.own) {
+    gs_store(A.cg.s_new, A.F, q, sn);
+    gs_store(A.F.r, A.F, q, s.r);
+  }
+}
+// ... and p and x.
+__device__ __forceinline__ void cg_update_own(const MgArgs& A, const GsPos& q, const CgOwn& g,
+                                              double alpha, double beta) {
+  if (!q.own) return;
+  double pn[4], xn[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const int b = c >> 1;
+    const bool hi = c & 1;
+    const double u = hi ? g.u[b].y : g.u[b].x, po = hi ? g.p[b].y : g.p[b].x;
+    pn[c] = A.cg.first ? u : u + beta * po;
+    xn[c] = (hi ? g.x[b].y : g.x[b].x) + alpha * pn[c];
+  }
+  gs_store(A.cg.p, A.F, q, pn);
+  gs_store(A.cg.x, A.F, q, xn);
+}
+
+// A value that is the same in every lane, held in scalar registers.
+__device__ __forceinline__ double uniform(double v) {
+  const uint64_t u = __double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
 // Down: pre-smooth M x = r on each tile, keep x1, restrict the residual into
@@ -1999,37 +2073,37 @@ __device__ __forceinline__ void cg_update(const MgArgs& A, GsTile<kGsH>& s, int 
 // CG form it first applies the CG update (alpha and beta from the up kernel's
 // partials) and writes the partials of the new |r/V|^2, which the next
 // kernel tests.  The partial sums are loaded together with the first tile.
-template <int kInstance, bool kCg>
+// (The sums' grouping, thread k taking the staged cells k, k + 256, ... in
+// rows of 40, is part of the results.)
+//
+// kEarly (a grid that leaves the chip idle, one tile per workgroup: latency
+// counts): every load of the first tile is issued with the solver state,
+// before the test of `done`; every address is in bounds whatever the state (a
+// block without tiles loads cells outside the level, which read the planes'
+// first elements).  Otherwise (ensembles, and grids of several tiles per
+// workgroup, where more waves in flight count) the loads follow the test; the
+// CG form loads its tiles after the reduction, and u, p and x behind the
+// residual's update, which keeps it at 128 VGPRs, four workgroups per CU.
+template <int kInstance, bool kCg, bool kEarly>
 __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
-  constexpr int W = GsTile<kGsH>::W, R = GsTile<kGsH>::R;
-  __shared__ GsTile<kGsH> s;
-  __shared__ double s_res[kGsTY][kGsTX / 2];
+  __shared__ GsX s;
+  __shared__ double s_tab[kGsTY][kGsTX];
   __shared__ double s_red[8 * kNW];
   DevScalars* sc = A.sc;
   const MgLevel &F = A.F, &C = A.C;
   const int ntx = gs_tiles_x(F);
   const TileRange tr = tile_range(gs_ntiles(F), bid, nb);
   const bool red = A.check || kCg;
-  // The first tile's loads and the partials'.  In the level-0 CG form of a
-  // single discharge they are issued with the solver state, before the test
-  // of `done`: every address is in bounds whatever the state (a block without
-  // tiles loads cells outside the level, which read the planes' first
-  // element), so that kernel waits for one memory round trip instead of two
-  // (measured: 0.4 us faster at 512^2; the coarser levels' kernels were
-  // measured 0.2-0.4 us slower so).  An ensemble's kernels issue them after
-  // the test and after the blocks without tiles have left: their launches
-  // fill the chip, where registers held across the warm-start block cost a
-  // wave per SIMD (256 members: 47.5 ms per pass against 35.5 ms), and they
-  // cover members whose solve has stopped.  The LDS stores follow the loads.
-  constexpr bool kEarly = kCg && kInstance == 0;
-  CgCells cc;
-  CgRegs cgr;
-  GsRegs<kGsH, false> gsr;
+  GsPos q = gs_pos(F, (tr.t0 % ntx) * kGsTX, (tr.t0 / ntx) * kGsTY);
+  CgRaw cgr;
+  CgOwn cgo;
+  GsRaw gsr;
   Part3 pl;
+  constexpr bool kFirst = kEarly || !kCg;  // the first tile's loads precede the reduction
   auto issue_first = [&]() {
-    const int i0 = (tr.t0 % ntx) * kGsTX, j0 = (tr.t0 / ntx) * kGsTY;
-    if (kCg) cg_load(A, i0, j0, cc, cgr);
-    else gs_load<kGsH, false>(F, i0, j0, C, gsr);
+    if (kCg && kFirst) cg_load(A, q, cgr);
+    if (!kCg) gs_load<true>(F, F.r, q, gsr);
+    if (kCg && kEarly) cg_load_own(A, q, cgo);
     if (red) part3_load(A.part_in, A.nb_in, pl);
   };
   if (kEarly) issue_first();
@@ -2097,8 +2171,7 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
     return;
   }
   if (!kEarly) issue_first();
-  if (kCg) cg_store(cgr, s, cc);
-  else gs_store<kGsH, false>(gsr, s, 0.0);
+  gs_ring(s, [](int, int) { return 0.0; });
   double pv[3];
   if (red) part3_sum(pl, A.nb_in, pv);
   double alpha = 0.0, beta = 0.0;
@@ -2147,7 +2220,8 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
           ps = del;
         }
       }
-      alpha = gam / ps;
+      beta = uniform(beta);
+      alpha = uniform(gam / ps);
       if (ps == 0.0 || !isfinite(alpha)) {  // breakdown: stop, not converged
         if (bid == 0 && threadIdx.x == 0) sc->done = 2;
         return;
@@ -2173,70 +2247,64 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
       }
     }
   }
-  MgLevel Fs = F;  // the level as staged (r from rhs after a discarded start)
-  if (zero_start) Fs.r = const_cast<double*>(A.rhs0);
   for (int t = tr.t0; t < tr.t1; t++) {
-    const int i0 = (t % ntx) * kGsTX, j0 = (t / ntx) * kGsTY;
-    if (t > tr.t0 || zero_start) {
-      __syncthreads();
-      if (kCg) cg_stage(A, s, i0, j0, cc);
-      else gs_stage<kGsH, false>(Fs, s, i0, j0, C, 0.0);
+    if (!kFirst || t > tr.t0 || zero_start) {
+      __syncthreads();  // the previous tile's iterates and tables have been read
+      q = gs_pos(F, (t % ntx) * kGsTX, (t / ntx) * kGsTY);
+      if (kCg) cg_load(A, q, cgr);
+      else gs_load<true>(F, zero_start ? A.rhs0 : F.r, q, gsr);
+      if (kCg && kEarly) cg_load_own(A, q, cgo);
     }
-    if (kCg) cg_update(A, s, i0, j0, cc, alpha, beta, racc[0]);
-    __syncthreads();
-    // first (red) half-sweep from zero is pointwise: the whole staged halo
-    // (batched as the half-sweeps are: every read of a thread's cells before
-    // its writes)
-    if constexpr (kInstance != 0) {
-      for (int k = threadIdx.x; k < R * W; k += kNT) {
-        const int b = k / W, a = k % W;
-        s.x[b][a] = ((i0 + a + j0 + b) & 1) == 0 ? s.r[b][a] * s.dinv[b][a] : 0.0;
-      }
+    GsAgg g;
+    if (kCg) {
+      gs_set(cgr.op, q.in, g);
+      cg_update(A, q, cgr, alpha, beta, g, s_tab);
+      if (kEarly) cg_update_own(A, q, cgo, alpha, beta);
+      else cg_load_own(A, q, cgo);
     } else {
-      constexpr int NP = (R * W + kNT - 1) / kNT;
-      double v[NP];
-#pragma unroll
-      for (int q = 0; q < NP; q++) {
-        const int k = threadIdx.x + kNT * q;
-        if (k < R * W) {
-          const int b = k / W, a = k % W;
-          v[q] = ((i0 + a + j0 + b) & 1) == 0 ? s.r[b][a] * s.dinv[b][a] : 0.0;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < NP; q++) {
-        const int k = threadIdx.x + kNT * q;
-        if (k < R * W) (&s.x[0][0])[k] = v[q];
-      }
+      gs_set(gsr, q.in, g);
+      gs_set_r(gsr.r, q.in, g);
     }
+    // first (red) half-sweep from zero: pointwise
+    g.x[0] = g.r[0] * g.dinv[0];
+    g.x[3] = g.r[3] * g.dinv[3];
+    g.x[1] = g.x[2] = 0.0;
+    gs_put<0>(g, s, q);
     __syncthreads();
-    gs_half<kInstance == 0>(s, i0, j0, 1, 3);
-    __syncthreads();
-    gs_half<kInstance == 0>(s, i0, j0, 0, 2);
-    __syncthreads();
-    gs_half<kInstance == 0>(s, i0, j0, 1, 1);
-    __syncthreads();
-    // residual of one horizontal cell pair (half an aggregate) per thread
-    const int cI = threadIdx.x % (kGsTX / 2), fj = threadIdx.x / (kGsTX / 2);
-    double rs = 0.0;
-    for (int q = 0; q < 2; q++) {
-      const int a = kGsH + 2 * cI + q, b = kGsH + fj;
-      const int i = i0 + 2 * cI + q, j = j0 + fj;
-      if (i < F.nx && j < F.ny) {
-        F.x1[mg_at(F, i, j)] = s.x[b][a];
-        rs += s.r[b][a] - gs_mx(s, b, a);
+    gs_half<1>(g, s, q);
+    if (kCg)
+      for (int k = threadIdx.x; k < kGsR * kGsW; k += kNT) {
+        const int b = k / kGsW - kGsH, a = k % kGsW - kGsH;
+        const int i = (t % ntx) * kGsTX + a, j = (t / ntx) * kGsTY + b;
+        if (a >= 0 && a < kGsTX && b >= 0 && b < kGsTY && i < F.nx && j < F.ny)
+          racc[0] += s_tab[b][a];
       }
+    __syncthreads();
+    gs_half<0>(g, s, q);
+    __syncthreads();
+    gs_half<1>(g, s, q);
+    __syncthreads();
+    if (kCg && !kEarly) cg_update_own(A, q, cgo, alpha, beta);
+    // the residual of the aggregate, a cell of the coarse level
+    if (q.own) {
+      double mx[4];
+      gs_mx(g, s, q, mx);
+      gs_store(F.x1, F, q, g.x);
+      double r0 = g.r[0] - mx[0], r1 = 0.0;
+      if (q.in & 2) r0 += g.r[1] - mx[1];
+      if (q.in & 4) r1 = g.r[2] - mx[2];
+      if (q.in & 8) r1 += g.r[3] - mx[3];
+      const size_t mc = mg_at(C, q.i / 2, q.j / 2);
+      const double rc = r0 + r1;
+      C.r[mc] = rc;
+      if (A.part_scale) s_tab[q.J - kGsH / 2][q.I - kGsH / 2] = rc * rc / C.d[mc];
     }
-    s_res[fj][cI] = rs;
-    __syncthreads();
-    if ((fj & 1) == 0) {
-      const int I = i0 / 2 + cI, J = (j0 + fj) / 2;
-      if (I < C.nx && J < C.ny) {
-        const size_t mc = mg_at(C, I, J);
-        const double rc = s_res[fj][cI] + s_res[fj + 1][cI];
-        C.r[mc] = rc;
-        if (A.part_scale) sacc[0] += rc * rc / C.d[mc];
-      }
+    if (A.part_scale) {
+      __syncthreads();
+      const int I = threadIdx.x & 15, J = threadIdx.x >> 5;
+      if (!(threadIdx.x & 16) && (t % ntx) * kGsTX / 2 + I < C.nx &&
+          (t / ntx) * kGsTY / 2 + J < C.ny)
+        sacc[0] += s_tab[J][I];
     }
   }
   if (A.part_scale) write_partials3(sacc, A.part_scale, s_red, bid);
@@ -2245,30 +2313,37 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
 
 // kCg: the level-0 CG form (its own instance: the CG vectors it keeps in
 // registers would otherwise limit the occupancy of the other levels' launches)
-template <bool kCg>
-__global__ void __launch_bounds__(kNT) k_mg_down(MgArgs A) {
-  mg_down_body<0, kCg>(A, blockIdx.x, gridDim.x);
+template <bool kCg, bool kEarly>
+__global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_down(MgArgs A) {
+  mg_down_body<0, kCg, kEarly>(A, blockIdx.x, gridDim.x);
 }
 
 // Up: x2 = x1 + oc * e_c(aggregate) on the staged halo, post-smooth, write e.
 // Level 0 writes u = B r and the partials of r.u, and of z.q (flexible CG) or,
 // in the CG form, w = M u and the partials of u.w; M u needs u one cell past
-// the tile, so that kernel stages a halo of H = 5 and sweeps one cell wider.
-template <int kInstance, int H>
+// the tile, so that kernel (H = 5) also stages the ring around the 4-cell halo.
+// kEarly as in the down kernel: the first tile's loads before the test of
+// `done` (in bounds whatever the state).
+template <int kInstance, int H, bool kEarly>
 __device__ __forceinline__ void mg_up_body(const MgArgs& A, int bid, int nb) {
-  constexpr int W = GsTile<H>::W, R = GsTile<H>::R;
-  __shared__ GsTile<H> s;
+  constexpr bool kW = H > kGsH;
+  __shared__ GsX s;
+  __shared__ double s_t0[kGsTY][kGsTX], s_t1[kGsTY][kGsTX];
   __shared__ double s_red[8 * kNW];
   const MgLevel &F = A.F, &C = A.C;
   const int ntx = gs_tiles_x(F);
   const TileRange tr = tile_range(gs_ntiles(F), bid, nb);
-  // A single discharge issues the first tile's loads before the test of
-  // `done` (in bounds whatever the state, as in the down kernel).  An
-  // ensemble stages every tile in the loop: its launches cover members whose
-  // solve has stopped, and the first tile's registers, live across the loop,
-  // would cost it a wave per SIMD.
-  GsRegs<H, true> g0;
-  if (kInstance == 0) gs_load<H, true>(F, (tr.t0 % ntx) * kGsTX, (tr.t0 / ntx) * kGsTY, C, g0);
+  GsPos q = gs_pos(F, (tr.t0 % ntx) * kGsTX, (tr.t0 / ntx) * kGsTY);
+  GsRaw gr;
+  d2 x1[2];
+  double ec;
+  auto load = [&]() {
+    gs_load<true>(F, F.r, q, gr);
+#pragma unroll
+    for (int b = 0; b < 2; b++) x1[b] = gld2(F.x1, gs_row(F, q, b));
+    ec = gld((const double*)C.e, q.in ? mg_at(C, q.i >> 1, q.j >> 1) : 0);
+  };
+  if (kEarly) load();
   {
     const int done = A.sc->done;
     if (kInstance == 0) {
@@ -2280,34 +2355,64 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int bid, int nb) {
   double acc[3] = {0.0, 0.0, 0.0};
   for (int t = tr.t0; t < tr.t1; t++) {
     const int i0 = (t % ntx) * kGsTX, j0 = (t / ntx) * kGsTY;
-    if (kInstance != 0 || t > tr.t0) {
-      if (t > tr.t0) __syncthreads();
-      gs_stage<H, true>(F, s, i0, j0, C, A.oc);
-    } else {
-      gs_store<H, true>(g0, s, A.oc);
+    if (!kEarly || t > tr.t0) {
+      if (t > tr.t0) {
+        __syncthreads();  // the previous tile's iterates and tables have been read
+        q = gs_pos(F, i0, j0);
+      }
+      load();
     }
+    // the ring (H = 5: the iterate there; H = 4: zero, set once)
+    if (kW || t == tr.t0)
+      gs_ring(s, [&](int col, int row) {
+        const int i = i0 - kGsH + col, j = j0 - kGsH + row;
+        if (!kW || i < 0 || i >= F.nx || j < 0 || j >= F.ny) return 0.0;
+        return gld((const double*)F.x1, mg_at(F, i, j)) +
+               A.oc * gld((const double*)C.e, mg_at(C, i >> 1, j >> 1));
+      });
+    GsAgg g;
+    gs_set(gr, q.in, g);
+    gs_set_r(gr.r, q.in, g);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      g.x[c] = q.in & (1 << c) ? (c & 1 ? x1[c >> 1].y : x1[c >> 1].x) + A.oc * ec : 0.0;
+    gs_put<0>(g, s, q);
+    gs_put<1>(g, s, q);
     __syncthreads();
-    gs_half<kInstance == 0>(s, i0, j0, 1, H - 1);
+    gs_half<1>(g, s, q);
     __syncthreads();
-    gs_half<kInstance == 0>(s, i0, j0, 0, H - 2);
+    gs_half<0>(g, s, q);
     __syncthreads();
-    gs_half<kInstance == 0>(s, i0, j0, 1, H - 3);
+    gs_half<1>(g, s, q);
     __syncthreads();
-    gs_half<kInstance == 0>(s, i0, j0, 0, H - 4);
-    __syncthreads();
-    for (int k = threadIdx.x; k < kGsTX * kGsTY; k += kNT) {
-      const int i = i0 + k % kGsTX, j = j0 + k / kGsTX;
-      if (i < F.nx && j < F.ny) {
-        const int b = H + k / kGsTX, a = H + k % kGsTX;
-        const double e = s.x[b][a];
-        const size_t m = mg_at(F, i, j);
-        F.e[m] = e;
-        acc[0] += s.r[b][a] * e;
-        if (A.q) acc[1] += A.q[m] * e;
-        if (H > kGsH && A.cg.on) {
-          const double w = gs_mx(s, b, a);
-          A.cg.w[m] = w;
-          acc[1] += e * w;
+    gs_half<0>(g, s, q);
+    if (kW && A.cg.on) {
+      __syncthreads();
+      if (q.own) {
+        double w[4];
+        gs_mx(g, s, q, w);
+        gs_store(A.cg.w, F, q, w);
+#pragma unroll
+        for (int c = 0; c < 4; c++) gs_table(s_t1, q, c, g.x[c] * w[c]);
+      }
+    }
+    if (q.own) {
+      gs_store(F.e, F, q, g.x);
+      if (A.level0)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          gs_table(s_t0, q, c, g.r[c] * g.x[c]);
+          if (A.q && (q.in & (1 << c)))
+            gs_table(s_t1, q, c, A.q[mg_at(F, q.i + (c & 1), q.j + (c >> 1))] * g.x[c]);
+        }
+    }
+    if (A.level0) {
+      __syncthreads();
+      for (int k = threadIdx.x; k < kGsTX * kGsTY; k += kNT) {
+        const int a = k % kGsTX, b = k / kGsTX;
+        if (i0 + a < F.nx && j0 + b < F.ny) {
+          acc[0] += s_t0[b][a];
+          if (A.q || (kW && A.cg.on)) acc[1] += s_t1[b][a];
         }
       }
     }
@@ -2315,8 +2420,10 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int bid, int nb) {
   if (A.level0) write_partials3(acc, A.part_out, s_red, bid);
 }
 
-template <int H>
-__global__ void __launch_bounds__(kNT) k_mg_up(MgArgs A) { mg_up_body<0, H>(A, blockIdx.x, gridDim.x); }
+template <int H, bool kEarly>
+__global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_up(MgArgs A) {
+  mg_up_body<0, H, kEarly>(A, blockIdx.x, gridDim.x);
+}
 
 // Once per solve, for the one-workgroup levels f .. L-1 (1024 threads):
 //  * levels f+1 .. L-1 are coarsened from level f (written by the tile
@@ -3257,14 +3364,14 @@ __global__ void __launch_bounds__(1024) kb_mg_coarse_setup(const MgCycleArgs* t,
   if (ens_slot(m, i, bid, nb)) mg_coarse_setup_body<1>(ens_arg(t, s, i));
 }
 template <bool kCg>
-__global__ void __launch_bounds__(kNT) kb_mg_down(const MgArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(kNT, 4) kb_mg_down(const MgArgs* t, EnsMap m, EnsSel s) {
   int i, bid, nb;
-  if (ens_slot(m, i, bid, nb)) mg_down_body<1, kCg>(ens_arg(t, s, i), bid, nb);
+  if (ens_slot(m, i, bid, nb)) mg_down_body<1, kCg, false>(ens_arg(t, s, i), bid, nb);
 }
 template <int H>
 __global__ void __launch_bounds__(kNT) kb_mg_up(const MgArgs* t, EnsMap m, EnsSel s) {
   int i, bid, nb;
-  if (ens_slot(m, i, bid, nb)) mg_up_body<1, H>(ens_arg(t, s, i), bid, nb);
+  if (ens_slot(m, i, bid, nb)) mg_up_body<1, H, false>(ens_arg(t, s, i), bid, nb);
 }
 __global__ void __launch_bounds__(1024) kb_mg_coarse_cycle(const MgCycleArgs* t, EnsMap m,
                                                            EnsSel s) {
@@ -3376,16 +3483,25 @@ static int cells_blocks(int n) { return (n + 255) / 256; }
 void launch_mg_coarsen(const MgArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_mg_coarsen, dim3(cells_blocks(a.C.nx * a.C.ny)), dim3(256), 0, s, a);
 }
-int mg_grid(const MgLevel& F) {
-  return capped_grid(((F.nx + kGsTX - 1) / kGsTX) * ((F.ny + kGsTY - 1) / kGsTY));
+static int mg_tiles(const MgLevel& F) {
+  return ((F.nx + kGsTX - 1) / kGsTX) * ((F.ny + kGsTY - 1) / kGsTY);
 }
+int mg_grid(const MgLevel& F) { return capped_grid(mg_tiles(F)); }
 void launch_mg_down(const MgArgs& a, hipStream_t s) {
-  if (a.cg.on) hipLaunchKernelGGL(k_mg_down<true>, dim3(mg_grid(a.F)), dim3(kNT), 0, s, a);
-  else hipLaunchKernelGGL(k_mg_down<false>, dim3(mg_grid(a.F)), dim3(kNT), 0, s, a);
+  const dim3 g(mg_grid(a.F)), b(kNT);
+  if (!a.cg.on) hipLaunchKernelGGL((k_mg_down<false, false>), g, b, 0, s, a);
+  else if (mg_tiles(a.F) <= kMaxPartials) hipLaunchKernelGGL((k_mg_down<true, true>), g, b, 0, s, a);
+  else hipLaunchKernelGGL((k_mg_down<true, false>), g, b, 0, s, a);
 }
 void launch_mg_up(const MgArgs& a, hipStream_t s) {
-  if (a.cg.on) hipLaunchKernelGGL(k_mg_up<kGsH + 1>, dim3(mg_grid(a.F)), dim3(kNT), 0, s, a);
-  else hipLaunchKernelGGL(k_mg_up<kGsH>, dim3(mg_grid(a.F)), dim3(kNT), 0, s, a);
+  const dim3 g(mg_grid(a.F)), b(kNT);
+  if (mg_tiles(a.F) <= kMaxPartials) {
+    if (a.cg.on) hipLaunchKernelGGL((k_mg_up<kGsH + 1, true>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((k_mg_up<kGsH, true>), g, b, 0, s, a);
+  } else {
+    if (a.cg.on) hipLaunchKernelGGL((k_mg_up<kGsH + 1, false>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((k_mg_up<kGsH, false>), g, b, 0, s, a);
+  }
 }
 void launch_mg_coarse_setup(const MgCycleArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_mg_coarse_setup, dim3(1), dim3(1024), 0, s, a);
