@@ -1357,8 +1357,14 @@ struct fs_ensemble {
   MgArgs* t_up = nullptr;         // [(i*kMgMaxLevels + l)*4 + v]
   MgCycleArgs* t_cc = nullptr;    // [i*4 + v]
   PcgArgs* t_fin = nullptr;       // [i]
-  EnsMapH m_stage, m_one, m_pcg, m_coarsen[kMgMaxLevels], m_down[kMgMaxLevels], m_up[kMgMaxLevels];
+  EnsMapH m_stage, m_one, m_pcg, m_coarsen[kMgMaxLevels], m_down[kMgMaxLevels];
   EnsMapH m_st;                   // the stage kernel's tiles (kTX x sty) of every member
+  // the tile kernels' (member, band) lists per level, [count, pad, pairs]: of
+  // every member, and of the members still iterating (rebuilt per chunk of
+  // iterations, in h_list, and copied to d_list)
+  std::vector<std::vector<int>> bands;  // bands per level and member
+  int32_t *d_all = nullptr, *d_list = nullptr, *h_list = nullptr;
+  size_t list_off[kMgMaxLevels + 1] = {};  // first entry of each level's list
   int sty = 8;                    // the stage kernel's tile height
   char* d_round = nullptr;
   char* h_round = nullptr;
@@ -1477,6 +1483,25 @@ int ens_tables(fs_ensemble* E) {
   return 0;
 }
 
+// The lists of every level over the members that `on` takes, in E->h_list.
+template <class On>
+void ens_fill_lists(fs_ensemble* E, On on) {
+  for (int l = 0; l < kMgMaxLevels; l++) {
+    int32_t* p = E->h_list + E->list_off[l];
+    int32_t count = 0;
+    for (int i = 0; i < E->n; i++) {
+      if (!on(i)) continue;
+      for (int b = 0; b < E->bands[l][i]; b++) {
+        p[2 + 2 * count] = i;
+        p[3 + 2 * count] = b;
+        count++;
+      }
+    }
+    p[0] = count;
+    p[1] = 0;
+  }
+}
+
 int ens_maps(fs_ensemble* E) {
   const int n = E->n;
   std::vector<int> stage(n), one(n, 1), pcg(n);
@@ -1493,6 +1518,7 @@ int ens_maps(fs_ensemble* E) {
   if (make_map(E->m_stage, stage) || make_map(E->m_one, one) || make_map(E->m_pcg, pcg) ||
       make_map(E->m_st, st))
     return FS_E_HIP;
+  E->bands.assign(kMgMaxLevels, std::vector<int>());
   for (int l = 0; l < kMgMaxLevels; l++) {
     std::vector<int> co(n, 0), dn(n, 0);
     for (int i = 0; i < n; i++) {
@@ -1503,9 +1529,24 @@ int ens_maps(fs_ensemble* E) {
       }
       if (l < (int)h->mg_first) dn[i] = mg_grid(h->mg[l]);
     }
-    if (make_map(E->m_coarsen[l], co) || make_map(E->m_down[l], dn) || make_map(E->m_up[l], dn))
-      return FS_E_HIP;
+    if (make_map(E->m_coarsen[l], co) || make_map(E->m_down[l], dn)) return FS_E_HIP;
+    E->bands[l] = dn;
   }
+  size_t o = 0;
+  for (int l = 0; l < kMgMaxLevels; l++) {
+    E->list_off[l] = o;
+    o += 2 + 2 * (size_t)E->m_down[l].m.nblocks;
+  }
+  E->list_off[kMgMaxLevels] = o;
+  if (E->d_all) HIP_OK(hipFree(E->d_all));
+  if (E->d_list) HIP_OK(hipFree(E->d_list));
+  if (E->h_list) HIP_OK(hipHostFree(E->h_list));
+  E->d_all = E->d_list = E->h_list = nullptr;
+  HIP_OK(hipMalloc(&E->d_all, o * sizeof(int32_t)));
+  HIP_OK(hipMalloc(&E->d_list, o * sizeof(int32_t)));
+  HIP_OK(hipHostMalloc(&E->h_list, o * sizeof(int32_t)));
+  ens_fill_lists(E, [](int) { return true; });
+  HIP_OK(hipMemcpy(E->d_all, E->h_list, o * sizeof(int32_t), hipMemcpyHostToDevice));
   return 0;
 }
 
@@ -1587,18 +1628,23 @@ int ens_fail(fs_ensemble* E, int i) {
 // One V-cycle of every Poisson member: down over the tile levels, the
 // one-workgroup coarse cycle, up.  v: 0 the initial cycle, then one CG
 // iteration each: 1 odd, 2 even, 3 the first.
-void ens_vcycle(fs_ensemble* E, int v, const uint8_t* mask) {
-  for (int l = 0; l < E->maxF; l++)
-    launch_ens_mg_down(E->t_down, with_mask(E->m_down[l], mask),
-                       EnsSel{nullptr, kMgMaxLevels * 4, l * 4 + v}, l == 0 && v != 0, E->st);
+// lists: of every member (E->d_all), or of those still iterating (E->d_list).
+void ens_vcycle(fs_ensemble* E, int v, const uint8_t* mask, const int32_t* lists) {
+  auto list = [&](int l) { return EnsList{lists + E->list_off[l], lists + E->list_off[l] + 2}; };
+  for (int l = 0; l < E->maxF; l++) {
+    const EnsMap m = with_mask(E->m_down[l], mask);
+    const EnsSel s{nullptr, kMgMaxLevels * 4, l * 4 + v};
+    if (l == 0 && v == 0) launch_ens_mg_down_init(E->t_down, m, s, E->st);
+    else launch_ens_mg_down(E->t_down, m, s, list(l), l == 0, E->st);
+  }
   launch_ens_mg_coarse_cycle(E->t_cc, with_mask(E->m_one, mask), EnsSel{nullptr, 4, v}, E->st);
   for (int l = E->maxF; l-- > 0;)
-    launch_ens_mg_up(E->t_up, with_mask(E->m_up[l], mask), EnsSel{nullptr, kMgMaxLevels * 4, l * 4 + v},
-                     l == 0, E->st);
+    launch_ens_mg_up(E->t_up, with_mask(E->m_down[l], mask),
+                     EnsSel{nullptr, kMgMaxLevels * 4, l * 4 + v}, list(l), l == 0, E->st);
 }
 
-void ens_iteration(fs_ensemble* E, int it, const uint8_t* mask) {
-  ens_vcycle(E, it == 0 ? 3 : (it & 1) ? 1 : 2, mask);
+void ens_iteration(fs_ensemble* E, int it, const uint8_t* mask, const int32_t* lists) {
+  ens_vcycle(E, it == 0 ? 3 : (it & 1) ? 1 : 2, mask, lists);
 }
 
 void ens_drop_graphs(fs_ensemble* E) {
@@ -1719,16 +1765,25 @@ int ens_round(fs_ensemble* E, std::vector<int>& left) {
                                      with_mask(E->m_one, r.pois), EnsSel{r.sel2, 1, 0}, E->st);
           launch_ens_mgpcg_init(E->t_init, with_mask(E->m_pcg, r.pois), EnsSel{r.sel2, 1, 0},
                                 E->st);
-          ens_vcycle(E, 0, r.pois);
-          for (int it = 0; it <= 8; it++) ens_iteration(E, it, r.pois);
+          ens_vcycle(E, 0, r.pois, E->d_all);
+          for (int it = 0; it <= 8; it++) ens_iteration(E, it, r.pois, E->d_all);
         }))
       return FS_E_HIP;
     for (bool first = true;; first = false) {
-      if (!first &&
-          ens_launch(E, &E->g_iter, [&]() {
-            for (int k = 0; k < 8; k++) ens_iteration(E, 9 + k, r.pois);
-          }))
-        return FS_E_HIP;
+      if (!first) {
+        // the members that have not stopped (E->h_sc is current)
+        ens_fill_lists(E, [&](int i) { return pois[i] && !E->h_sc[i].done; });
+        for (int l = 0; l < E->maxF; l++) {
+          const int32_t* p = E->h_list + E->list_off[l];
+          HIP_OK(hipMemcpyAsync(E->d_list + E->list_off[l], p,
+                                (2 + 2 * (size_t)p[0]) * sizeof(int32_t), hipMemcpyHostToDevice,
+                                E->st));
+        }
+        if (ens_launch(E, &E->g_iter, [&]() {
+              for (int k = 0; k < 8; k++) ens_iteration(E, 9 + k, r.pois, E->d_list);
+            }))
+          return FS_E_HIP;
+      }
       if (ens_sync(E)) return FS_E_HIP;
       bool all = true;
       for (int i = 0; i < n; i++) {
@@ -1809,8 +1864,9 @@ void ens_release(fs_ensemble* E) {
   for (int l = 0; l < kMgMaxLevels; l++) {
     fr(E->m_coarsen[l].d);
     fr(E->m_down[l].d);
-    fr(E->m_up[l].d);
   }
+  fr(E->d_all); fr(E->d_list);
+  if (E->h_list) (void)hipHostFree(E->h_list);
   if (E->h_sc) (void)hipHostFree(E->h_sc);
   if (E->h_round) (void)hipHostFree(E->h_round);
   if (E->st) (void)hipStreamDestroy(E->st);

@@ -287,6 +287,12 @@ struct EnsMap {
   const uint8_t* active;  // per member: takes part in this launch
   int32_t nblocks;        // blocks of the launch
 };
+// The (member, band) pairs that a launch of the multigrid tile kernels covers,
+// members in order, each member's bands 0 .. nb[member] - 1 in order.
+struct EnsList {
+  const int32_t* count;
+  const int32_t* at;  // 2 per entry
+};
 // A member's arguments: table[(sel ? sel[member] : member) * stride + off].
 struct EnsSel {
   const int32_t* sel;
@@ -306,10 +312,13 @@ void launch_ens_mg_coarsen(const MgArgs* t, const EnsMap& m, const EnsSel& s, hi
 void launch_ens_mg_coarse_setup(const MgCycleArgs* t, const EnsMap& m, const EnsSel& s,
                                 hipStream_t st);
 // cg: the members' level-0 CG form (cg.on in every selected entry)
-void launch_ens_mg_down(const MgArgs* t, const EnsMap& m, const EnsSel& s, bool cg,
-                        hipStream_t st);
+void launch_ens_mg_down(const MgArgs* t, const EnsMap& m, const EnsSel& s, const EnsList& l,
+                        bool cg, hipStream_t st);
+// the finest level of the initial cycle
+void launch_ens_mg_down_init(const MgArgs* t, const EnsMap& m, const EnsSel& s, hipStream_t st);
 // cg: the level-0 up kernel of the multigrid-PCG (wider halo, w = M u)
-void launch_ens_mg_up(const MgArgs* t, const EnsMap& m, const EnsSel& s, bool cg, hipStream_t st);
+void launch_ens_mg_up(const MgArgs* t, const EnsMap& m, const EnsSel& s, const EnsList& l, bool cg,
+                      hipStream_t st);
 void launch_ens_mg_coarse_cycle(const MgCycleArgs* t, const EnsMap& m, const EnsSel& s,
                                 hipStream_t st);
 void launch_ens_mgpcg_init(const MgPcgArgs* t, const EnsMap& m, const EnsSel& s, hipStream_t st);

@@ -71,16 +71,25 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
   return (b % 8) * (nb8 / 8) + b / 8;
 }
 
+// The block that xcd_tile sends to band position t.
+__device__ __forceinline__ int xcd_block(int t, int nb) {
+  const int w = nb / 8;
+  if (t >= 8 * w) return t;
+  return (t % w) * 8 + t / w;
+}
+
 // Contiguous range [t0, t1) of the ntiles tiles for this block when a capped
 // grid covers them (XCD-aware block order; trailing blocks may be empty).
 struct TileRange {
   int t0, t1;
 };
-__device__ __forceinline__ TileRange tile_range(int ntiles, int bid, int nb) {
-  const int b = xcd_tile(bid, nb);
+__device__ __forceinline__ TileRange band_range(int ntiles, int b, int nb) {
   const int per = (ntiles + nb - 1) / nb;
   const int t0 = b * per;
   return {t0, t0 + per < ntiles ? t0 + per : ntiles};
+}
+__device__ __forceinline__ TileRange tile_range(int ntiles, int bid, int nb) {
+  return band_range(ntiles, xcd_tile(bid, nb), nb);
 }
 
 // Block-wide sums (s_red: NV * NW doubles) and minimum of NW waves.
@@ -2074,7 +2083,8 @@ __device__ __forceinline__ double uniform(double v) {
 // partials) and writes the partials of the new |r/V|^2, which the next
 // kernel tests.  The partial sums are loaded together with the first tile.
 // (The sums' grouping, thread k taking the staged cells k, k + 256, ... in
-// rows of 40, is part of the results.)
+// rows of 40, is part of the results.)  A launch's blocks take bands of
+// consecutive tiles; the body covers the bands [band0, band1) of the nb.
 //
 // kEarly (a grid that leaves the chip idle, one tile per workgroup: latency
 // counts): every load of the first tile is issued with the solver state,
@@ -2085,14 +2095,17 @@ __device__ __forceinline__ double uniform(double v) {
 // CG form loads its tiles after the reduction, and u, p and x behind the
 // residual's update, which keeps it at 128 VGPRs, four workgroups per CU.
 template <int kInstance, bool kCg, bool kEarly>
-__device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
+__device__ __forceinline__ void mg_down_body(const MgArgs& A, int band0, int band1, int nb) {
   __shared__ GsX s;
   __shared__ double s_tab[kGsTY][kGsTX];
   __shared__ double s_red[8 * kNW];
   DevScalars* sc = A.sc;
   const MgLevel &F = A.F, &C = A.C;
   const int ntx = gs_tiles_x(F);
-  const TileRange tr = tile_range(gs_ntiles(F), bid, nb);
+  const int ntiles = gs_ntiles(F);
+  TileRange tr = band_range(ntiles, band0, nb);
+  if (kInstance == 1) tr.t1 = band_range(ntiles, band1 - 1, nb).t1;
+  const bool writer = band0 == 0 && threadIdx.x == 0;  // (band 0 always has tiles)
   const bool red = A.check || kCg;
   GsPos q = gs_pos(F, (tr.t0 % ntx) * kGsTX, (tr.t0 / ntx) * kGsTY);
   CgRaw cgr;
@@ -2155,7 +2168,7 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
         }
       }
     }
-    if (bid == 0 && threadIdx.x == 0) {
+    if (writer) {
       sc->x3_ok = wn && sc->x2_ok;
       sc->dt_warm3 = sc->dt_warm2;
       sc->dt_warm2 = sc->dt_warm;
@@ -2165,9 +2178,15 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
   }
   double sacc[3] = {0.0, 0.0, 0.0};  // sum r_c^2 / d_c for the learned coarse solver
   double racc[3] = {0.0, 0.0, 0.0};  // sum |r/V|^2 after the CG update
-  if (tr.t0 >= tr.t1) {  // block 0 always has tiles (it writes the scalars)
-    if (A.part_scale) write_partials3(sacc, A.part_scale, s_red, bid);
-    if (kCg) write_partials3(racc, A.part_out, s_red, bid);
+  // the sums of a band, at the place of the block whose band it is
+  auto put_sums = [&](int band) {
+    const int b = xcd_block(band, nb);
+    if (A.part_scale) write_partials3(sacc, A.part_scale, s_red, b);
+    if (kCg) write_partials3(racc, A.part_out, s_red, b);
+    sacc[0] = racc[0] = 0.0;
+  };
+  if (tr.t0 >= tr.t1) {
+    for (int band = band0; band < band1; band++) put_sums(band);
     return;
   }
   if (!kEarly) issue_first();
@@ -2188,12 +2207,12 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
         // first transport step's, after the Poisson-only passes, is many
         // times larger than the next ones): the next start extrapolates
         // from this solve's correction alone, as after a solve from zero
-        if (bid == 0 && threadIdx.x == 0) {
+        if (writer) {
           sc->x2_ok = 0;
           sc->x3_ok = 0;
         }
       }
-      if (mg_check(sc, cs, tot[0], tot[1], A.init, A.it, bid == 0 && threadIdx.x == 0)) return;
+      if (mg_check(sc, cs, tot[0], tot[1], A.init, A.it, writer)) return;
     } else {
       // gamma = r.u, delta = u.M u; p.s = delta - beta gamma / alpha_old
       // (0 < p.s <= delta in exact arithmetic for a definite operator).  Near
@@ -2223,10 +2242,10 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
       beta = uniform(beta);
       alpha = uniform(gam / ps);
       if (ps == 0.0 || !isfinite(alpha)) {  // breakdown: stop, not converged
-        if (bid == 0 && threadIdx.x == 0) sc->done = 2;
+        if (writer) sc->done = 2;
         return;
       }
-      if (bid == 0 && threadIdx.x == 0) {
+      if (writer) {
         sc->cg_gam[A.it & 1] = gam;
         sc->cg_alpha[A.it & 1] = alpha;
       }
@@ -2247,6 +2266,7 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
       }
     }
   }
+  int band = band0, tend = kInstance == 1 ? band_range(ntiles, band, nb).t1 : 0;
   for (int t = tr.t0; t < tr.t1; t++) {
     if (!kFirst || t > tr.t0 || zero_start) {
       __syncthreads();  // the previous tile's iterates and tables have been read
@@ -2306,16 +2326,22 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int bid, int nb) {
           (t / ntx) * kGsTY / 2 + J < C.ny)
         sacc[0] += s_tab[J][I];
     }
+    if (kInstance == 1 && t + 1 == tend) {
+      put_sums(band++);
+      tend = band_range(ntiles, band, nb).t1;
+    }
   }
-  if (A.part_scale) write_partials3(sacc, A.part_scale, s_red, bid);
-  if (kCg) write_partials3(racc, A.part_out, s_red, bid);
+  if (kInstance != 1) put_sums(band);  // a single band
+  else
+    while (band < band1) put_sums(band++);  // trailing bands without tiles
 }
 
 // kCg: the level-0 CG form (its own instance: the CG vectors it keeps in
 // registers would otherwise limit the occupancy of the other levels' launches)
 template <bool kCg, bool kEarly>
 __global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_down(MgArgs A) {
-  mg_down_body<0, kCg, kEarly>(A, blockIdx.x, gridDim.x);
+  const int band = xcd_tile(blockIdx.x, gridDim.x);
+  mg_down_body<0, kCg, kEarly>(A, band, band + 1, gridDim.x);
 }
 
 // Up: x2 = x1 + oc * e_c(aggregate) on the staged halo, post-smooth, write e.
@@ -2325,14 +2351,16 @@ __global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_down(MgArgs A) {
 // kEarly as in the down kernel: the first tile's loads before the test of
 // `done` (in bounds whatever the state).
 template <int kInstance, int H, bool kEarly>
-__device__ __forceinline__ void mg_up_body(const MgArgs& A, int bid, int nb) {
+__device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1, int nb) {
   constexpr bool kW = H > kGsH;
   __shared__ GsX s;
   __shared__ double s_t0[kGsTY][kGsTX], s_t1[kGsTY][kGsTX];
   __shared__ double s_red[8 * kNW];
   const MgLevel &F = A.F, &C = A.C;
   const int ntx = gs_tiles_x(F);
-  const TileRange tr = tile_range(gs_ntiles(F), bid, nb);
+  const int ntiles = gs_ntiles(F);
+  TileRange tr = band_range(ntiles, band0, nb);
+  if (kInstance == 1) tr.t1 = band_range(ntiles, band1 - 1, nb).t1;
   GsPos q = gs_pos(F, (tr.t0 % ntx) * kGsTX, (tr.t0 / ntx) * kGsTY);
   GsRaw gr;
   d2 x1[2];
@@ -2353,6 +2381,13 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int bid, int nb) {
     if (done) return;
   }
   double acc[3] = {0.0, 0.0, 0.0};
+  int band = band0, tend = kInstance == 1 ? band_range(ntiles, band, nb).t1 : 0;
+  auto put_sums = [&]() {
+    if (A.level0) write_partials3(acc, A.part_out, s_red, xcd_block(band, nb));
+    acc[0] = acc[1] = 0.0;
+    band++;
+    if (kInstance == 1) tend = band_range(ntiles, band, nb).t1;
+  };
   for (int t = tr.t0; t < tr.t1; t++) {
     const int i0 = (t % ntx) * kGsTX, j0 = (t / ntx) * kGsTY;
     if (!kEarly || t > tr.t0) {
@@ -2416,13 +2451,17 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int bid, int nb) {
         }
       }
     }
+    if (kInstance == 1 && t + 1 == tend) put_sums();
   }
-  if (A.level0) write_partials3(acc, A.part_out, s_red, bid);
+  if (kInstance != 1) put_sums();  // a single band
+  else
+    while (band < band1) put_sums();  // trailing bands without tiles
 }
 
 template <int H, bool kEarly>
 __global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_up(MgArgs A) {
-  mg_up_body<0, H, kEarly>(A, blockIdx.x, gridDim.x);
+  const int band = xcd_tile(blockIdx.x, gridDim.x);
+  mg_up_body<0, H, kEarly>(A, band, band + 1, gridDim.x);
 }
 
 // Once per solve, for the one-workgroup levels f .. L-1 (1024 threads):
@@ -3304,6 +3343,10 @@ __global__ void k_eval_flux(FsPhys K, const double* a, double* out, int n, int d
 // ---------------------------------------------------------------------------
 // Ensemble kernels: each block finds its member and its block index within
 // that member's own launch shape, then runs the same body as the solo kernel.
+// (The argument tables are __restrict__: without it every store might change
+// them, and a kernel loads each pointer again, behind a wait, wherever it is
+// used, and through flat instructions: the finest down kernel took 435 us
+// instead of 326 us, the up kernel 200 instead of 150 us.)
 __device__ __forceinline__ bool ens_slot(const EnsMap& m, int& i, int& bid, int& nb) {
   i = m.inst[blockIdx.x];
   if (!m.active[i]) return false;
@@ -3318,17 +3361,17 @@ __device__ __forceinline__ const T& ens_arg(const T* t, const EnsSel& s, int i) 
 }
 
 template <int TY>
-__global__ void __launch_bounds__(kTX * TY, 4) kb_stage(const StageArgs* t, const FsPhys* K,
+__global__ void __launch_bounds__(kTX * TY, 4) kb_stage(const StageArgs* __restrict__ t, const FsPhys* __restrict__ K,
                                                     EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) stage_body<1, TY>(ens_arg(t, s, i), K[i], bid, nb);
 }
-__global__ void __launch_bounds__(kNT) kb_circ(const CircArgs* t, const FsPhys* K, EnsMap m,
+__global__ void __launch_bounds__(kNT) kb_circ(const CircArgs* __restrict__ t, const FsPhys* __restrict__ K, EnsMap m,
                                                EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) circ_body<1>(ens_arg(t, s, i), K[i]);
 }
-__global__ void __launch_bounds__(kNT) kb_ctrl(const CtrlArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(kNT) kb_ctrl(const CtrlArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) ctrl_body<1>(ens_arg(t, s, i));
 }
@@ -3350,57 +3393,94 @@ __global__ void kb_scalars(DevScalars* sc, const uint8_t* mask, int n, int op) {
     c->Vd_mi = c->Vd_or;
   }
 }
-__global__ void __launch_bounds__(kSNT, 4) kb_lapl(const LaplArgs* t, const FsPhys* K, EnsMap m,
+__global__ void __launch_bounds__(kSNT, 4) kb_lapl(const LaplArgs* __restrict__ t, const FsPhys* __restrict__ K, EnsMap m,
                                                EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) lapl_body<1>(ens_arg(t, s, i), K[i], bid, nb);
 }
-__global__ void __launch_bounds__(256) kb_mg_coarsen(const MgArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(256) kb_mg_coarsen(const MgArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) mg_coarsen_body<1>(ens_arg(t, s, i), bid, nb);
 }
-__global__ void __launch_bounds__(1024) kb_mg_coarse_setup(const MgCycleArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(1024) kb_mg_coarse_setup(const MgCycleArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) mg_coarse_setup_body<1>(ens_arg(t, s, i));
 }
+// The tile kernels of an ensemble run on a list of (member, band) pairs, in
+// order, which a grid that is resident at once shares out in contiguous
+// ranges: three workgroups per CU of the down kernels (148-168 VGPRs; held to
+// the 128 of four per CU they spill, and the finest takes 326 us instead of
+// 245 us), four of the up kernels.  A workgroup tests a member's state and
+// reduces its partial sums once for all its bands of that member, and what a
+// launch costs follows the members on the list.  Measured on the 256-member
+// sweep (14 327 bands on the finest level): down 245 us, up 150 us with every
+// member iterating (a workgroup per band: 310 and 185 us), 12 and 8 us for the
+// last few members (18 and 13 us), 3 us for none (14 us each).
+constexpr int kListDown = 3 * 256, kListUp = 4 * 256;
+template <class F>
+__device__ __forceinline__ void ens_bands(const EnsList& l, const EnsMap& m, F body) {
+  const int count = *l.count, per = (count + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int k0 = xcd_tile(blockIdx.x, gridDim.x) * per, k1 = min(count, k0 + per);
+  for (int k = k0; k < k1;) {
+    const int i = l.at[2 * k], band = l.at[2 * k + 1], nb = m.nb[i];
+    const int n = min(k1 - k, nb - band);  // its bands follow one another
+    if (m.active[i]) {
+      if (k > k0) __syncthreads();  // the last member's LDS has been read
+      body(i, band, band + n, nb);
+    }
+    k += n;
+  }
+}
 template <bool kCg>
-__global__ void __launch_bounds__(kNT, 4) kb_mg_down(const MgArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(kNT, 3) kb_mg_down(const MgArgs* __restrict__ t, EnsMap m, EnsSel s,
+                                                     EnsList l) {
+  ens_bands(l, m, [&](int i, int b0, int b1, int nb) {
+    mg_down_body<1, kCg, false>(ens_arg(t, s, i), b0, b1, nb);
+  });
+}
+// The initial cycle's finest level keeps a workgroup per band: its blocks form
+// the warm starts before the convergence test, so none may come so late that
+// it finds the solve already stopped by that test.
+__global__ void __launch_bounds__(kNT, 4) kb_mg_down_init(const MgArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
-  if (ens_slot(m, i, bid, nb)) mg_down_body<1, kCg, false>(ens_arg(t, s, i), bid, nb);
+  if (!ens_slot(m, i, bid, nb)) return;
+  const int band = xcd_tile(bid, nb);
+  mg_down_body<2, false, false>(ens_arg(t, s, i), band, band + 1, nb);
 }
 template <int H>
-__global__ void __launch_bounds__(kNT) kb_mg_up(const MgArgs* t, EnsMap m, EnsSel s) {
-  int i, bid, nb;
-  if (ens_slot(m, i, bid, nb)) mg_up_body<1, H, false>(ens_arg(t, s, i), bid, nb);
+__global__ void __launch_bounds__(kNT, 4) kb_mg_up(const MgArgs* __restrict__ t, EnsMap m, EnsSel s, EnsList l) {
+  ens_bands(l, m, [&](int i, int b0, int b1, int nb) {
+    mg_up_body<1, H, false>(ens_arg(t, s, i), b0, b1, nb);
+  });
 }
-__global__ void __launch_bounds__(1024) kb_mg_coarse_cycle(const MgCycleArgs* t, EnsMap m,
+__global__ void __launch_bounds__(1024) kb_mg_coarse_cycle(const MgCycleArgs* __restrict__ t, EnsMap m,
                                                            EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) mg_coarse_cycle_body<1>(ens_arg(t, s, i));
 }
-__global__ void __launch_bounds__(kNT) kb_mgpcg_init(const MgPcgArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(kNT) kb_mgpcg_init(const MgPcgArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) mgpcg_init_body<1>(ens_arg(t, s, i), bid, nb);
 }
 // the projected warm start of the members whose start takes it (the others
 // return at once): the start kernel's map, then one block per member
-__global__ void __launch_bounds__(kNT) kb_mgpcg_warm_ls(const MgPcgArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(kNT) kb_mgpcg_warm_ls(const MgPcgArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (!ens_slot(m, i, bid, nb)) return;
   const MgPcgArgs& A = ens_arg(t, s, i);
   if (A.warm && A.ls) mgpcg_warm_ls_body(A, bid, nb);
 }
-__global__ void __launch_bounds__(kNT) kb_mgpcg_warm_solve(const MgPcgArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(kNT) kb_mgpcg_warm_solve(const MgPcgArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (!ens_slot(m, i, bid, nb)) return;
   const MgPcgArgs& A = ens_arg(t, s, i);
   if (A.warm && A.ls) mgpcg_warm_solve_body(A);
 }
-__global__ void __launch_bounds__(kNT) kb_pcg_finish(const PcgArgs* t, EnsMap m, EnsSel s) {
+__global__ void __launch_bounds__(kNT) kb_pcg_finish(const PcgArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (ens_slot(m, i, bid, nb)) pcg_finish_body<1>(ens_arg(t, s, i), bid, nb);
 }
-__global__ void __launch_bounds__(kNT) kb_pcg_tres(const PcgArgs* t, EnsMap one, EnsSel s,
+__global__ void __launch_bounds__(kNT) kb_pcg_tres(const PcgArgs* __restrict__ t, EnsMap one, EnsSel s,
                                                    const int32_t* nbfin) {
   int i, bid, nb;
   if (ens_slot(one, i, bid, nb)) pcg_tres_body<1>(ens_arg(t, s, i), nbfin[i]);
@@ -3567,16 +3647,21 @@ void launch_ens_mg_coarse_setup(const MgCycleArgs* t, const EnsMap& m, const Ens
                                 hipStream_t st) {
   if (m.nblocks) hipLaunchKernelGGL(kb_mg_coarse_setup, dim3(m.nblocks), dim3(1024), 0, st, t, m, s);
 }
-void launch_ens_mg_down(const MgArgs* t, const EnsMap& m, const EnsSel& s, bool cg,
+static dim3 list_grid(const EnsMap& m, int most) { return dim3(m.nblocks < most ? m.nblocks : most); }
+void launch_ens_mg_down(const MgArgs* t, const EnsMap& m, const EnsSel& s, const EnsList& l, bool cg,
                         hipStream_t st) {
   if (!m.nblocks) return;
-  if (cg) hipLaunchKernelGGL(kb_mg_down<true>, dim3(m.nblocks), dim3(kNT), 0, st, t, m, s);
-  else hipLaunchKernelGGL(kb_mg_down<false>, dim3(m.nblocks), dim3(kNT), 0, st, t, m, s);
+  if (cg) hipLaunchKernelGGL(kb_mg_down<true>, list_grid(m, kListDown), dim3(kNT), 0, st, t, m, s, l);
+  else hipLaunchKernelGGL(kb_mg_down<false>, list_grid(m, kListDown), dim3(kNT), 0, st, t, m, s, l);
 }
-void launch_ens_mg_up(const MgArgs* t, const EnsMap& m, const EnsSel& s, bool cg, hipStream_t st) {
+void launch_ens_mg_down_init(const MgArgs* t, const EnsMap& m, const EnsSel& s, hipStream_t st) {
+  if (m.nblocks) hipLaunchKernelGGL(kb_mg_down_init, dim3(m.nblocks), dim3(kNT), 0, st, t, m, s);
+}
+void launch_ens_mg_up(const MgArgs* t, const EnsMap& m, const EnsSel& s, const EnsList& l, bool cg,
+                      hipStream_t st) {
   if (!m.nblocks) return;
-  if (cg) hipLaunchKernelGGL(kb_mg_up<kGsH + 1>, dim3(m.nblocks), dim3(kNT), 0, st, t, m, s);
-  else hipLaunchKernelGGL(kb_mg_up<kGsH>, dim3(m.nblocks), dim3(kNT), 0, st, t, m, s);
+  if (cg) hipLaunchKernelGGL(kb_mg_up<kGsH + 1>, list_grid(m, kListUp), dim3(kNT), 0, st, t, m, s, l);
+  else hipLaunchKernelGGL(kb_mg_up<kGsH>, list_grid(m, kListUp), dim3(kNT), 0, st, t, m, s, l);
 }
 void launch_ens_mg_coarse_cycle(const MgCycleArgs* t, const EnsMap& m, const EnsSel& s,
                                 hipStream_t st) {
