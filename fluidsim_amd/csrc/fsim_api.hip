@@ -165,7 +165,7 @@ struct fs_handle {
   DevScalars* h_sc = nullptr;  // pinned mirror
   DevScalars* h_pub = nullptr; // host-mapped copy written by k_publish (and its device address)
   DevScalars* d_pub = nullptr;
-  uint32_t* d_pubcnt = nullptr;  // publications run (device)
+  uint32_t* d_pubcnt = nullptr;  // publications run (device); [32] launch_io's count
   uint32_t pub_tok = 0;          // publications enqueued (host)
   bool spec_taken = false;       // the next pass's k_begin_step and stage 1 are enqueued and run
   double* d_pois = nullptr;    // rhs0 r0 cx cy dg x p r1 w0 w1 s0 s1 (kPois planes)
@@ -213,7 +213,15 @@ struct fs_handle {
   bool timing = false;
   hipEvent_t ev[8] = {};
   double tms[4] = {0, 0, 0, 0};
-  std::vector<double> stage_buf;
+  // Fields cross the boundary through pinned, device-mapped host memory (one
+  // block with the scalars' mirror and published copy): io_cap doubles, twice
+  // when a plane takes several pieces.  A piece's kernel is followed by its
+  // number in *h_iof, which the host polls.
+  char* h_pin = nullptr;
+  double *h_io = nullptr, *d_io = nullptr;
+  uint32_t *h_iof = nullptr, *d_iof = nullptr;
+  uint32_t io_tok = 0;  // pieces enqueued
+  size_t io_cap = 0;
 
   double* lev(int buf, int sp) const { return d_lev + ((size_t)buf * 4 + sp) * PL; }
   int bufA() const { return rot; }
@@ -266,23 +274,28 @@ int upload(fs_handle* h, double* dst, const double* src, size_t n) {
   return 0;
 }
 
-// Waits until the last publication enqueued (k_publish) has reached host
-// memory, and copies it to h_sc.  The poll asks the stream every 1024 rounds,
-// so that an error, or a stream that drained without publishing (which would
-// be a bug), ends the wait.
-int wait_published(fs_handle* h) {
-  const uint32_t tok = h->pub_tok;
-  const volatile uint32_t* seq = &h->h_pub->pub_seq;
-  for (unsigned k = 1; *seq != tok; k++) {
+// Waits until the count *seq in host memory, which kernels on the handle's
+// stream advance, has reached tok.  The poll asks the stream every 1024
+// rounds, so that an error, or a stream that drained without writing the count
+// (which would be a bug), ends the wait.
+int wait_count(fs_handle* h, const volatile uint32_t* seq, uint32_t tok) {
+  for (unsigned k = 1; (int32_t)(*seq - tok) < 0; k++) {
     if ((k & 1023) == 0) {
       const hipError_t q = hipStreamQuery(h->st);
       if (q == hipErrorNotReady) continue;
       if (q != hipSuccess) HIP_OK(q);
-      if (*seq != tok) return fail(FS_E_HIP, "scalars were not published%s");
+      if ((int32_t)(*seq - tok) < 0) return fail(FS_E_HIP, "the stream drained without a result%s");
       break;
     }
   }
   std::atomic_thread_fence(std::memory_order_acquire);
+  return 0;
+}
+
+// Waits until the last publication enqueued (k_publish) has reached host
+// memory, and copies it to h_sc.
+int wait_published(fs_handle* h) {
+  if (wait_count(h, &h->h_pub->pub_seq, h->pub_tok)) return FS_E_HIP;
   memcpy(h->h_sc, const_cast<const DevScalars*>(h->h_pub), sizeof(DevScalars));
   return 0;
 }
@@ -305,6 +318,82 @@ int sync_scalars(fs_handle* h) {
   enqueue_publish(h);
   HIP_OK(hipGetLastError());
   return wait_published(h);
+}
+
+// The handle's pinned host memory: published scalars, their mirror, the count
+// of field pieces, the pieces.  A piece holds whole rows, at most kIoPiece
+// doubles (or one row): small enough that copying it out of the pinned memory
+// overlaps the next piece's transfer, and that creating a handle does not pay
+// for pinning whole planes.
+constexpr size_t kIoPiece = 1 << 17;
+hipError_t alloc_pinned(fs_handle* h) {
+  const size_t sc = (sizeof(DevScalars) + 255) / 256 * 256;
+  const size_t rows = std::max<size_t>(1, std::min<size_t>(h->by + 2, kIoPiece / h->P));
+  h->io_cap = (rows * h->P + 1) / 2 * 2;
+  const size_t pieces = rows * h->P < h->PL ? 2 : 1;
+  const size_t bytes = 2 * sc + 256 + pieces * h->io_cap * sizeof(double);
+  hipError_t e = hipHostMalloc(&h->h_pin, bytes, hipHostMallocMapped | hipHostMallocCoherent);
+  if (e != hipSuccess) return e;
+  char* d = nullptr;
+  if ((e = hipHostGetDevicePointer((void**)&d, h->h_pin, 0)) != hipSuccess) return e;
+  memset(h->h_pin, 0, 2 * sc + 256);  // publication count 0, as *d_pubcnt; no piece yet
+  h->h_pub = (DevScalars*)h->h_pin;
+  h->d_pub = (DevScalars*)d;
+  h->h_sc = (DevScalars*)(h->h_pin + sc);
+  h->h_iof = (uint32_t*)(h->h_pin + 2 * sc);
+  h->d_iof = (uint32_t*)(d + 2 * sc);
+  h->h_io = (double*)(h->h_pin + 2 * sc + 256);
+  h->d_io = (double*)(d + 2 * sc + 256);
+  return hipSuccess;
+}
+
+// One plane between the device and the caller's array (leading dimension ld),
+// piece by piece: the copy of a piece between the pinned memory and the array
+// overlaps the transfer of the next.  A read into a fresh array: 64^2 26 us, 512^2
+// 135 us, 2048^2 2.4 ms, which is the array's page faults; through the
+// runtime's pageable copy and a second host copy 26 us, 209 us, 4.2 ms.  Pieces
+// a quarter the size take 512^2 to 165 us, twice the size 130 us.
+int field_io(fs_handle* h, double* dev, double* host, int32_t ld, bool out) {
+  const size_t P = h->P, rows = h->io_cap / P, ny = (size_t)h->by + 2;
+  const size_t n = (ny + rows - 1) / rows;
+  auto count = [&](size_t c) { return std::min(rows, ny - c * rows); };
+  auto half = [&](double* io, size_t c) { return io + (c & 1) * h->io_cap; };
+  auto copy = [&](size_t c) {
+    double *a = half(h->h_io, c), *b = host + c * rows * (size_t)ld;
+    if ((size_t)ld == P) {
+      memcpy(out ? b : a, out ? a : b, count(c) * P * sizeof(double));
+      return;
+    }
+    for (size_t r = 0; r < count(c); r++)
+      memcpy(out ? b + r * ld : a + r * P, out ? a + r * P : b + r * ld, P * sizeof(double));
+  };
+  auto transfer = [&](size_t c) {
+    double *a = half(h->d_io, c), *b = dev + c * rows * P;
+    launch_io(out ? b : a, out ? a : b, (int)(count(c) * P), out, h->d_pubcnt + 32, h->d_iof,
+              ++h->io_tok, h->st);
+  };
+  if (!out) {
+    // (returns with the last pieces in flight: what follows on the stream, and
+    // the next use of the pinned memory, waits for them)
+    for (size_t c = 0; c < n; c++) {
+      // both halves free before the first piece, then this one's last reader
+      if (c != 1 && wait_count(h, h->h_iof, c ? h->io_tok - 1 : h->io_tok)) return FS_E_HIP;
+      copy(c);
+      transfer(c);
+    }
+    HIP_OK(hipGetLastError());
+    return 0;
+  }
+  const uint32_t tok = h->io_tok;
+  for (size_t c = 0; c < n && c < 2; c++) transfer(c);
+  HIP_OK(hipGetLastError());
+  for (size_t c = 0; c < n; c++) {
+    if (wait_count(h, h->h_iof, tok + 1 + (uint32_t)c)) return FS_E_HIP;
+    copy(c);
+    if (c + 2 < n) transfer(c + 2);
+  }
+  HIP_OK(hipGetLastError());
+  return 0;
 }
 
 int push_scalars(fs_handle* h) {
@@ -1986,17 +2075,13 @@ int fs_create(const fs_grid_desc* g, const fs_params* p, fs_handle** out) {
       bad(hipMalloc(&h->d_part, 3 * h->npart * 8 * sizeof(double))) ||
       bad(hipMalloc(&h->d_lspart, 9 * kMaxPartials * sizeof(double))) ||
       bad(hipMalloc(&h->d_sc, sizeof(DevScalars))) ||
-      bad(hipHostMalloc(&h->h_sc, sizeof(DevScalars), hipHostMallocDefault)) ||
-      bad(hipHostMalloc(&h->h_pub, sizeof(DevScalars),
-                        hipHostMallocMapped | hipHostMallocCoherent)) ||
-      bad(hipHostGetDevicePointer((void**)&h->d_pub, h->h_pub, 0)) ||
+      bad(alloc_pinned(h)) ||
       bad(hipMalloc(&h->d_pubcnt, 256)) || bad(hipMemset(h->d_pubcnt, 0, 256)) ||
       bad(hipMalloc(&h->d_pois, kPois * PL * sizeof(double))) ||
       (g->rwall && bad(hipMalloc(&h->d_sig, 8 * ((size_t)bx + 2) * sizeof(double))))) {
     fs_destroy(h);
     return FS_E_HIP;
   }
-  memset(h->h_pub, 0, sizeof(DevScalars));  // publication count 0, as *d_pubcnt
   // sfc_init (sfc_lib.F90:82-90): the wall starts uncharged
   if (h->d_sig) (void)hipMemsetAsync(h->d_sig, 0, 8 * ((size_t)bx + 2) * sizeof(double), h->st);
   if (p->debug_keep_k) {
@@ -2067,7 +2152,6 @@ int fs_create(const fs_grid_desc* g, const fs_params* p, fs_handle** out) {
     fs_destroy(h);
     return FS_E_HIP;
   }
-  h->stage_buf.resize(PL);
   if (build_arg_tables(h) || fs_init_uniform(h) != 0 || choose_stage_tile(h)) {
     fs_destroy(h);
     return FS_E_HIP;
@@ -2091,8 +2175,7 @@ int fs_destroy(fs_handle* h) {
   (void)hipFree(h->d_part);
   (void)hipFree(h->d_lspart);
   (void)hipFree(h->d_sc);
-  (void)hipHostFree(h->h_sc);
-  if (h->h_pub) (void)hipHostFree(h->h_pub);
+  if (h->h_pin) (void)hipHostFree(h->h_pin);
   (void)hipFree(h->d_pubcnt);
   (void)hipFree(h->d_pois);
   (void)hipFree(h->d_dbg);
@@ -2162,8 +2245,6 @@ int fs_set_field(fs_handle* h, int32_t field, int32_t level, const double* host,
   if (ld < h->P) return fail(FS_E_ARG, "ld < nx+2%s");
   double* d = field_dev(h, field, level, true);
   if (!d) return fail(FS_E_ARG, "bad field/level%s");
-  for (int j = 0; j < h->by + 2; j++)
-    memcpy(&h->stage_buf[(size_t)j * h->P], host + (size_t)j * ld, h->P * sizeof(double));
   if (field <= FS_NM && (level == 1 || level == 2) && h->alias) {
     // level 1 stops aliasing level 2 (a write to either would change both):
     // give it its own copy first
@@ -2172,7 +2253,7 @@ int fs_set_field(fs_handle* h, int32_t field, int32_t level, const double* host,
                             hipMemcpyDeviceToDevice, h->st));
     h->alias = false;
   }
-  return upload(h, d, h->stage_buf.data(), h->PL);
+  return field_io(h, d, const_cast<double*>(host), ld, false);
 }
 
 int fs_get_field(const fs_handle* h, int32_t field, int32_t level, double* host, int32_t ld) {
@@ -2188,13 +2269,7 @@ int fs_get_field(const fs_handle* h, int32_t field, int32_t level, double* host,
   if (ld < h->P) return fail(FS_E_ARG, "ld < nx+2%s");
   double* d = field_dev(h, field, level, false);
   if (!d) return fail(FS_E_ARG, "bad field/level%s");
-  fs_handle* hm = const_cast<fs_handle*>(h);
-  HIP_OK(hipMemcpyAsync(hm->stage_buf.data(), d, h->PL * sizeof(double), hipMemcpyDeviceToHost,
-                        h->st));
-  HIP_OK(hipStreamSynchronize(h->st));
-  for (int j = 0; j < h->by + 2; j++)
-    memcpy(host + (size_t)j * ld, &hm->stage_buf[(size_t)j * h->P], h->P * sizeof(double));
-  return 0;
+  return field_io(const_cast<fs_handle*>(h), d, host, ld, true);
 }
 
 static int set_all_levels(fs_handle* h, int sp, const std::vector<double>& v) {
@@ -2417,87 +2492,111 @@ int fs_lapl_assemble(fs_handle* h, double* b, double* A5) {
   return check_status(h);
 }
 
-int fs_eval_fits(double p, int32_t n, const double* T, double* out) {
-  if (n <= 0) return 0;
-  FsPhys K;
-  fs_phys_init(&K, p, 0.1);
-  double *dT = nullptr, *dO = nullptr;
-  HIP_OK(hipMalloc(&dT, n * sizeof(double)));
-  HIP_OK(hipMalloc(&dO, 12 * (size_t)n * sizeof(double)));
-  HIP_OK(hipMemcpy(dT, T, n * sizeof(double), hipMemcpyHostToDevice));
-  launch_eval_fits(K, dT, dO, n, nullptr);
-  HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpy(out, dO, 12 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
-  (void)hipFree(dT);
-  (void)hipFree(dO);
-  return 0;
-}
-
-static int eval_flux_common(int32_t n, const double* a, double* out, int dfdph) {
-  if (n <= 0) return 0;
-  FsPhys K;
-  fs_phys_init(&K, 10.0, 0.1);
-  double *dA = nullptr, *dO = nullptr;
-  HIP_OK(hipMalloc(&dA, 7 * (size_t)n * sizeof(double)));
-  HIP_OK(hipMalloc(&dO, (size_t)n * sizeof(double)));
-  HIP_OK(hipMemcpy(dA, a, 7 * (size_t)n * sizeof(double), hipMemcpyHostToDevice));
-  launch_eval_flux(K, dA, dO, n, dfdph, nullptr);
-  HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpy(out, dO, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
-  (void)hipFree(dA);
-  (void)hipFree(dO);
-  return 0;
-}
-
-int fs_eval_flux(int32_t n, const double* a, double* out) { return eval_flux_common(n, a, out, 0); }
-int fs_eval_dfdph(int32_t n, const double* a, double* out) {
-  return eval_flux_common(n, a, out, 1);
-}
-
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// Staging of fs_eval_flux_noalloc: a file-scope device array instead of the
-// per-call hipMalloc of eval_flux_common.  Each device holds its own copy for
-// the life of the process; its address comes from hipGetSymbolAddress once per
-// device (the array's name is a host-side stand-in, never a device address).
+// Staging of the flux and fit evaluations: a file-scope device array instead
+// of an allocation per call (two hipMalloc and two hipFree took half of a small
+// call's 39 us; it takes 19 us).  Each device holds its own copy for the life of
+// the process; its address comes from hipGetSymbolAddress once per device (the
+// array's name is a host-side stand-in, never a device address).
 namespace {
 constexpr size_t kNoAllocScratchBytes = (size_t)2 << 20;  // 2 MiB per device
-constexpr int32_t kNoAllocMaxN = (int32_t)(kNoAllocScratchBytes / (8 * sizeof(double)));
+constexpr size_t kScratchDoubles = kNoAllocScratchBytes / sizeof(double);
+constexpr int32_t kNoAllocMaxN = (int32_t)(kScratchDoubles / 8);
 constexpr int kNoAllocMaxDevices = 64;
 std::mutex g_noalloc_mu;
 double* g_noalloc_ptr[kNoAllocMaxDevices];  // device address of `scratch`, per device
 }  // namespace
 
-static __device__ __align__(256) double scratch[kNoAllocScratchBytes / sizeof(double)];
+static __device__ __align__(256) double scratch[kScratchDoubles];
+
+namespace {
+// The current device's scratch (the caller holds g_noalloc_mu).
+int scratch_ptr(double** out) {
+  int dev = -1;
+  HIP_OK(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kNoAllocMaxDevices) return fail(FS_E_ARG, "device id out of range%s");
+  double*& ptr = g_noalloc_ptr[dev];
+  if (!ptr) {
+    HIP_OK(hipGetSymbolAddress((void**)&ptr, HIP_SYMBOL(scratch)));
+    if (!ptr) return fail(FS_E_HIP, "no device address for the staging array%s");
+  }
+  *out = ptr;
+  return 0;
+}
+
+// ni inputs and no outputs per entry: to the device, launch(in, out), back.
+// Up to kEvalInline inputs travel in the launch's arguments instead of a copy.
+template <class L, class LV>
+int eval_staged(double* d, int32_t n, int ni, int no, const double* a, double* out, L&& launch,
+                LV&& launch_inline) {
+  double *dA = d, *dO = d + (size_t)ni * n;
+  if ((size_t)ni * n <= (size_t)kEvalInline) {
+    EvalInline v;
+    memcpy(v.a, a, (size_t)ni * n * sizeof(double));
+    launch_inline(v, dO);
+  } else {
+    HIP_OK(hipMemcpy(dA, a, (size_t)ni * n * sizeof(double), hipMemcpyHostToDevice));
+    launch(dA, dO);
+  }
+  HIP_OK(hipGetLastError());
+  HIP_OK(hipMemcpy(out, dO, (size_t)no * n * sizeof(double), hipMemcpyDeviceToHost));
+  return 0;
+}
+template <class L, class LV>
+int eval_any(int32_t n, int ni, int no, const double* a, double* out, L&& launch,
+             LV&& launch_inline) {
+  const size_t len = (size_t)(ni + no) * n;
+  int dev = -1;
+  HIP_OK(hipGetDevice(&dev));
+  if (len <= kScratchDoubles && dev < kNoAllocMaxDevices) {
+    // calls in this process are serialised: they share the device's one array
+    std::lock_guard<std::mutex> lock(g_noalloc_mu);
+    double* d = nullptr;
+    if (int e = scratch_ptr(&d)) return e;
+    return eval_staged(d, n, ni, no, a, out, launch, launch_inline);
+  }
+  double* d = nullptr;
+  HIP_OK(hipMalloc(&d, len * sizeof(double)));
+  const int e = eval_staged(d, n, ni, no, a, out, launch, launch_inline);
+  (void)hipFree(d);
+  return e;
+}
+
+int eval_flux_common(int32_t n, const double* a, double* out, int dfdph) {
+  FsPhys K;
+  fs_phys_init(&K, 10.0, 0.1);
+  return eval_any(
+      n, 7, 1, a, out, [&](const double* i, double* o) { launch_eval_flux(K, i, o, n, dfdph, nullptr); },
+      [&](const EvalInline& v, double* o) { launch_eval_flux_inline(K, v, o, n, dfdph, nullptr); });
+}
+}  // namespace
 
 extern "C" {
+
+int fs_eval_fits(double p, int32_t n, const double* T, double* out) {
+  if (n <= 0) return 0;
+  FsPhys K;
+  fs_phys_init(&K, p, 0.1);
+  return eval_any(
+      n, 1, 12, T, out, [&](const double* i, double* o) { launch_eval_fits(K, i, o, n, nullptr); },
+      [&](const EvalInline& v, double* o) { launch_eval_fits_inline(K, v, o, n, nullptr); });
+}
+
+int fs_eval_flux(int32_t n, const double* a, double* out) {
+  return n <= 0 ? 0 : eval_flux_common(n, a, out, 0);
+}
+int fs_eval_dfdph(int32_t n, const double* a, double* out) {
+  return n <= 0 ? 0 : eval_flux_common(n, a, out, 1);
+}
 
 int fs_eval_flux_noalloc(int32_t n, const double* a, double* out, int32_t dfdph) {
   if (n < 0 || n > kNoAllocMaxN)
     return fail(FS_E_ARG, "fs_eval_flux_noalloc: n must lie in 0..%s%d", "", kNoAllocMaxN);
   if (n == 0) return 0;
   if (!a || !out) return fail(FS_E_ARG, "null argument%s");
-  int dev = -1;
-  HIP_OK(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kNoAllocMaxDevices) return fail(FS_E_ARG, "device id out of range%s");
-  // calls in this process are serialised: they share the device's one array
-  std::lock_guard<std::mutex> lock(g_noalloc_mu);
-  double* ptr = g_noalloc_ptr[dev];
-  if (!ptr) {
-    HIP_OK(hipGetSymbolAddress((void**)&ptr, HIP_SYMBOL(scratch)));
-    if (!ptr) return fail(FS_E_HIP, "no device address for the staging array%s");
-    g_noalloc_ptr[dev] = ptr;
-  }
-  FsPhys K;
-  fs_phys_init(&K, 10.0, 0.1);
-  double* dA = ptr;                    // 7 n doubles of arguments
-  double* dO = ptr + 7 * (size_t)n;    // n doubles of results
-  HIP_OK(hipMemcpy(dA, a, 7 * (size_t)n * sizeof(double), hipMemcpyHostToDevice));
-  launch_eval_flux(K, dA, dO, n, dfdph ? 1 : 0, nullptr);
-  HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpy(out, dO, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
-  return 0;
+  return eval_flux_common(n, a, out, dfdph ? 1 : 0);
 }
 
 int fs_time_kernel(fs_handle* h, int32_t which, int32_t n, double* avg_ms) {

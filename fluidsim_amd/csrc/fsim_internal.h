@@ -360,6 +360,19 @@ void launch_mgpcg_pq(const MgPcgArgs& a, hipStream_t s);
 void launch_mgpcg_xr(const MgPcgArgs& a, hipStream_t s);
 void launch_fill(double* p, double v, size_t n, hipStream_t s);
 void launch_copy(const double* a, double* b, size_t n2, hipStream_t s);
+// n doubles from src to dst, of which the host's side (dst if out, otherwise
+// src) is pinned and 16-byte aligned, then seq into *flag; *done is 0 between uses
+void launch_io(const double* src, double* dst, int n, bool out, unsigned* done, uint32_t* flag,
+               uint32_t seq, hipStream_t s);
+// inputs of a small evaluation, passed in the launch's arguments
+constexpr int kEvalInline = 112;
+struct EvalInline {
+  double a[kEvalInline];
+};
+void launch_eval_fits_inline(const FsPhys& K, const EvalInline& T, double* out, int n,
+                             hipStream_t s);
+void launch_eval_flux_inline(const FsPhys& K, const EvalInline& a, double* out, int n, int dfdph,
+                             hipStream_t s);
 void launch_eval_fits(const FsPhys& K, const double* T, double* out, int n, hipStream_t s);
 void launch_eval_flux(const FsPhys& K, const double* a, double* out, int n, int dfdph,
                       hipStream_t s);

@@ -3311,12 +3311,42 @@ __global__ void k_fill(double* p, double v, size_t n) {
   if (i < n) p[i] = v;
 }
 
-__global__ void k_eval_fits(FsPhys K, const double* T, double* out, int n) {
-  int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= n) return;
-  double t = T[m], v = t * K.ph0, xa = fit_x(v), xs = fit_x_stage(v);
-  Rates R = cell_rates(K, v, xs);  // as the stage kernel evaluates them
-  double* o = out + 12 * (size_t)m;
+// n doubles between the device and pinned host memory (fs_set_field,
+// fs_get_field), in pairs: the pinned side, 16-byte aligned, takes one access a
+// pair.  The last workgroup to finish (*done counts them and ends at zero)
+// writes the piece's number to *flag, which the host polls: a second kernel
+// for that took another 5 us a piece.
+template <bool kOut>
+__global__ void __launch_bounds__(256) k_io(const double* __restrict__ src,
+                                            double* __restrict__ dst, int n, unsigned* done,
+                                            uint32_t* flag, uint32_t seq) {
+  const int step = (int)gridDim.x * 512;
+  for (int k = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 2; k < n; k += step) {
+    if (k + 1 < n) {
+      if (kOut) {
+        *reinterpret_cast<double2*>(dst + k) = make_double2(src[k], src[k + 1]);
+      } else {
+        const double2 v = *reinterpret_cast<const double2*>(src + k);
+        dst[k] = v.x;
+        dst[k + 1] = v.y;
+      }
+    } else {
+      dst[k] = src[k];
+    }
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(done, 1u) == gridDim.x - 1) {
+    *done = 0;
+    __threadfence_system();
+    *reinterpret_cast<volatile uint32_t*>(flag) = seq;
+    __threadfence_system();
+  }
+}
+
+__device__ __forceinline__ void eval_fits_body(const FsPhys& K, double t, double* o) {
+  const double v = t * K.ph0, xa = fit_x(v), xs = fit_x_stage(v);
+  const Rates R = cell_rates(K, v, xs);  // as the stage kernel evaluates them
   o[0] = mue_of_x(K, xa);
   o[1] = mut_of_x(K, xa);
   o[2] = de_of_x(K, xa);
@@ -3330,14 +3360,27 @@ __global__ void k_eval_fits(FsPhys K, const double* T, double* out, int n) {
   o[10] = mue_of_x_folded(K, xs);  // the stage kernel's mobility and diffusion
   o[11] = de_of_x_folded(K, xs);
 }
+__global__ void k_eval_fits(FsPhys K, const double* T, double* out, int n) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < n) eval_fits_body(K, T[m], out + 12 * (size_t)m);
+}
+__global__ void k_eval_fits_inline(FsPhys K, EvalInline T, double* out, int n) {
+  const int m = threadIdx.x;
+  if (m < n) eval_fits_body(K, T.a[m], out + 12 * (size_t)m);
+}
 
-__global__ void k_eval_flux(FsPhys K, const double* a, double* out, int n, int dfdph) {
-  int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= n) return;
-  const double* v = a + 7 * (size_t)m;
+__device__ __forceinline__ double eval_flux_body(const FsPhys& K, const double* v, int dfdph) {
   double f, df;
   sg_flux_dfdph(K, v[0], v[1], v[2], v[3], v[4], v[5], v[6], f, df);
-  out[m] = dfdph ? df : sg_flux(K, v[0], v[1], 1.0 / v[1], v[2], v[3], v[4], v[5], v[6]);
+  return dfdph ? df : sg_flux(K, v[0], v[1], 1.0 / v[1], v[2], v[3], v[4], v[5], v[6]);
+}
+__global__ void k_eval_flux(FsPhys K, const double* a, double* out, int n, int dfdph) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < n) out[m] = eval_flux_body(K, a + 7 * (size_t)m, dfdph);
+}
+__global__ void k_eval_flux_inline(FsPhys K, EvalInline a, double* out, int n, int dfdph) {
+  const int m = threadIdx.x;
+  if (m < n) out[m] = eval_flux_body(K, a.a + 7 * m, dfdph);
 }
 
 // ---------------------------------------------------------------------------
@@ -3609,6 +3652,20 @@ void launch_copy(const double* a, double* b, size_t n2, hipStream_t s) {
 void launch_fill(double* p, double v, size_t n, hipStream_t s) {
   if (n == 0) return;
   hipLaunchKernelGGL(k_fill, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, v, n);
+}
+void launch_io(const double* src, double* dst, int n, bool out, unsigned* done, uint32_t* flag,
+               uint32_t seq, hipStream_t s) {
+  const int nb = (n + 511) / 512;
+  auto k = out ? k_io<true> : k_io<false>;
+  hipLaunchKernelGGL(k, dim3(nb < 256 ? nb : 256), dim3(256), 0, s, src, dst, n, done, flag, seq);
+}
+void launch_eval_fits_inline(const FsPhys& K, const EvalInline& T, double* out, int n,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(k_eval_fits_inline, dim3(1), dim3(kEvalInline), 0, s, K, T, out, n);
+}
+void launch_eval_flux_inline(const FsPhys& K, const EvalInline& a, double* out, int n, int dfdph,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(k_eval_flux_inline, dim3(1), dim3(64), 0, s, K, a, out, n, dfdph);
 }
 void launch_eval_fits(const FsPhys& K, const double* T, double* out, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_eval_fits, dim3((n + 255) / 256), dim3(256), 0, s, K, T, out, n);

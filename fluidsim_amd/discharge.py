@@ -87,7 +87,7 @@ class Discharge:
 
     # ---- module arrays ----
     def get(self, name: str, level: int = 1) -> np.ndarray:
-        out = np.zeros((self.ny + 2, self.P))
+        out = np.empty((self.ny + 2, self.P))
         _L.check(_L.load().fs_get_field(self.h, _L.FIELDS[name], level, _dp(out), self.P))
         return out
 
@@ -227,20 +227,20 @@ def constants(p_torr=10.0, gam=0.1) -> np.ndarray:
 
 def eval_fits(T, p_torr=10.0) -> np.ndarray:
     T = np.ascontiguousarray(T, dtype=np.float64)
-    out = np.zeros((T.size, 12))
+    out = np.empty((T.size, 12))
     _L.check(_L.load().fs_eval_fits(p_torr, T.size, _dp(T), _dp(out)))
     return out
 
 
 def eval_flux(args) -> np.ndarray:
     a = np.ascontiguousarray(args, dtype=np.float64).reshape(-1, 7)
-    out = np.zeros(a.shape[0])
+    out = np.empty(a.shape[0])
     _L.check(_L.load().fs_eval_flux(a.shape[0], _dp(a), _dp(out)))
     return out
 
 
 def eval_dfdph(args) -> np.ndarray:
     a = np.ascontiguousarray(args, dtype=np.float64).reshape(-1, 7)
-    out = np.zeros(a.shape[0])
+    out = np.empty(a.shape[0])
     _L.check(_L.load().fs_eval_dfdph(a.shape[0], _dp(a), _dp(out)))
     return out
