@@ -35,15 +35,28 @@ static_assert(3 * (kSNT + kSNT / 4 + kSNT / 16 + kSNT / 64) <= 4 * kNF, "assembl
 constexpr int kNW = kNT / 64;
 constexpr int kPcgSmallPlane = 5120;  // LDS doubles of k_pcg_small's padded plane (two dimensions)
 constexpr int kSNW = kSNT / 64;
+// Tiles of the stage and assembly kernels take more waves than cells where a
+// launch has at most this many, the card's CUs: each then has a CU to itself
+// and is bound by the latency of its phases, two trips each of some waves for
+// the halo and the outer faces.  A pass at 64^2 takes 441 us instead of 464
+// (five stage launches and the assembly), at 100 x 75 637 instead of 660; with
+// more tiles the waves compete and the narrow form stays.
+constexpr int kWideBlocks = 256;
 
 // The stage kernel's tile: kTX x TY cells (TY = 4, 8 or 16, chosen per grid by
 // timing them), one thread per cell, a one-cell halo, its x and y faces.  Its
 // error sums are reduced per group of kStageRows rows (a divisor of every TY).
-template <int TY>
+//
+// kWide: a wave per started 64 x faces and per 64 y faces (ten for 64x4 cells
+// instead of four), so that the cells of tile and halo, then all faces, take
+// one trip of every thread and one barrier fewer, for twice the face buffer.
+template <int TY, bool kWide = false>
 struct StageTile {
-  static constexpr int kNT = kTX * TY, kNW = kNT / 64, kHY = TY + 2, kNH = kHX * kHY;
+  static constexpr int kHY = TY + 2, kNH = kHX * kHY;
   static constexpr int kNFX = (kTX + 1) * TY, kNFY = kTX * (TY + 1);
   static constexpr int kNF = kNFX > kNFY ? kNFX : kNFY;
+  static constexpr int kY0 = (kNFX + 63) / 64 * 64;  // kWide: thread of the first y face
+  static constexpr int kNT = kWide ? kY0 + kNFY : kTX * TY, kNW = kNT / 64;
 };
 
 // Device pointers held in argument blocks in device memory are generic
@@ -229,14 +242,20 @@ __device__ __forceinline__ Flux4 interior_face(const FsPhys& K, double E, double
 
 // ---------------------------------------------------------------------------
 // one instance per kernel: the LDS arrays declared here then belong to one kernel each
-template <int kInstance, int TY>
+template <int kInstance, int TY, bool kWide = false>
 __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, int bid, int nb) {
-  using ST = StageTile<TY>;
+  using ST = StageTile<TY, kWide>;
   __shared__ double s_ni[ST::kNH], s_ne[ST::kNH], s_nt[ST::kNH], s_nm[ST::kNH], s_ph[ST::kNH];
   __shared__ double s_te[ST::kNH], s_mue[ST::kNH], s_de[ST::kNH], s_xa[ST::kNH];
   __shared__ double s_f[4][ST::kNF];
+  __shared__ double s_y[kWide ? 4 : 1][kWide ? ST::kNFY : 1];
   __shared__ double s_red[8 * ST::kNW];
   __shared__ int s_bad;
+  // the y faces' fluxes: their own buffer, or that of the x faces once read
+  auto fy_ = [&](int q, int f) -> double& {
+    if constexpr (kWide) return s_y[q][f];
+    else return s_f[q][f];
+  };
 
   const Geo& G = A.G;
   const int bx = G.bx, by = G.by, P = G.P;
@@ -299,7 +318,8 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
   // overlaps the flux phases
   const int tx = threadIdx.x % kTX, ty = threadIdx.x / kTX;
   const int ci = i0 + tx, cj = j0 + ty;
-  const bool valid = (ci < bx) && (cj < by);
+  const bool cell = !kWide || threadIdx.x < kTX * TY;
+  const bool valid = cell && (ci < bx) && (cj < by);
   const size_t mc = (size_t)(cj + 1) * P + (ci + 1);
   const int stage = A.stage;
   double pn3[4] = {0, 0, 0, 0}, pk1[4] = {0, 0, 0, 0}, pk3[4] = {0, 0, 0, 0},
@@ -382,13 +402,13 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
     s_f[2][f] = F.t;
     s_f[3][f] = F.m;
   }
-  __syncthreads();
+  if constexpr (!kWide) __syncthreads();
 
   // ---- phase 3a: x divergence per cell (kept in registers)
   const int hc = (ty + 1) * kHX + tx + 1;
   double dfx[4] = {0, 0, 0, 0}, feX = 0, exA = 0, mue2 = 0;
   int typx = 0;
-  if (valid) {
+  auto x_div = [&]() {
     typx = ci == 0 ? gld(G.ltype, cj) : (ci == bx - 1 ? gld(G.rtype, cj) : 0);
     int fL = ty * (kTX + 1) + tx, fR = fL + 1;
     double rdlx = gld(G.rdlx, ci);
@@ -411,11 +431,15 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
     if (typx == 2) mue2 = s_mue[hc];
     else if (typx == 1) mue2 = 0.0;
     else mue2 = 5e-1 * (s_mue[hc] + s_mue[hc + 1]);
+  };
+  if constexpr (!kWide) {
+    if (valid) x_div();
+    __syncthreads();
   }
-  __syncthreads();
 
   // ---- phase 2b: y faces (bottom face of rows j0..j0+TY, columns i0..i0+TX-1)
-  for (int f = threadIdx.x; f < ST::kNFY; f += ST::kNT) {
+  for (int f = kWide ? (int)threadIdx.x - ST::kY0 : threadIdx.x; f < ST::kNFY; f += ST::kNT) {
+    if (kWide && f < 0) break;  // (a wave of x faces)
     int fx = f % kTX, fy = f / kTX;
     int fci = i0 + fx, fj = j0 + fy;
     Flux4 F = {0, 0, 0, 0};
@@ -438,12 +462,13 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
       F.t = sg_flux(K, E, h, rh, -1.0, mut_of_x(K, xa), dt_of_x(K, xa), s_nt[hL], 0.0);
       F.m = K.Dm * s_nm[hL] / h;
     }
-    s_f[0][f] = F.i;
-    s_f[1][f] = F.e;
-    s_f[2][f] = F.t;
-    s_f[3][f] = F.m;
+    fy_(0, f) = F.i;
+    fy_(1, f) = F.e;
+    fy_(2, f) = F.t;
+    fy_(3, f) = F.m;
   }
   __syncthreads();
+  if (kWide && valid) x_div();
 
   // ---- phase 3b: y divergence, sources, stage slope, RK-Merson update
   double acc[4] = {0, 0, 0, 0};
@@ -457,10 +482,10 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
       double w = rdly / rj;
 #pragma unroll
       for (int s = 0; s < 4; s++)
-        dfy[s] = (s_f[s][fT] * (rp + rj) / 2.0 - s_f[s][fB] * (rj + rm) / 2.0) * w;
+        dfy[s] = (fy_(s, fT) * (rp + rj) / 2.0 - fy_(s, fB) * (rj + rm) / 2.0) * w;
     } else {
 #pragma unroll
-      for (int s = 0; s < 4; s++) dfy[s] = (s_f[s][fT] - s_f[s][fB]) * rdly;
+      for (int s = 0; s < 4; s++) dfy[s] = (fy_(s, fT) - fy_(s, fB)) * rdly;
     }
     // (one dimension: no y branch at all, typy 2 is never assigned otherwise;
     // Ey and the y fluxes stay zero, mue(2) is the x branch's)
@@ -477,7 +502,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
       eyB = -(s_ph[hc] - s_ph[hc - kHX]) * gld(G.rdy, cj);
       eyT = -(s_ph[hc + kHX] - s_ph[hc]) * gld(G.rdy, cj + 1);
     }
-    double feY = (s_f[1][fT] + s_f[1][fB]) / 2.0;
+    double feY = (fy_(1, fT) + fy_(1, fB)) / 2.0;
     double eyA = (eyB + eyT) / 2.0;
     if (typy <= 0) mue2 = 5e-1 * (s_mue[hc] + s_mue[hc + kHX]);
     else if (typy == 3) mue2 = s_mue[hc];  // get_mue(Te(2)) of the wall branch (:398)
@@ -576,7 +601,7 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
       s_red[w * 5 + 4] = tmin;
     }
     __syncthreads();
-    if ((threadIdx.x & 63) == 0 && w % kStageRows == 0 && cj < by) {
+    if (cell && (threadIdx.x & 63) == 0 && w % kStageRows == 0 && cj < by) {
       double v[5];
 #pragma unroll
       for (int k = 0; k < 5; k++) v[k] = s_red[w * 5 + k];
@@ -600,11 +625,11 @@ __device__ __forceinline__ void stage_body(const StageArgs& A, const FsPhys& K, 
 // argument block live in SGPRs and spills it to VGPR lanes).
 // gated: issued before the host has read the last pass's outcome; runs only
 // if k_accept_spec accepted that pass.
-template <int TY>
-__global__ void __launch_bounds__(kTX * TY, 4) k_stage(const StageArgs* __restrict__ A,
-                                                   const FsPhys* __restrict__ K, int gated) {
+template <int TY, bool kWide>
+__global__ void __launch_bounds__((StageTile<TY, kWide>::kNT), kWide ? 1 : 4)
+    k_stage(const StageArgs* __restrict__ A, const FsPhys* __restrict__ K, int gated) {
   if (gated && A->sc->spec == 0) return;
-  stage_body<0, TY>(*A, *K, blockIdx.x, gridDim.x);
+  stage_body<0, TY, kWide>(*A, *K, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -872,11 +897,14 @@ __device__ __forceinline__ FaceJ lapl_face(const FsPhys& K, double E, double h, 
   return F;
 }
 
-template <int kInstance>
+// kWide: a wave per started 64 cells of tile and halo (eleven instead of
+// eight), so that every phase is one trip of every thread.
+constexpr int kLaplWide = (kNH + 63) / 64 * 64;
+template <int kInstance, bool kWide = false>
 __device__ __forceinline__ void lapl_body(const LaplArgs& A, const FsPhys& K, int bid, int nb) {
   __shared__ double s_ni[kNH], s_ne[kNH], s_ph[kNH], s_te[kNH], s_mue[kNH], s_de[kNH];
   __shared__ double s_f[4][kNF];
-  __shared__ double s_red[8 * kSNW];
+  constexpr int kThreads = kWide ? kLaplWide : kSNT;
   __shared__ int s_bad;
   if (A.gate && A.sc->accept == 0) {  // the attempt was rejected: no solve
     if (bid == 0 && threadIdx.x == 0) A.sc->done = 3;
@@ -890,7 +918,7 @@ __device__ __forceinline__ void lapl_body(const LaplArgs& A, const FsPhys& K, in
   if (threadIdx.x == 0) s_bad = 0;
   __syncthreads();
 
-  for (int h = threadIdx.x; h < kNH; h += kSNT) {
+  for (int h = threadIdx.x; h < kNH; h += kThreads) {
     int hx = h % kHX, hy = h / kHX;
     int ci = i0 - 1 + hx, cj = j0 - 1 + hy;
     double vi = 0, ve = 0, vp = 0, te = 0, mue = 0, de = 0;
@@ -922,7 +950,7 @@ __device__ __forceinline__ void lapl_body(const LaplArgs& A, const FsPhys& K, in
   __syncthreads();
 
   // x faces: fluxes (laplEqn) and Jacobian terms (laplJ)
-  for (int f = threadIdx.x; f < kNFX; f += kSNT) {
+  for (int f = threadIdx.x; f < kNFX; f += kThreads) {
     int fx = f % (kTX + 1), fy = f / (kTX + 1);
     int fi = i0 + fx, cj = j0 + fy;
     FaceJ F = {0, 0, 0, 0};
@@ -965,7 +993,8 @@ __device__ __forceinline__ void lapl_body(const LaplArgs& A, const FsPhys& K, in
 
   const int tx = threadIdx.x % kTX, ty = threadIdx.x / kTX;
   const int ci = i0 + tx, cj = j0 + ty;
-  const bool valid = (ci < bx) && (cj < by);
+  const bool cell = !kWide || threadIdx.x < kSNT;
+  const bool valid = cell && (ci < bx) && (cj < by);
   const int hc = (ty + 1) * kHX + tx + 1;
   double o_d = 0.0, o_cx = 0.0, o_cy = 0.0;  // this cell's operator row, as stored
   double dflxi_x = 0, dflxe_x = 0, dfdx = 0, Cx = 0, aW = 0, aE = 0, gR = 0;
@@ -1020,7 +1049,7 @@ __device__ __forceinline__ void lapl_body(const LaplArgs& A, const FsPhys& K, in
   __syncthreads();
 
   // y faces (those on y = 0 and y = w carry nothing: type_y = -1 / 1)
-  for (int f = threadIdx.x; f < kNFY; f += kSNT) {
+  for (int f = threadIdx.x; f < kNFY; f += kThreads) {
     int fx = f % kTX, fy = f / kTX;
     int fci = i0 + fx, fj = j0 + fy;
     FaceJ F = {0, 0, 0, 0};
@@ -1152,9 +1181,11 @@ __device__ __forceinline__ void lapl_body(const LaplArgs& A, const FsPhys& K, in
     // face buffer (free once every cell has read its faces).
     double* s_lv = &s_f[0][0];
     __syncthreads();
-    s_lv[threadIdx.x] = o_d;
-    s_lv[kSNT + threadIdx.x] = o_cx;
-    s_lv[2 * kSNT + threadIdx.x] = o_cy;
+    if (cell) {
+      s_lv[threadIdx.x] = o_d;
+      s_lv[kSNT + threadIdx.x] = o_cx;
+      s_lv[2 * kSNT + threadIdx.x] = o_cy;
+    }
     __syncthreads();
     int off = 0, fnx = bx, fny = by;
     for (int q = 1; q <= A.ncl; q++) {
@@ -1195,9 +1226,10 @@ __device__ __forceinline__ void lapl_body(const LaplArgs& A, const FsPhys& K, in
   }
 }
 
-__global__ void __launch_bounds__(kSNT, 4) k_lapl(const LaplArgs* __restrict__ A,
-                                              const FsPhys* __restrict__ K) {
-  lapl_body<0>(*A, *K, blockIdx.x, gridDim.x);
+template <bool kWide>
+__global__ void __launch_bounds__(kWide ? kLaplWide : kSNT, kWide ? 1 : 4)
+    k_lapl(const LaplArgs* __restrict__ A, const FsPhys* __restrict__ K) {
+  lapl_body<0, kWide>(*A, *K, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -3541,9 +3573,13 @@ int stage_blocks(int nbx, int by, int ty) { return nbx * ((by + ty - 1) / ty); }
 void launch_stage(const StageArgs* a, const FsPhys* K, int nbx, int by, int ty, hipStream_t s,
                   int gated) {
   const dim3 g(stage_blocks(nbx, by, ty));
-  if (ty == 4) hipLaunchKernelGGL(k_stage<4>, g, dim3(kTX * 4), 0, s, a, K, gated);
-  else if (ty == 16) hipLaunchKernelGGL(k_stage<16>, g, dim3(kTX * 16), 0, s, a, K, gated);
-  else hipLaunchKernelGGL(k_stage<8>, g, dim3(kTX * 8), 0, s, a, K, gated);
+  // 64x4 tiles that each have a CU to themselves are bound by the latency of
+  // their phases; ten waves instead of four then cost nothing
+  if (ty == 4 && g.x <= (unsigned)kWideBlocks)
+    hipLaunchKernelGGL((k_stage<4, true>), g, dim3(StageTile<4, true>::kNT), 0, s, a, K, gated);
+  else if (ty == 4) hipLaunchKernelGGL((k_stage<4, false>), g, dim3(kTX * 4), 0, s, a, K, gated);
+  else if (ty == 16) hipLaunchKernelGGL((k_stage<16, false>), g, dim3(kTX * 16), 0, s, a, K, gated);
+  else hipLaunchKernelGGL((k_stage<8, false>), g, dim3(kTX * 8), 0, s, a, K, gated);
 }
 void launch_circ(const CircArgs& a, const FsPhys& K, hipStream_t s) {
   hipLaunchKernelGGL(k_circ, dim3(1), dim3(kNT), 0, s, a, K);
@@ -3567,7 +3603,9 @@ void launch_publish(const DevScalars* sc, DevScalars* pub, uint32_t* cnt, hipStr
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, sc, pub, cnt);
 }
 void launch_lapl_assemble(const LaplArgs* a, const FsPhys* K, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_lapl, dim3(nblocks), dim3(kSNT), 0, s, a, K);
+  if (nblocks <= kWideBlocks)
+    hipLaunchKernelGGL(k_lapl<true>, dim3(nblocks), dim3(kLaplWide), 0, s, a, K);
+  else hipLaunchKernelGGL(k_lapl<false>, dim3(nblocks), dim3(kSNT), 0, s, a, K);
 }
 void launch_pcg_init(const PcgArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_pcg_init, dim3(capped_grid(a.nbx * a.nby)), dim3(kNT), 0, s, a);
