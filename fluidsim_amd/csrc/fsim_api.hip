@@ -2919,19 +2919,22 @@ int fs_learn_train(fs_learn* n, int32_t steps, int32_t batch, float lr, uint64_t
                    double* loss) {
   if (!n || steps < 0 || batch <= 0) return fail(FS_E_ARG, "bad argument%s");
   if (n->net.count == 0) return fail(FS_E_ARG, "empty training set%s");
-  std::vector<int> idx(batch);
+  std::vector<int> idx;
+  std::vector<double> l;
   uint64_t s = seed;
-  for (int k = 0; k < steps; k++) {
-    for (int b = 0; b < batch; b++) {
+  for (int k0 = 0; k0 < steps; k0 += fsl::kTrainRound) {
+    const int n_now = std::min(fsl::kTrainRound, steps - k0);
+    idx.resize((size_t)n_now * batch);
+    for (int& i : idx) {
       uint64_t z = (s += 0x9e3779b97f4a7c15ull);
       z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
       z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-      idx[b] = (int)((z ^ (z >> 31)) % (uint64_t)n->net.count);
+      i = (int)((z ^ (z >> 31)) % (uint64_t)n->net.count);
     }
-    double l = 0.0;
-    if (fsl::train_step(&n->net, idx.data(), batch, lr, &l))
+    l.assign(n_now, 0.0);
+    if (fsl::train_steps(&n->net, idx.data(), n_now, batch, lr, l.data()))
       return fail(FS_E_HIP, "training step failed (batch too large?)%s");
-    if (loss) loss[k] = l;
+    if (loss) std::copy(l.begin(), l.end(), loss + k0);
   }
   return 0;
 }

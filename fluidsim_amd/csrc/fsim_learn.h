@@ -24,6 +24,8 @@ constexpr int kPadIn = 16;       // input channels as stored
 constexpr int kOutCh = 16;       // channels feeding the 1x1 output convolution
 constexpr int kAlign = 8;        // network grid sides are multiples of 8 (three poolings)
 
+constexpr int kTrainRound = 64;  // training steps enqueued before the host waits
+
 enum InMode { kPlain = 0, kPool = 1, kUpCat = 2 };
 
 // Layer table: input mode, input channels (a, b for the concatenation), output
@@ -90,8 +92,8 @@ int net_apply(Net* net, const MgLevel& L, const double* part, int nb, DevScalars
 int net_store_sample(Net* net, const MgLevel& L, hipStream_t st);
 // Regenerate the BF16 weight copies after the FP32 masters changed.
 void net_refresh(Net* net);
-// One Adam step on the samples idx[0..B) of the training set; mean loss.
-int train_step(Net* net, const int* idx, int B, float lr, double* loss);
+// Adam steps on the samples idx[step][0..B) of the training set; mean losses.
+int train_steps(Net* net, const int* idx, int steps, int B, float lr, double* loss);
 // Loss and gradient of a host batch (see fs_learn_loss_grad).
 int loss_grad(Net* net, int B, int H, int W, const float* in5, const float* rhat, const float* op,
               double* loss, float* grad, float* out);

@@ -15,6 +15,7 @@
 // FP32; weights are FP32 masters with BF16 copies.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <math.h>
 #include <string.h>
@@ -159,11 +160,10 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A) {
 constexpr int kWgradParts = 256;
 
 // Weight gradient dW[t][o][i] = sum_p x(p + tap t)[i] dpre(p)[o]: GEMM with
-// M = output channels, N = input channels, K = pixels.  Block (gx, gy, gz):
-// the pixel range of gx in steps of kWgPixels, the 16 input channels of gy,
-// the three taps of kernel row gz and every output tile (wave w takes the
-// (tap, o-tile) pairs w, w + 4, ...).  Partials per gx, reduced by
-// k_wgrad_reduce.
+// M = output channels, N = input channels, K = pixels.  Block (bx, by, bz) of a
+// layer: the pixel range of bx in steps of kWgPixels, the 16 input channels of
+// by, the three taps of kernel row bz and every output tile (wave w takes the
+// (tap, o-tile) pairs w, w + 4, ...).  Partials per bx, reduced by k_update.
 //
 // The matrix cores want four consecutive pixels of one channel per lane, the
 // activations hold the channels of one pixel together.  A step is therefore
@@ -178,11 +178,21 @@ constexpr int kWgradParts = 256;
 // samples of 64 x 64: 7-14 us per layer instead of 85-98 us when the lanes
 // gathered their operands from global memory two bytes at a time (the sums are
 // the same, bit for bit); 64-pixel steps with all nine taps: 14-29 us.
+//
+// No weight gradient is read before the last one is made, so the layers of one
+// channel count (one instance: the LDS of the output gradients) share a
+// launch at the end of the backward pass: 28, 21, 15 and 11 us at batch 16
+// instead of 6-16 us for each of the 14 layers.
 struct WgradArgs {
   ConvArgs X;            // the layer's input (mode, channels, resolution)
   const uint16_t* dp;    // dpre [N][H][W][cout]
-  int cout;
-  float* part;           // [gridDim.x][9][cout][cin]
+  int gx;                // pixel ranges
+  float* part;           // [gx][9][cout][cin]
+};
+constexpr int kWgGroup = 4;  // layers of one channel count
+struct WgradGroup {
+  WgradArgs a[kWgGroup];
+  int first[kWgGroup + 1];  // the layers' first blocks, then the block count
 };
 
 constexpr int kWgPixels = 256;             // pixels per step: 4 per (thread / 4)
@@ -197,23 +207,22 @@ __device__ __forceinline__ void transpose4(const bf4 (&v)[4], bf4 (&t)[4]) {
 }
 
 template <int MODE, int NM>
-__global__ void __launch_bounds__(256) k_wgrad(WgradArgs A) {
-  __shared__ __align__(16) uint16_t s_x[3 * 16 * kWgPitch];
-  __shared__ __align__(16) uint16_t s_d[NM * 16 * kWgPitch];
+__device__ __forceinline__ void wgrad_body(const WgradArgs& A, int bx, int by, int bz,
+                                           uint16_t* s_x, uint16_t* s_d) {
   constexpr int cout = 16 * NM, NC = (3 * NM + 3) / 4;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int kg = lane >> 4, col = lane & 15;
   const int pq = tid >> 2, cq = tid & 3;  // this thread's pixel and channel quads
   const ConvArgs& X = A.X;
   const int cin = MODE == kUpCat ? X.ca + X.cb : X.ca;
-  const int n0 = blockIdx.y * 16, row = blockIdx.z, HW = X.H * X.W;
+  const int n0 = by * 16, row = bz, HW = X.H * X.W;
   f4 acc[NC];
 #pragma unroll
   for (int j = 0; j < NC; j++) acc[j] = (f4){0.f, 0.f, 0.f, 0.f};
   const int total = X.N * HW, chunks = (total + 63) / 64;
-  const int per = (chunks + gridDim.x - 1) / gridDim.x;
-  const int pend = min(total, ((int)blockIdx.x + 1) * per * 64);  // the range's end
-  for (int ps = blockIdx.x * per * 64; ps < pend; ps += kWgPixels) {
+  const int per = (chunks + A.gx - 1) / A.gx;
+  const int pend = min(total, (bx + 1) * per * 64);  // the range's end
+  for (int ps = bx * per * 64; ps < pend; ps += kWgPixels) {
     const int p0 = ps + 4 * pq;
     bf4 x[3][4], d[NM][4], t[4];
     int n = p0 / HW, h = p0 % HW / X.W, w = p0 % HW % X.W;
@@ -265,7 +274,7 @@ __global__ void __launch_bounds__(256) k_wgrad(WgradArgs A) {
       }
     }
   }
-  float* out = A.part + (size_t)blockIdx.x * 9 * cout * cin;
+  float* out = A.part + (size_t)bx * 9 * cout * cin;
 #pragma unroll
   for (int j = 0; j < NC; j++) {
     const int c = wave + 4 * j;
@@ -277,38 +286,80 @@ __global__ void __launch_bounds__(256) k_wgrad(WgradArgs A) {
   }
 }
 
-// Sum of the ranges' partials in their order.  The chain of additions is
-// serial, the loads need not be: kWgReduceBatch of them are in flight at a
-// time (5 us for the 256 ranges of a full-resolution layer at batch 16; one by
-// one they took 58 us).
-constexpr int kWgReduceBatch = 32;
-__global__ void k_wgrad_reduce(const float* part, int nparts, int len, float* g) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= len) return;
-  float s = 0.0f;
-  int k = 0;
-  for (; k + kWgReduceBatch <= nparts; k += kWgReduceBatch) {
-    float v[kWgReduceBatch];
-#pragma unroll
-    for (int b = 0; b < kWgReduceBatch; b++) v[b] = part[(size_t)(k + b) * len + i];
-#pragma unroll
-    for (int b = 0; b < kWgReduceBatch; b++) s += v[b];
-  }
-  for (; k < nparts; k++) s += part[(size_t)k * len + i];
-  g[i] = s;
+template <int NM>
+__global__ void __launch_bounds__(256) k_wgrad(WgradGroup G) {
+  __shared__ __align__(16) uint16_t s_x[3 * 16 * kWgPitch];
+  __shared__ __align__(16) uint16_t s_d[NM * 16 * kWgPitch];
+  int l = 0;
+  while (l + 1 < kWgGroup && (int)blockIdx.x >= G.first[l + 1]) l++;
+  const WgradArgs& A = G.a[l];
+  const int b = (int)blockIdx.x - G.first[l];
+  const int ny = (A.X.mode == kUpCat ? A.X.ca + A.X.cb : A.X.ca) / 16;
+  const int bx = b % A.gx, by = b / A.gx % ny, bz = b / A.gx / ny;
+  if (A.X.mode == kPlain) wgrad_body<kPlain, NM>(A, bx, by, bz, s_x, s_d);
+  else if (A.X.mode == kPool) wgrad_body<kPool, NM>(A, bx, by, bz, s_x, s_d);
+  else wgrad_body<kUpCat, NM>(A, bx, by, bz, s_x, s_d);
 }
 
-// Adam on the FP32 masters.
-__global__ void k_adam(float* w, const float* g, float* m, float* v, int n, float lr, float b1,
-                       float b2, float c1, float c2, float eps) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+// The gradient of every parameter: the sum of its layer's partials in the
+// ranges' order; with kAdam also the step on the FP32 masters and their BF16
+// copies (wb as stored, wt with the taps flipped and the channel axes swapped).
+// The chain of additions is serial, the loads need not be: kReduceBatch of them
+// are in flight at a time.  One launch for the whole network, of 64 parameters
+// per block (layers are multiples of 64 but for the last, the output weights):
+// 10 us at batch 16, where a launch per layer took 5 us each and the step and
+// the copies 10 us more.
+constexpr int kReduceBatch = 32;
+struct Reduce {
+  int off[kLayers + 2];      // parameter offsets, then their number
+  int nparts[kLayers + 1];
+  int cin[kLayers], cout[kLayers];
+  size_t part[kLayers + 1];  // the layers' partials, [nparts][parameters]
+};
+struct AdamStep {
+  float lr, b1, b2, c1, c2, eps;
+};
+template <bool kAdam>
+__global__ void __launch_bounds__(64) k_update(Reduce R, const float* __restrict__ wpart, float* g,
+                                               float* w, float* m, float* v, uint16_t* wb,
+                                               uint16_t* wt, AdamStep S) {
+  const int i0 = blockIdx.x * 64, i = i0 + threadIdx.x;
+  int l = 0;
+  while (l < kLayers && i0 >= R.off[l + 1]) l++;
+  if (i >= R.off[kLayers + 1]) return;
+  const int len = R.off[l + 1] - R.off[l], e = i - R.off[l], nparts = R.nparts[l];
+  const float* part = wpart + R.part[l] + e;
+  float mo = 0.0f, vo = 0.0f, wo = 0.0f;
+  if (kAdam) {
+    mo = m[i];
+    vo = v[i];
+    wo = w[i];
+  }
+  float s = 0.0f;
+  int k = 0;
+  for (; k + kReduceBatch <= nparts; k += kReduceBatch) {
+    float p[kReduceBatch];
+#pragma unroll
+    for (int b = 0; b < kReduceBatch; b++) p[b] = part[(size_t)(k + b) * len];
+#pragma unroll
+    for (int b = 0; b < kReduceBatch; b++) s += p[b];
+  }
+  for (; k < nparts; k++) s += part[(size_t)k * len];
+  g[i] = s;
+  if (!kAdam) return;
+  const float mi = S.b1 * mo + (1.0f - S.b1) * s;
+  const float vi = S.b2 * vo + (1.0f - S.b2) * s * s;
   m[i] = mi;
   v[i] = vi;
-  w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+  wo -= S.lr * (mi / S.c1) / (sqrtf(vi / S.c2) + S.eps);
+  w[i] = wo;
+  const uint16_t q = f2bf(wo);
+  wb[i] = q;
+  if (l == kLayers) return;  // 1x1 output weights
+  // wt[8 - t][i][o] = w[t][o][i]
+  const int ci = R.cin[l], co = R.cout[l];
+  const int t = e / (ci * co), rem = e % (ci * co), oo = rem / ci, ii = rem % ci;
+  wt[R.off[l] + ((8 - t) * ci + ii) * co + oo] = q;
 }
 
 struct WOff {
@@ -595,39 +646,56 @@ int forward(const Net* net, const Acts& a, hipStream_t st, bool split = false) {
 
 int ceil_div(size_t a, size_t b) { return (int)((a + b - 1) / b); }
 
-template <int MODE>
-int launch_wgrad(const WgradArgs& w, dim3 g, hipStream_t st) {
-  switch (w.cout / 16) {
-    case 1: hipLaunchKernelGGL((k_wgrad<MODE, 1>), g, dim3(256), 0, st, w); return 0;
-    case 2: hipLaunchKernelGGL((k_wgrad<MODE, 2>), g, dim3(256), 0, st, w); return 0;
-    case 3: hipLaunchKernelGGL((k_wgrad<MODE, 3>), g, dim3(256), 0, st, w); return 0;
-    case 4: hipLaunchKernelGGL((k_wgrad<MODE, 4>), g, dim3(256), 0, st, w); return 0;
-  }
-  return -1;
+// Pixel ranges of layer l's weight gradient: chunks of 64 pixels, at least 4 per
+// block, at most kWgradParts blocks.
+int wgrad_ranges(const Acts& a, int l) {
+  const int gx = ceil_div((size_t)a.N * (a.H >> kNet[l].level) * (a.W >> kNet[l].level), 64 * 4);
+  return gx < 1 ? 1 : gx > kWgradParts ? kWgradParts : gx;
 }
 
-// dW of layer l into net->g, from a.dpre[l].
-int wgrad(Net* net, const Acts& a, int l, hipStream_t st) {
-  WgradArgs w;
-  w.X = fwd_args(net, a, l);
-  w.dp = a.dpre[l];
-  w.cout = kNet[l].cout;
-  w.part = net->wpart;
-  const int cin = layer_cin(l), len = 9 * w.cout * cin;
-  const int total = a.N * (a.H >> kNet[l].level) * (a.W >> kNet[l].level);
-  // pixel chunks of 64, at least 4 per block, at most kWgradParts blocks along x
-  int gx = ceil_div(total, 64 * 4);
-  const int cap = (int)(net->wpart_len / (size_t)len);
-  gx = gx < 1 ? 1 : gx > kWgradParts ? kWgradParts : gx;
-  if (gx > cap) gx = cap;
-  const dim3 g(gx, cin / 16, 3);
-  if (w.X.mode == kPlain ? launch_wgrad<kPlain>(w, g, st)
-      : w.X.mode == kPool ? launch_wgrad<kPool>(w, g, st)
-                          : launch_wgrad<kUpCat>(w, g, st))
-    return -1;
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(len, 64)), dim3(64), 0, st, net->wpart, gx,
-                     len, net->g + net->off[l]);
+// Where the layers' partial sums lie in net->wpart, which grows to hold them.
+int plan_reduce(Net* net, const Acts& a, Reduce& R) {
+  size_t o = 0;
+  for (int l = 0; l <= kLayers; l++) {
+    const int len = (int)((l < kLayers ? net->off[l + 1] : net->nparam) - net->off[l]);
+    R.off[l] = (int)net->off[l];
+    R.nparts[l] = l < kLayers ? wgrad_ranges(a, l) : ceil_div((size_t)a.N * a.H * a.W, 256);
+    R.part[l] = o;
+    o += (size_t)R.nparts[l] * len;
+    if (l < kLayers) {
+      R.cin[l] = layer_cin(l);
+      R.cout[l] = kNet[l].cout;
+    }
+  }
+  R.off[kLayers + 1] = (int)net->nparam;
+  if (o > net->wpart_len) {
+    (void)hipFree(net->wpart);
+    net->wpart = nullptr;
+    net->wpart_len = 0;
+    HIPC(hipMalloc(&net->wpart, o * sizeof(float)));
+    net->wpart_len = o;
+  }
   return 0;
+}
+
+// The partial sums of dW of every layer, from a.dpre: a launch per channel count.
+template <int NM>
+void wgrad_group(Net* net, const Acts& a, const Reduce& R, hipStream_t st) {
+  WgradGroup G;
+  memset(&G, 0, sizeof(G));
+  int k = 0, blocks = 0;
+  for (int l = 0; l < kLayers; l++) {
+    if (kNet[l].cout != 16 * NM) continue;
+    WgradArgs& w = G.a[k];
+    w.X = fwd_args(net, a, l);
+    w.dp = a.dpre[l];
+    w.gx = R.nparts[l];
+    w.part = net->wpart + R.part[l];
+    G.first[k++] = blocks;
+    blocks += w.gx * (layer_cin(l) / 16) * 3;
+  }
+  for (; k <= kWgGroup; k++) G.first[k] = blocks;
+  hipLaunchKernelGGL(k_wgrad<NM>, dim3(blocks), dim3(256), 0, st, G);
 }
 
 // Input gradient of layer l (l > 0): masked BF16 into dpre[l - 1] for plain
@@ -670,14 +738,15 @@ void refresh_bf16(Net* net, hipStream_t st) {
                      net->wb, net->wt, woff(net), (int)net->nparam);
 }
 
-// Full backward from a.dout; parameter gradients into net->g.
-int backward(Net* net, const Acts& a, hipStream_t st) {
+// Full backward from a.dout: parameter gradients into net->g and, with `adam`,
+// the step on the parameters.
+int backward(Net* net, const Acts& a, hipStream_t st, const AdamStep* adam = nullptr) {
+  Reduce R;
+  if (plan_reduce(net, a, R)) return -1;
   const int n0 = a.N * a.H * a.W;
   const float* wout = net->w + net->off[kLayers];
   hipLaunchKernelGGL(k_out_bwd, dim3(ceil_div(n0, 256)), dim3(256), 0, st, a.y[13], wout, a.dout,
-                     n0, a.dpre[13], net->wpart);
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3(1), dim3(64), 0, st, net->wpart, ceil_div(n0, 256),
-                     kOutCh, net->g + net->off[kLayers]);
+                     n0, a.dpre[13], net->wpart + R.part[kLayers]);
   // per-level scratch for the concatenated-input gradients, kept until the
   // matching skip is consumed
   float* dxcat[3];
@@ -687,9 +756,7 @@ int backward(Net* net, const Acts& a, hipStream_t st) {
     const int l = 12 - 2 * lv;
     offc += (size_t)a.N * (a.H >> lv) * (a.W >> lv) * layer_cin(l);
   }
-  for (int l = kLayers - 1; l >= 0; l--) {
-    if (wgrad(net, a, l, st)) return -1;
-    if (l == 0) break;
+  for (int l = kLayers - 1; l > 0; l--) {
     const LayerDesc& L = kNet[l];
     if (L.mode == kPlain) {
       if (dgrad(net, a, l, nullptr, st)) return -1;
@@ -711,6 +778,17 @@ int backward(Net* net, const Acts& a, hipStream_t st) {
                          a.dpre[l - 1]);
     }
   }
+  wgrad_group<1>(net, a, R, st);
+  wgrad_group<2>(net, a, R, st);
+  wgrad_group<3>(net, a, R, st);
+  wgrad_group<4>(net, a, R, st);
+  const dim3 g(ceil_div(net->nparam, 64)), b(64);
+  if (adam)
+    hipLaunchKernelGGL(k_update<true>, g, b, 0, st, R, net->wpart, net->g, net->w, net->m, net->v,
+                       net->wb, net->wt, *adam);
+  else
+    hipLaunchKernelGGL(k_update<false>, g, b, 0, st, R, net->wpart, net->g, net->w, net->m, net->v,
+                       net->wb, net->wt, AdamStep{});
   return 0;
 }
 
@@ -877,38 +955,51 @@ int net_store_sample(Net* net, const MgLevel& L, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// One training step on `B` samples (indices given), returns the mean loss.
-int train_step(Net* net, const int* idx_host, int B, float lr, double* loss) {
+// Training steps on the batches idx[step][B]; mean losses.  The steps of a round
+// (as many as the loss partials have room for) are enqueued together: their
+// indices go up once and their losses come back once, so that the host waits
+// once per round and not in every step.
+int train_steps(Net* net, const int* idx, int steps, int B, float lr, double* loss) {
   Acts& a = net->train;
   hipStream_t st = net->st;
   if (a.N != B || a.H != net->H || a.W != net->W) {
     if (acts_alloc(a, B, net->H, net->W)) return -1;
   }
-  int* d_idx = (int*)(net->lpart + kLossSlots / 2);
-  HIPC(hipMemcpyAsync(d_idx, idx_host, B * sizeof(int), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_gather, dim3(B), dim3(1024), 0, st, net->data, d_idx, net->H, net->W,
-                     a.in, a.rhat, a.op, a.scale);
-  if (forward(net, a, st)) return -1;
   const int n0 = B * net->H * net->W;
-  hipLaunchKernelGGL(k_out_fwd, dim3(ceil_div(n0, 256)), dim3(256), 0, st, a.y[13],
-                     net->w + net->off[kLayers], a.out, n0);
   const int nbl = ceil_div(n0, 256);
   if (nbl > kLossSlots / 2 || B > kLossSlots) return -1;
-  hipLaunchKernelGGL(k_loss, dim3(nbl), dim3(256), 0, st, a.out, a.rhat, a.op, B, net->H, net->W,
-                     a.dout, net->lpart);
-  if (backward(net, a, st)) return -1;
-  net->adam_t++;
-  const float b1 = 0.9f, b2 = 0.999f;
-  const float c1 = 1.0f - powf(b1, (float)net->adam_t), c2 = 1.0f - powf(b2, (float)net->adam_t);
-  hipLaunchKernelGGL(k_adam, dim3(ceil_div(net->nparam, 256)), dim3(256), 0, st, net->w, net->g,
-                     net->m, net->v, (int)net->nparam, lr, b1, b2, c1, c2, 1e-8f);
-  refresh_bf16(net, st);
-  std::vector<float> lp(nbl);
-  HIPC(hipMemcpyAsync(lp.data(), net->lpart, nbl * sizeof(float), hipMemcpyDeviceToHost, st));
-  HIPC(hipStreamSynchronize(st));
-  double s = 0.0;
-  for (float v : lp) s += v;
-  *loss = s / B;
+  int* d_idx = (int*)(net->lpart + kLossSlots / 2);
+  const int most = std::max(1, std::min(kTrainRound, std::min(kLossSlots / 2 / nbl, kLossSlots / B)));
+  std::vector<float> lp;
+  for (int k0 = 0; k0 < steps; k0 += most) {
+    const int n = std::min(most, steps - k0);
+    HIPC(hipMemcpyAsync(d_idx, idx + (size_t)k0 * B, (size_t)n * B * sizeof(int),
+                        hipMemcpyHostToDevice, st));
+    for (int k = 0; k < n; k++) {
+      hipLaunchKernelGGL(k_gather, dim3(B), dim3(1024), 0, st, net->data, d_idx + (size_t)k * B,
+                         net->H, net->W, a.in, a.rhat, a.op, a.scale);
+      if (forward(net, a, st)) return -1;
+      hipLaunchKernelGGL(k_out_fwd, dim3(ceil_div(n0, 256)), dim3(256), 0, st, a.y[13],
+                         net->w + net->off[kLayers], a.out, n0);
+      hipLaunchKernelGGL(k_loss, dim3(nbl), dim3(256), 0, st, a.out, a.rhat, a.op, B, net->H,
+                         net->W, a.dout, net->lpart + (size_t)k * nbl);
+      net->adam_t++;
+      const float b1 = 0.9f, b2 = 0.999f;
+      const AdamStep S{lr, b1, b2, 1.0f - powf(b1, (float)net->adam_t),
+                       1.0f - powf(b2, (float)net->adam_t), 1e-8f};
+      if (backward(net, a, st, &S)) return -1;
+    }
+    HIPC(hipGetLastError());
+    lp.resize((size_t)n * nbl);
+    HIPC(hipMemcpyAsync(lp.data(), net->lpart, lp.size() * sizeof(float), hipMemcpyDeviceToHost,
+                        st));
+    HIPC(hipStreamSynchronize(st));
+    for (int k = 0; k < n; k++) {
+      double s = 0.0;
+      for (int q = 0; q < nbl; q++) s += lp[(size_t)k * nbl + q];
+      loss[k0 + k] = s / B;
+    }
+  }
   return 0;
 }
 
