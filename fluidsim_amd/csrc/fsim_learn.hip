@@ -76,39 +76,68 @@ struct ConvArgs {
   int N, H, W;           // output resolution
 };
 
-// Four input channels c0..c0+3 of pixel (n, hh, ww) at the output resolution.
+// Input channels 16 cb + 4 kg .. + 3 of pixel (n, hh, ww) at the output
+// resolution: the loads (of the four pixels of a pooled input), and the value.
+// The pixel lies inside the image: a caller whose tap does not loads another
+// pixel and drops the value, since a load under a condition is a branch, which
+// ends the batch of loads in flight.
 template <int MODE>
-__device__ __forceinline__ bf4 conv_in4(const ConvArgs& A, int n, int hh, int ww, int c0) {
-  if (MODE == kPlain)
-    return *(const bf4*)(A.xa + (((size_t)n * A.H + hh) * A.W + ww) * A.ca + c0);
-  if (MODE == kPool) {
+struct ConvRaw {
+  bf4 q[MODE == kPool ? 4 : 1];
+};
+template <int MODE>
+__device__ __forceinline__ void conv_load(const ConvArgs& A, int n, int hh, int ww, int cb, int kg,
+                                          ConvRaw<MODE>& r) {
+  const int c0 = 16 * cb + 4 * kg;
+  if (MODE == kPlain) {
+    r.q[0] = *(const bf4*)(A.xa + (((size_t)n * A.H + hh) * A.W + ww) * A.ca + c0);
+  } else if (MODE == kPool) {
     const size_t W2 = 2 * (size_t)A.W;
     const size_t b = (((size_t)n * 2 * A.H + 2 * hh) * W2 + 2 * ww) * A.ca + c0;
-    const bf4 q0 = *(const bf4*)(A.xa + b), q1 = *(const bf4*)(A.xa + b + A.ca);
-    const bf4 q2 = *(const bf4*)(A.xa + b + W2 * A.ca), q3 = *(const bf4*)(A.xa + b + (W2 + 1) * A.ca);
-    bf4 r;
+    const size_t o[4] = {0, (size_t)A.ca, W2 * A.ca, (W2 + 1) * A.ca};
+#pragma unroll
+    for (int k = 0; k < (MODE == kPool ? 4 : 1); k++) r.q[k] = *(const bf4*)(A.xa + b + o[k]);
+  } else {  // (the same source for every lane: channel counts are multiples of 16)
+    const bool up = 16 * cb < A.ca;
+    const size_t pa = ((size_t)n * (A.H / 2) + hh / 2) * (A.W / 2) + ww / 2;
+    const size_t pb = ((size_t)n * A.H + hh) * A.W + ww;
+    r.q[0] = *(const bf4*)(up ? A.xa + pa * A.ca + c0 : A.xb + pb * A.cb + (c0 - A.ca));
+  }
+}
+template <int MODE>
+__device__ __forceinline__ bf4 conv_value(const ConvRaw<MODE>& r, bool ok) {
+  bf4 v = r.q[0];
+  if (MODE == kPool) {
 #pragma unroll
     for (int e = 0; e < 4; e++)
-      r[e] = (short)f2bf((bf2f((uint16_t)q0[e]) + bf2f((uint16_t)q1[e]) + bf2f((uint16_t)q2[e]) +
-                          bf2f((uint16_t)q3[e])) *
+      v[e] = (short)f2bf((bf2f((uint16_t)r.q[0][e]) + bf2f((uint16_t)r.q[MODE == kPool ? 1 : 0][e]) +
+                          bf2f((uint16_t)r.q[MODE == kPool ? 2 : 0][e]) +
+                          bf2f((uint16_t)r.q[MODE == kPool ? 3 : 0][e])) *
                          0.25f);
-    return r;
   }
-  if (c0 < A.ca)
-    return *(const bf4*)(A.xa + (((size_t)n * (A.H / 2) + hh / 2) * (A.W / 2) + ww / 2) * A.ca + c0);
-  return *(const bf4*)(A.xb + (((size_t)n * A.H + hh) * A.W + ww) * A.cb + (c0 - A.ca));
+  return ok ? v : (bf4){0, 0, 0, 0};
 }
 
 // Forward (and input-gradient) 3x3 convolution: each wave computes NT output
 // tiles of 16 channels (from tile NT * blockIdx.y on; cout = 16 * NT *
-// gridDim.y) for 16 pixels, over CB = cin / 16 input-channel blocks, fully
-// unrolled so that the operand loads of all taps are issued ahead of the MFMA
-// chain.  The network application (one sample) launches one tile per wave
-// and the output tiles along y, so that the deep layers' few pixels still
-// spread over many waves with short MFMA chains.
+// gridDim.y) for 16 pixels, over CB = cin / 16 input-channel blocks.  The
+// network application (one sample) launches one tile per wave and the output
+// tiles along y, so that the deep layers' few pixels still spread over many
+// waves with short MFMA chains.
+//
+// A layer is bound by the latency of its operand loads (the network has a
+// few thousand waves at most), so the loads of kTaps taps are issued before the
+// first product: all nine where their operands fit the registers, else a
+// kernel row, and so are those of the output's mask.  Measured against loads
+// under the taps' conditions, a few at a time: 48 channels at 16 x 16, batch
+// 16, 6.2 -> 4.8 us, the whole network on one 64 x 64 sample (25 times per 512^2
+// solve) some 14 us less.  (The weight gradients keep conditional loads: without
+// them they are 10% slower, bound by their transposes.)
+constexpr int kConvRegs = 280;  // most registers for operands in flight
 template <int MODE, int NT, int CB>
-__global__ void __launch_bounds__(256) k_conv(ConvArgs A) {
+__global__ void __launch_bounds__(256, 1) k_conv(ConvArgs A) {
   constexpr int cin = 16 * CB;
+  constexpr int kTaps = 9 * CB * (NT + (MODE == kPool ? 4 : 1)) * 2 <= kConvRegs ? 9 : 3;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int co0 = (int)blockIdx.y * NT * 16;
   const int HW = A.H * A.W, total = A.N * HW;
@@ -122,23 +151,46 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A) {
   f4 acc[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; nt++) acc[nt] = (f4){0.f, 0.f, 0.f, 0.f};
+  uint16_t mask[NT][4];  // of the outputs this lane receives
+  if (A.mask) {
 #pragma unroll
-  for (int t = 0; t < 9; t++) {
-    const int hh = h + t / 3 - 1, ww = w + t % 3 - 1;
-    const bool ok = pin && hh >= 0 && hh < A.H && ww >= 0 && ww < A.W;
-    const uint16_t* wt = A.w + ((size_t)t * A.cout + co0 + col) * cin + 4 * kg;
-    bf4 a[CB], b[CB][NT];
+    for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-    for (int cb = 0; cb < CB; cb++) {
-      a[cb] = ok ? conv_in4<MODE>(A, n, hh, ww, 16 * cb + 4 * kg) : (bf4){0, 0, 0, 0};
+      for (int i = 0; i < 4; i++) {
+        const int p = p0 + 4 * kg + i;
+        mask[nt][i] = A.mask[(size_t)(p < total ? p : p0) * A.cout + co0 + nt * 16 + col];
+      }
+  }
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++) b[cb][nt] = *(const bf4*)(wt + (size_t)nt * 16 * cin + 16 * cb);
+  for (int t0 = 0; t0 < 9; t0 += kTaps) {
+    ConvRaw<MODE> a[kTaps][CB];
+    bf4 b[kTaps][CB][NT];
+#pragma unroll
+    for (int k = 0; k < kTaps; k++) {
+      const int t = t0 + k, hh = h + t / 3 - 1, ww = w + t % 3 - 1;
+      const bool ok = hh >= 0 && hh < A.H && ww >= 0 && ww < A.W;
+      const uint16_t* wt = A.w + ((size_t)t * A.cout + co0 + col) * cin + 4 * kg;
+#pragma unroll
+      for (int cb = 0; cb < CB; cb++) {
+        conv_load<MODE>(A, n, ok ? hh : h, ok ? ww : w, cb, kg, a[k][cb]);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+          b[k][cb][nt] = *(const bf4*)(wt + (size_t)nt * 16 * cin + 16 * cb);
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);  // the products stay behind the loads
 #pragma unroll
-    for (int cb = 0; cb < CB; cb++)
+    for (int k = 0; k < kTaps; k++) {
+      const int t = t0 + k, hh = h + t / 3 - 1, ww = w + t % 3 - 1;
+      const bool ok = pin && hh >= 0 && hh < A.H && ww >= 0 && ww < A.W;
 #pragma unroll
-      for (int nt = 0; nt < NT; nt++)
-        acc[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[cb], b[cb][nt], acc[nt], 0, 0, 0);
+      for (int cb = 0; cb < CB; cb++) {
+        const bf4 av = conv_value<MODE>(a[k][cb], ok);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b[k][cb][nt], acc[nt], 0, 0, 0);
+      }
+    }
   }
 #pragma unroll
   for (int nt = 0; nt < NT; nt++)
@@ -150,7 +202,7 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A) {
       const size_t o = (size_t)p * A.cout + co;
       float v = acc[nt][i];
       if (A.relu) v = fmaxf(v, 0.0f);
-      if (A.mask && !(bf2f(A.mask[o]) > 0.0f)) v = 0.0f;
+      if (A.mask && !(bf2f(mask[nt][i]) > 0.0f)) v = 0.0f;
       if (A.y) A.y[o] = f2bf(v);
       if (A.yf) A.yf[o] = v;
     }
@@ -233,7 +285,12 @@ __device__ __forceinline__ void wgrad_body(const WgradArgs& A, int bx, int by, i
       for (int k = 0; k < 3; k++) {
         const int ww = w + k - 1;
         const bool in = p0 + e < pend && hh >= 0 && hh < X.H && ww >= 0 && ww < X.W;
-        x[k][e] = in ? conv_in4<MODE>(X, n, hh, ww, n0 + 4 * cq) : (bf4){0, 0, 0, 0};
+        x[k][e] = (bf4){0, 0, 0, 0};
+        if (in) {
+          ConvRaw<MODE> r;
+          conv_load<MODE>(X, n, hh, ww, by, cq, r);
+          x[k][e] = conv_value<MODE>(r, true);
+        }
       }
       const bool in = p0 + e < pend;
 #pragma unroll
