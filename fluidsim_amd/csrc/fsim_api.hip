@@ -740,6 +740,15 @@ size_t learned_level(const fs_handle* h) {
   return c;
 }
 
+// Whether the up step of level l makes that of level l + 1 too: the finest tile
+// level of few enough tiles whose coarse level is a tile level, then every
+// second one below.
+bool up_pair(const fs_handle* h, size_t l) {
+  size_t k = 0;
+  while (k + 1 < h->mg_first && !mg_up_pairs(h->mg[k])) k++;
+  return l >= k && l + 1 < h->mg_first && (l - k) % 2 == 0;
+}
+
 // V-cycle `it` of the multigrid-PCG (-1: the initial cycle; it >= 0: one
 // whole CG iteration, its update fused into the finest down kernel).  Only
 // the parity of `it` matters after it = 0.  With `harvest`, the residual
@@ -756,7 +765,17 @@ int launch_vcycle(fs_handle* h, int it, fsl::Net* harvest = nullptr) {
     }
   }
   launch_mg_coarse_cycle(cycle_args(h, it), h->st);
-  for (size_t l = f; l-- > 0;) launch_mg_up(mg_up_args(h, l, it), h->st);
+  for (size_t l = f; l-- > 0;) {
+    if (l > 0 && up_pair(h, l - 1)) continue;  // made by the next level's launch
+    MgArgs a = mg_up_args(h, l, it);
+    if (up_pair(h, l)) {
+      a.e2 = h->mg[l + 2].e;
+      a.P2 = h->mg[l + 2].P;
+      launch_mg_up_pair(a, h->st);
+    } else {
+      launch_mg_up(a, h->st);
+    }
+  }
   return 0;
 }
 

@@ -204,6 +204,8 @@ struct MgArgs {
   double* xs2;           // correction x2, advanced here (warm_a, warm_b)
   double* xs3;           // correction x3, advanced here (warm_c)
   const double* rhs0;    // level-0 initial test: the right-hand side (zero start)
+  const double* e2;      // up with its coarse level (pair): the correction of the level below that
+  int32_t P2, pad_2;     // ... and its row pitch
 };
 
 // Kernels whose per-block partial sums every block of the next kernel reads
@@ -352,6 +354,9 @@ void launch_mg_coarsen(const MgArgs& a, hipStream_t s);
 int mg_grid(const MgLevel& F);  // blocks (= partials) of a down/up launch
 void launch_mg_down(const MgArgs& a, hipStream_t s);
 void launch_mg_up(const MgArgs& a, hipStream_t s);
+// the up kernels of a.C and then a.F in one launch (mg_up_pairs(a.F))
+bool mg_up_pairs(const MgLevel& F);
+void launch_mg_up_pair(const MgArgs& a, hipStream_t s);
 void launch_mg_coarse_setup(const MgCycleArgs& a, hipStream_t s);
 void launch_mg_coarse_cycle(const MgCycleArgs& a, hipStream_t s);
 void launch_mgpcg_init(const MgPcgArgs& a, hipStream_t s);

@@ -21,6 +21,8 @@
 #include <hip/hip_runtime.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "fsim_internal.h"
 
 namespace {
@@ -1881,6 +1883,20 @@ __device__ __forceinline__ GsPos gs_pos(const MgLevel& F, int i0, int j0) {
   q.own = ok && q.I >= kGsH / 2 && q.I < kAgX - kGsH / 2 && q.J >= kGsH / 2 && q.J < kAgY - kGsH / 2;
   return q;
 }
+// ... of aggregate (I, J) of a region whose first cell is (i0, j0) (even).
+__device__ __forceinline__ GsPos gs_pos_at(const MgLevel& F, int I, int J, int i0, int j0,
+                                           bool act) {
+  GsPos q{};
+  q.act = act;
+  q.I = act ? I : 0;
+  q.J = act ? J : 0;
+  q.i = i0 + 2 * q.I;
+  q.j = j0 + 2 * q.J;
+  const bool ok = act && q.i >= 0 && q.i < F.nx && q.j >= 0 && q.j < F.ny;
+  const bool x1 = q.i + 1 < F.nx, y1 = q.j + 1 < F.ny;
+  q.in = ok ? 1 | (x1 ? 2 : 0) | (y1 ? 4 : 0) | (x1 && y1 ? 8 : 0) : 0;
+  return q;
+}
 // The padded index of row b's pair of children, 0 (the plane's first elements,
 // loaded and discarded) for a row outside the level.
 __device__ __forceinline__ size_t gs_row(const MgLevel& F, const GsPos& q, int b) {
@@ -2451,9 +2467,21 @@ __global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_down(MgArgs A) {
 // the tile, so that kernel (H = 5) also stages the ring around the 4-cell halo.
 // kEarly as in the down kernel: the first tile's loads before the test of
 // `done` (in bounds whatever the state).
-template <int kInstance, int H, bool kEarly>
+//
+// kPair: the coarse level's up step first, in the same launch: each tile makes
+// it on the coarse cells it reads and four rings around them (32 x 24 cells as
+// 16 x 12 aggregates), so that what a launch of its own would write is
+// recomputed in LDS, the same operations on the same values.  Where a tile has
+// a CU to itself the repeated work costs less than the launch: at
+// 256^2 over 128^2 cells 5.0 us instead of 4.7 and 4.6 us and a launch's gap, a
+// 512^2 solve 1010 instead of 1055 us.
+constexpr int kPairX = 16, kPairY = 12, kPairH = 8;  // aggregates, and cells before the tile's first
+static_assert(kPairX * kPairY <= kNT && 2 * kPairX >= kGsTX / 2 + 2 * kPairH &&
+                  2 * kPairY >= kGsTY / 2 + 2 * kPairH, "pair region");
+template <int kInstance, int H, bool kEarly, bool kPair = false>
 __device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1, int nb) {
   constexpr bool kW = H > kGsH;
+  static_assert(!kPair || (kEarly && kInstance == 0), "a pair covers one tile per workgroup");
   __shared__ GsX s;
   __shared__ double s_t0[kGsTY][kGsTX], s_t1[kGsTY][kGsTX];
   __shared__ double s_red[8 * kNW];
@@ -2470,7 +2498,27 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1
     gs_load<true>(F, F.r, q, gr);
 #pragma unroll
     for (int b = 0; b < 2; b++) x1[b] = gld2(F.x1, gs_row(F, q, b));
-    ec = gld((const double*)C.e, q.in ? mg_at(C, q.i >> 1, q.j >> 1) : 0);
+    if (!kPair) ec = gld((const double*)C.e, q.in ? mg_at(C, q.i >> 1, q.j >> 1) : 0);
+  };
+  // kPair: this thread's aggregate of the coarse level
+  __shared__ std::conditional_t<kPair, GsX, char> s_c[1];
+  GsPos qc{};
+  GsRaw gc;
+  d2 xc[2];
+  double ec2 = 0.0;
+  const int c0 = (tr.t0 % ntx) * (kGsTX / 2) - kPairH, r0 = (tr.t0 / ntx) * (kGsTY / 2) - kPairH;
+  if (kPair) {
+    qc = gs_pos_at(C, threadIdx.x % kPairX, threadIdx.x / kPairX, c0, r0,
+                   threadIdx.x < kPairX * kPairY);
+    gs_load<true>(C, C.r, qc, gc);
+#pragma unroll
+    for (int b = 0; b < 2; b++) xc[b] = gld2(C.x1, gs_row(C, qc, b));
+    ec2 = gld(A.e2, qc.in ? (size_t)((qc.j >> 1) + 1) * A.P2 + (qc.i >> 1) + 1 : 0);
+  }
+  // the coarse level's correction at its cell (i, j), in the tile's reach
+  auto coarse_e = [&](int i, int j) {
+    if constexpr (kPair) return s_c[0].v[(i - c0) & 1][j - r0 + 1][((i - c0) >> 1) + 1];
+    else return gld((const double*)C.e, mg_at(C, i, j));
   };
   if (kEarly) load();
   {
@@ -2480,6 +2528,35 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1
       hold(nb);
     }
     if (done) return;
+  }
+  if constexpr (kPair) {
+    GsAgg g;
+    gs_set(gc, qc.in, g);
+    gs_set_r(gc.r, qc.in, g);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      g.x[c] = qc.in & (1 << c) ? (c & 1 ? xc[c >> 1].y : xc[c >> 1].x) + A.oc * ec2 : 0.0;
+    // the ring around the region: no cell that is read depends on it
+    if (threadIdx.x < kGsR + 2) {
+      s_c[0].v[1][threadIdx.x][0] = 0.0;
+      s_c[0].v[0][threadIdx.x][kPairX + 1] = 0.0;
+    } else if (threadIdx.x >= 64 && threadIdx.x < 64 + kPairX + 2) {
+      const int p = threadIdx.x - 64;
+#pragma unroll
+      for (int a = 0; a < 2; a++) s_c[0].v[a][0][p] = s_c[0].v[a][2 * kPairY + 1][p] = 0.0;
+    }
+    gs_put<0>(g, s_c[0], qc);
+    gs_put<1>(g, s_c[0], qc);
+    __syncthreads();
+    if (qc.act) gs_half<1>(g, s_c[0], qc);
+    __syncthreads();
+    if (qc.act) gs_half<0>(g, s_c[0], qc);
+    __syncthreads();
+    if (qc.act) gs_half<1>(g, s_c[0], qc);
+    __syncthreads();
+    if (qc.act) gs_half<0>(g, s_c[0], qc);
+    __syncthreads();
+    ec = q.in ? coarse_e(q.i >> 1, q.j >> 1) : 0.0;
   }
   double acc[3] = {0.0, 0.0, 0.0};
   int band = band0, tend = kInstance == 1 ? band_range(ntiles, band, nb).t1 : 0;
@@ -2503,8 +2580,7 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1
       gs_ring(s, [&](int col, int row) {
         const int i = i0 - kGsH + col, j = j0 - kGsH + row;
         if (!kW || i < 0 || i >= F.nx || j < 0 || j >= F.ny) return 0.0;
-        return gld((const double*)F.x1, mg_at(F, i, j)) +
-               A.oc * gld((const double*)C.e, mg_at(C, i >> 1, j >> 1));
+        return gld((const double*)F.x1, mg_at(F, i, j)) + A.oc * coarse_e(i >> 1, j >> 1);
       });
     GsAgg g;
     gs_set(gr, q.in, g);
@@ -2559,10 +2635,10 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1
     while (band < band1) put_sums();  // trailing bands without tiles
 }
 
-template <int H, bool kEarly>
+template <int H, bool kEarly, bool kPair = false>
 __global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_up(MgArgs A) {
   const int band = xcd_tile(blockIdx.x, gridDim.x);
-  mg_up_body<0, H, kEarly>(A, band, band + 1, gridDim.x);
+  mg_up_body<0, H, kEarly, kPair>(A, band, band + 1, gridDim.x);
 }
 
 // Once per solve, for the one-workgroup levels f .. L-1 (1024 threads):
@@ -3732,6 +3808,12 @@ void launch_mg_up(const MgArgs& a, hipStream_t s) {
     if (a.cg.on) hipLaunchKernelGGL((k_mg_up<kGsH + 1, false>), g, b, 0, s, a);
     else hipLaunchKernelGGL((k_mg_up<kGsH, false>), g, b, 0, s, a);
   }
+}
+bool mg_up_pairs(const MgLevel& F) { return mg_tiles(F) <= kWideBlocks; }
+void launch_mg_up_pair(const MgArgs& a, hipStream_t s) {
+  const dim3 g(mg_grid(a.F)), b(kNT);
+  if (a.cg.on) hipLaunchKernelGGL((k_mg_up<kGsH + 1, true, true>), g, b, 0, s, a);
+  else hipLaunchKernelGGL((k_mg_up<kGsH, true, true>), g, b, 0, s, a);
 }
 void launch_mg_coarse_setup(const MgCycleArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_mg_coarse_setup, dim3(1), dim3(1024), 0, s, a);
