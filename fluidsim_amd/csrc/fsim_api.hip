@@ -740,13 +740,13 @@ size_t learned_level(const fs_handle* h) {
   return c;
 }
 
-// Whether the up step of level l makes that of level l + 1 too: the finest tile
-// level of few enough tiles whose coarse level is a tile level, then every
-// second one below.
-bool up_pair(const fs_handle* h, size_t l) {
+// How many levels below l the up launch of level l makes too: from the finest
+// level of few enough tiles on, two at most (the next launch then starts below).
+int up_depth(const fs_handle* h, size_t l) {
   size_t k = 0;
-  while (k + 1 < h->mg_first && !mg_up_pairs(h->mg[k])) k++;
-  return l >= k && l + 1 < h->mg_first && (l - k) % 2 == 0;
+  while (k + 1 < h->mg_first && !mg_up_deep(h->mg[k])) k++;
+  if (l < k || (l - k) % 3) return 0;
+  return (int)std::min<size_t>(2, h->mg_first - 1 - l);
 }
 
 // V-cycle `it` of the multigrid-PCG (-1: the initial cycle; it >= 0: one
@@ -766,14 +766,19 @@ int launch_vcycle(fs_handle* h, int it, fsl::Net* harvest = nullptr) {
   }
   launch_mg_coarse_cycle(cycle_args(h, it), h->st);
   for (size_t l = f; l-- > 0;) {
-    if (l > 0 && up_pair(h, l - 1)) continue;  // made by the next level's launch
-    MgArgs a = mg_up_args(h, l, it);
-    if (up_pair(h, l)) {
-      a.e2 = h->mg[l + 2].e;
-      a.P2 = h->mg[l + 2].P;
-      launch_mg_up_pair(a, h->st);
+    // (made by the launch of a level above)
+    if ((l > 0 && up_depth(h, l - 1) >= 1) || (l > 1 && up_depth(h, l - 2) >= 2)) continue;
+    const int d = up_depth(h, l);
+    if (d > 0) {
+      MgDeepArgs a;
+      memset(&a, 0, sizeof(a));
+      static_cast<MgArgs&>(a) = mg_up_args(h, l, it);
+      if (d == 2) a.T = h->mg[l + 2];
+      a.eb = h->mg[l + 1 + d].e;
+      a.Pb = h->mg[l + 1 + d].P;
+      launch_mg_up_deep(a, d, h->st);
     } else {
-      launch_mg_up(a, h->st);
+      launch_mg_up(mg_up_args(h, l, it), h->st);
     }
   }
   return 0;

@@ -204,8 +204,14 @@ struct MgArgs {
   double* xs2;           // correction x2, advanced here (warm_a, warm_b)
   double* xs3;           // correction x3, advanced here (warm_c)
   const double* rhs0;    // level-0 initial test: the right-hand side (zero start)
-  const double* e2;      // up with its coarse level (pair): the correction of the level below that
-  int32_t P2, pad_2;     // ... and its row pitch
+};
+// An up launch of several levels: F, C and (depth 2) T below it, started from
+// the correction eb (row pitch Pb) of the level below the last of them.  (Its
+// own type: 80 bytes more of arguments make the other launches 0.2 us longer.)
+struct MgDeepArgs : MgArgs {
+  MgLevel T;
+  const double* eb;
+  int32_t Pb, pad_b;
 };
 
 // Kernels whose per-block partial sums every block of the next kernel reads
@@ -354,9 +360,10 @@ void launch_mg_coarsen(const MgArgs& a, hipStream_t s);
 int mg_grid(const MgLevel& F);  // blocks (= partials) of a down/up launch
 void launch_mg_down(const MgArgs& a, hipStream_t s);
 void launch_mg_up(const MgArgs& a, hipStream_t s);
-// the up kernels of a.C and then a.F in one launch (mg_up_pairs(a.F))
-bool mg_up_pairs(const MgLevel& F);
-void launch_mg_up_pair(const MgArgs& a, hipStream_t s);
+// the up steps of the `depth` (1 or 2) levels below a.F and then a.F in one
+// launch (mg_up_deep(a.F))
+bool mg_up_deep(const MgLevel& F);
+void launch_mg_up_deep(const MgDeepArgs& a, int depth, hipStream_t s);
 void launch_mg_coarse_setup(const MgCycleArgs& a, hipStream_t s);
 void launch_mg_coarse_cycle(const MgCycleArgs& a, hipStream_t s);
 void launch_mgpcg_init(const MgPcgArgs& a, hipStream_t s);

@@ -1842,9 +1842,11 @@ struct GsAgg {
 // The iterates of the staged cells and one ring around them, by column parity
 // (even, odd), so that a wave's accesses have unit stride: cell (2I + a, y) of
 // the staged region is v[a][y + 1][I + 1].
-struct GsX {
-  double v[2][kGsR + 2][kAgX + 2];
+template <int AX, int AY>
+struct GsPlane {
+  double v[2][2 * AY + 2][AX + 2];
 };
+using GsX = GsPlane<kAgX, kAgY>;
 
 // Where this thread's aggregate lies: (i, j) its child 0 in the level, in bit
 // c: child c inside the level, own: inside the tile.
@@ -1955,8 +1957,8 @@ __device__ __forceinline__ void gs_set_r(const d2 (&r)[2], int in, GsAgg& s) {
 }
 
 // Writes one colour's children to LDS (red 0 and 3, black 1 and 2).
-template <int COL>
-__device__ __forceinline__ void gs_put(const GsAgg& g, GsX& s, const GsPos& q) {
+template <int COL, class S>
+__device__ __forceinline__ void gs_put(const GsAgg& g, S& s, const GsPos& q) {
   if (!q.act) return;
   const int y = 2 * q.J + 1, p = q.I + 1;
   if (COL == 0) {
@@ -1970,8 +1972,8 @@ __device__ __forceinline__ void gs_put(const GsAgg& g, GsX& s, const GsPos& q) {
 
 // One Gauss-Seidel half-sweep of colour COL (cells of one colour do not read
 // each other); the caller separates half-sweeps by barriers.
-template <int COL>
-__device__ __forceinline__ void gs_half(GsAgg& g, GsX& s, const GsPos& q) {
+template <int COL, class S>
+__device__ __forceinline__ void gs_half(GsAgg& g, S& s, const GsPos& q) {
   const int y = 2 * q.J + 1, p = q.I + 1;
   // (r + left + right + below + above) / d, fused as written: the smoother's
   // roundings are part of the results
@@ -2468,20 +2470,76 @@ __global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_down(MgArgs A) {
 // kEarly as in the down kernel: the first tile's loads before the test of
 // `done` (in bounds whatever the state).
 //
-// kPair: the coarse level's up step first, in the same launch: each tile makes
-// it on the coarse cells it reads and four rings around them (32 x 24 cells as
-// 16 x 12 aggregates), so that what a launch of its own would write is
-// recomputed in LDS, the same operations on the same values.  Where a tile has
-// a CU to itself the repeated work costs less than the launch: at
-// 256^2 over 128^2 cells 5.0 us instead of 4.7 and 4.6 us and a launch's gap, a
-// 512^2 solve 1010 instead of 1055 us.
-constexpr int kPairX = 16, kPairY = 12, kPairH = 8;  // aggregates, and cells before the tile's first
-static_assert(kPairX * kPairY <= kNT && 2 * kPairX >= kGsTX / 2 + 2 * kPairH &&
-                  2 * kPairY >= kGsTY / 2 + 2 * kPairH, "pair region");
-template <int kInstance, int H, bool kEarly, bool kPair = false>
-__device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1, int nb) {
+// kDeep: the up steps of the kDeep (1 or 2) levels below first, in the same
+// launch.  A tile makes the coarse level's on the coarse cells it reads and four
+// rings around them (32 x 24 cells, 16 x 12 aggregates), and before it the one
+// below on the cells that region reads and four rings (24 x 20 cells, 12 x 10
+// aggregates), in LDS, the same operations on the same values as launches of
+// their own.  Where a tile has a CU, or half of one, to itself the repeated work
+// costs less than a launch.
+// Measured at 512^2: one launch of 9.9 us in place of 6.6, 4.7 and 4.6 us and two
+// gaps of 1.7 us; an iteration takes 45.0 us (46.2 with the lower two in one
+// launch), at 350^2 38.6 (41.0).
+constexpr int kDeepX[2] = {16, 12}, kDeepY[2] = {12, 10};  // aggregates
+constexpr int kDeepH[2] = {8, 4};  // cells before the first one that the level above reads
+static_assert(2 * kDeepX[0] >= kGsTX / 2 + 2 * kDeepH[0] && 2 * kDeepY[0] >= kGsTY / 2 + 2 * kDeepH[0] &&
+                  2 * kDeepX[1] >= kDeepX[0] + 2 * kDeepH[1] &&
+                  2 * kDeepY[1] >= kDeepY[0] + 2 * kDeepH[1], "regions");
+// One of those levels: this thread's aggregate and its loads; the up step from
+// the correction e of its coarse cell; the result at a cell.
+template <int D>
+struct GsDeep {
+  GsPlane<kDeepX[D], kDeepY[D]>& s;
+  int c0, r0;  // the region's first cell
+  GsPos q;
+  GsRaw raw;
+  d2 x1[2];
+  __device__ __forceinline__ GsDeep(GsPlane<kDeepX[D], kDeepY[D]>& plane, int c, int r)
+      : s(plane), c0(c - kDeepH[D]), r0(r - kDeepH[D]) {}
+  __device__ __forceinline__ void load(const MgLevel& L) {
+    const int t = threadIdx.x;
+    q = gs_pos_at(L, t % kDeepX[D], t / kDeepX[D], c0, r0, t < kDeepX[D] * kDeepY[D]);
+    gs_load<true>(L, L.r, q, raw);
+#pragma unroll
+    for (int b = 0; b < 2; b++) x1[b] = gld2(L.x1, gs_row(L, q, b));
+  }
+  __device__ __forceinline__ double at(int i, int j) const {
+    return s.v[(i - c0) & 1][j - r0 + 1][((i - c0) >> 1) + 1];
+  }
+  __device__ __forceinline__ void up(double oc, double e) {
+    GsAgg g;
+    gs_set(raw, q.in, g);
+    gs_set_r(raw.r, q.in, g);
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      g.x[c] = q.in & (1 << c) ? (c & 1 ? x1[c >> 1].y : x1[c >> 1].x) + oc * e : 0.0;
+    // the ring around the region: no cell that is read depends on it
+    constexpr int X = kDeepX[D], Y = kDeepY[D];
+    const int t = threadIdx.x;
+    if (t < 2 * Y + 2) {
+      s.v[1][t][0] = 0.0;
+      s.v[0][t][X + 1] = 0.0;
+    } else if (t >= 64 && t < 64 + X + 2) {
+#pragma unroll
+      for (int a = 0; a < 2; a++) s.v[a][0][t - 64] = s.v[a][2 * Y + 1][t - 64] = 0.0;
+    }
+    gs_put<0>(g, s, q);
+    gs_put<1>(g, s, q);
+    __syncthreads();
+    if (q.act) gs_half<1>(g, s, q);
+    __syncthreads();
+    if (q.act) gs_half<0>(g, s, q);
+    __syncthreads();
+    if (q.act) gs_half<1>(g, s, q);
+    __syncthreads();
+    if (q.act) gs_half<0>(g, s, q);
+    __syncthreads();
+  }
+};
+template <int kInstance, int H, bool kEarly, int kDeep = 0, class Args = MgArgs>
+__device__ __forceinline__ void mg_up_body(const Args& A, int band0, int band1, int nb) {
   constexpr bool kW = H > kGsH;
-  static_assert(!kPair || (kEarly && kInstance == 0), "a pair covers one tile per workgroup");
+  static_assert(!kDeep || (kEarly && kInstance == 0), "one tile per workgroup");
   __shared__ GsX s;
   __shared__ double s_t0[kGsTY][kGsTX], s_t1[kGsTY][kGsTX];
   __shared__ double s_red[8 * kNW];
@@ -2498,65 +2556,55 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1
     gs_load<true>(F, F.r, q, gr);
 #pragma unroll
     for (int b = 0; b < 2; b++) x1[b] = gld2(F.x1, gs_row(F, q, b));
-    if (!kPair) ec = gld((const double*)C.e, q.in ? mg_at(C, q.i >> 1, q.j >> 1) : 0);
+    if (!kDeep) ec = gld((const double*)C.e, q.in ? mg_at(C, q.i >> 1, q.j >> 1) : 0);
   };
-  // kPair: this thread's aggregate of the coarse level
-  __shared__ std::conditional_t<kPair, GsX, char> s_c[1];
-  GsPos qc{};
-  GsRaw gc;
-  d2 xc[2];
-  double ec2 = 0.0;
-  const int c0 = (tr.t0 % ntx) * (kGsTX / 2) - kPairH, r0 = (tr.t0 / ntx) * (kGsTY / 2) - kPairH;
-  if (kPair) {
-    qc = gs_pos_at(C, threadIdx.x % kPairX, threadIdx.x / kPairX, c0, r0,
-                   threadIdx.x < kPairX * kPairY);
-    gs_load<true>(C, C.r, qc, gc);
-#pragma unroll
-    for (int b = 0; b < 2; b++) xc[b] = gld2(C.x1, gs_row(C, qc, b));
-    ec2 = gld(A.e2, qc.in ? (size_t)((qc.j >> 1) + 1) * A.P2 + (qc.i >> 1) + 1 : 0);
-  }
+  __shared__ std::conditional_t<(kDeep > 0), GsPlane<kDeepX[0], kDeepY[0]>, char> s_c[1];
+  __shared__ std::conditional_t<(kDeep > 1), GsPlane<kDeepX[1], kDeepY[1]>, char> s_t[1];
+  const int c0 = (tr.t0 % ntx) * (kGsTX / 2), r0 = (tr.t0 / ntx) * (kGsTY / 2);
   // the coarse level's correction at its cell (i, j), in the tile's reach
   auto coarse_e = [&](int i, int j) {
-    if constexpr (kPair) return s_c[0].v[(i - c0) & 1][j - r0 + 1][((i - c0) >> 1) + 1];
+    if constexpr (kDeep > 0) return GsDeep<0>(s_c[0], c0, r0).at(i, j);
     else return gld((const double*)C.e, mg_at(C, i, j));
   };
-  if (kEarly) load();
-  {
+  auto deep = [&](auto&& test) {  // loads of all levels, the test of `done`, the levels below
+    // the padded index of an aggregate's cell of the level below the launch's last
+    auto below = [&](const GsPos& p, int pitch) {
+      return p.in ? (size_t)((p.j >> 1) + 1) * pitch + (p.i >> 1) + 1 : 0;
+    };
+    if constexpr (kDeep == 1) {
+      GsDeep<0> c(s_c[0], c0, r0);
+      c.load(C);
+      const double e = gld(A.eb, below(c.q, A.Pb));
+      load();
+      if (test()) return true;
+      c.up(A.oc, e);
+    } else if constexpr (kDeep == 2) {
+      GsDeep<0> c(s_c[0], c0, r0);
+      c.load(C);
+      GsDeep<1> b(s_t[0], c.c0 / 2, c.r0 / 2);
+      b.load(A.T);
+      const double e = gld(A.eb, below(b.q, A.Pb));
+      load();
+      if (test()) return true;
+      b.up(A.oc, e);
+      c.up(A.oc, c.q.in ? b.at(c.q.i >> 1, c.q.j >> 1) : 0.0);
+    }
+    ec = q.in ? coarse_e(q.i >> 1, q.j >> 1) : 0.0;
+    return false;
+  };
+  auto stopped = [&]() {
     const int done = A.sc->done;
     if (kInstance == 0) {
       hold_mg_args(A, false);
       hold(nb);
     }
-    if (done) return;
-  }
-  if constexpr (kPair) {
-    GsAgg g;
-    gs_set(gc, qc.in, g);
-    gs_set_r(gc.r, qc.in, g);
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-      g.x[c] = qc.in & (1 << c) ? (c & 1 ? xc[c >> 1].y : xc[c >> 1].x) + A.oc * ec2 : 0.0;
-    // the ring around the region: no cell that is read depends on it
-    if (threadIdx.x < kGsR + 2) {
-      s_c[0].v[1][threadIdx.x][0] = 0.0;
-      s_c[0].v[0][threadIdx.x][kPairX + 1] = 0.0;
-    } else if (threadIdx.x >= 64 && threadIdx.x < 64 + kPairX + 2) {
-      const int p = threadIdx.x - 64;
-#pragma unroll
-      for (int a = 0; a < 2; a++) s_c[0].v[a][0][p] = s_c[0].v[a][2 * kPairY + 1][p] = 0.0;
-    }
-    gs_put<0>(g, s_c[0], qc);
-    gs_put<1>(g, s_c[0], qc);
-    __syncthreads();
-    if (qc.act) gs_half<1>(g, s_c[0], qc);
-    __syncthreads();
-    if (qc.act) gs_half<0>(g, s_c[0], qc);
-    __syncthreads();
-    if (qc.act) gs_half<1>(g, s_c[0], qc);
-    __syncthreads();
-    if (qc.act) gs_half<0>(g, s_c[0], qc);
-    __syncthreads();
-    ec = q.in ? coarse_e(q.i >> 1, q.j >> 1) : 0.0;
+    return done != 0;
+  };
+  if (kDeep) {
+    if (deep(stopped)) return;
+  } else {
+    if (kEarly) load();
+    if (stopped()) return;
   }
   double acc[3] = {0.0, 0.0, 0.0};
   int band = band0, tend = kInstance == 1 ? band_range(ntiles, band, nb).t1 : 0;
@@ -2635,10 +2683,15 @@ __device__ __forceinline__ void mg_up_body(const MgArgs& A, int band0, int band1
     while (band < band1) put_sums();  // trailing bands without tiles
 }
 
-template <int H, bool kEarly, bool kPair = false>
+template <int H, bool kEarly>
 __global__ void __launch_bounds__(kNT, kEarly ? 1 : 4) k_mg_up(MgArgs A) {
   const int band = xcd_tile(blockIdx.x, gridDim.x);
-  mg_up_body<0, H, kEarly, kPair>(A, band, band + 1, gridDim.x);
+  mg_up_body<0, H, kEarly>(A, band, band + 1, gridDim.x);
+}
+template <int H, int kDeep>
+__global__ void __launch_bounds__(kNT) k_mg_up_deep(MgDeepArgs A) {
+  const int band = xcd_tile(blockIdx.x, gridDim.x);
+  mg_up_body<0, H, true, kDeep>(A, band, band + 1, gridDim.x);
 }
 
 // Once per solve, for the one-workgroup levels f .. L-1 (1024 threads):
@@ -3809,11 +3862,17 @@ void launch_mg_up(const MgArgs& a, hipStream_t s) {
     else hipLaunchKernelGGL((k_mg_up<kGsH, false>), g, b, 0, s, a);
   }
 }
-bool mg_up_pairs(const MgLevel& F) { return mg_tiles(F) <= kWideBlocks; }
-void launch_mg_up_pair(const MgArgs& a, hipStream_t s) {
+// (a tile per workgroup, at most two workgroups per CU)
+bool mg_up_deep(const MgLevel& F) { return mg_tiles(F) <= 2 * kWideBlocks; }
+void launch_mg_up_deep(const MgDeepArgs& a, int depth, hipStream_t s) {
   const dim3 g(mg_grid(a.F)), b(kNT);
-  if (a.cg.on) hipLaunchKernelGGL((k_mg_up<kGsH + 1, true, true>), g, b, 0, s, a);
-  else hipLaunchKernelGGL((k_mg_up<kGsH, true, true>), g, b, 0, s, a);
+  if (a.cg.on) {
+    if (depth == 1) hipLaunchKernelGGL((k_mg_up_deep<kGsH + 1, 1>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((k_mg_up_deep<kGsH + 1, 2>), g, b, 0, s, a);
+  } else {
+    if (depth == 1) hipLaunchKernelGGL((k_mg_up_deep<kGsH, 1>), g, b, 0, s, a);
+    else hipLaunchKernelGGL((k_mg_up_deep<kGsH, 2>), g, b, 0, s, a);
+  }
 }
 void launch_mg_coarse_setup(const MgCycleArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_mg_coarse_setup, dim3(1), dim3(1024), 0, s, a);

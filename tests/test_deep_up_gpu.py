@@ -1,5 +1,6 @@
-"""GPU: a solo handle makes the up steps of two multigrid levels in one launch
-where the finer one has at most 256 tiles; an ensemble keeps a launch per level.
+"""GPU: a solo handle makes the up steps of two or three multigrid levels in one
+launch where the finest of them has at most 512 tiles; an ensemble keeps a launch
+per level.
 Members end bitwise where their solo runs do, on grids of two to four tile levels
 with odd sides, tile remainders and levels on both sides of the limit."""
 import numpy as np
