@@ -439,8 +439,18 @@ __global__ void k_weights_bf16(const float* w, uint16_t* wb, uint16_t* wt, WOff 
   wt[i] = f2bf(w[o.off[l] + ((8 - tp) * co + oo) * ci + ii]);
 }
 
+// A pixel's network input: the five values, the padding zero; two 16-byte
+// stores (pixels are 32 bytes, the activations aligned to 256).
+__device__ __forceinline__ void put_input(uint16_t* in, size_t p, const uint16_t (&v)[kInCh]) {
+  static_assert(kPadIn == 16 && kInCh == 5, "the packing below");
+  uint4* o = (uint4*)(in + p * kPadIn);
+  o[0] = make_uint4(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4], 0u);
+  o[1] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 // Training batch: sample scale s = sqrt(sum r^2/d / HW), inputs, r/s and the
-// loss operator.  One block per sample.
+// loss operator.  One block per sample: bound by the latency of its two passes
+// (15.4 -> 10.6 us with whole-pixel stores instead of sixteen 2-byte ones).
 __global__ void __launch_bounds__(1024) k_gather(const float* data, const int* idx, int H, int W,
                                                  uint16_t* in, float* rhat, float* op,
                                                  float* scale) {
@@ -449,6 +459,7 @@ __global__ void __launch_bounds__(1024) k_gather(const float* data, const int* i
   const float* r = data + (size_t)idx[b] * 4 * HW;
   const float *d = r + HW, *cx = r + 2 * HW, *cy = r + 3 * HW;
   float acc = 0.0f;
+#pragma unroll 4
   for (int p = threadIdx.x; p < HW; p += blockDim.x) acc += r[p] * r[p] / d[p];
   for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o);
   if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
@@ -465,13 +476,10 @@ __global__ void __launch_bounds__(1024) k_gather(const float* data, const int* i
   for (int p = threadIdx.x; p < HW; p += blockDim.x) {
     const int h = p / W, w = p % W;
     const float dd = d[p];
-    uint16_t* o = in + ((size_t)b * HW + p) * kPadIn;
-    o[0] = f2bf(r[p] / (s * dd));
-    o[1] = f2bf((w > 0 ? cx[p - 1] : 0.0f) / dd);
-    o[2] = f2bf(cx[p] / dd);
-    o[3] = f2bf((h > 0 ? cy[p - W] : 0.0f) / dd);
-    o[4] = f2bf(cy[p] / dd);
-    for (int c = kInCh; c < kPadIn; c++) o[c] = 0;
+    const float cl = cx[p > 0 ? p - 1 : 0], cb = cy[h > 0 ? p - W : p];
+    put_input(in, (size_t)b * HW + p,
+              {f2bf(r[p] / (s * dd)), f2bf((w > 0 ? cl : 0.0f) / dd), f2bf(cx[p] / dd),
+               f2bf((h > 0 ? cb : 0.0f) / dd), f2bf(cy[p] / dd)});
     rhat[(size_t)b * HW + p] = r[p] / s;
     float* ob = op + (size_t)b * 3 * HW;
     ob[p] = dd;
@@ -596,16 +604,16 @@ __global__ void k_nn_input(MgLevel L, const double* part, int nb, DevScalars* sc
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= H * W) return;
   const int h = p / W, w = p % W;
-  uint16_t* o = in + (size_t)p * kPadIn;
-  for (int c = 0; c < kPadIn; c++) o[c] = 0;
-  if (h >= L.ny || w >= L.nx) return;
+  if (h >= L.ny || w >= L.nx) {
+    put_input(in, p, {0, 0, 0, 0, 0});
+    return;
+  }
   const size_t m = (size_t)(h + 1) * L.P + (w + 1);
   const double d = L.d[m];
-  o[0] = f2bf((float)(L.r[m] / (s * d)));
-  o[1] = f2bf((float)(L.cx[m - 1] / d));
-  o[2] = f2bf((float)(L.cx[m] / d));
-  o[3] = f2bf((float)(L.cy[m - L.P] / d));
-  o[4] = f2bf((float)(L.cy[m] / d));
+  put_input(in, p,
+            {f2bf((float)(L.r[m] / (s * d))), f2bf((float)(L.cx[m - 1] / d)),
+             f2bf((float)(L.cx[m] / d)), f2bf((float)(L.cy[m - L.P] / d)),
+             f2bf((float)(L.cy[m] / d))});
 }
 
 __global__ void k_nn_output(const uint16_t* y, const float* wout, MgLevel L, DevScalars* sc,
