@@ -2244,7 +2244,7 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int band0, int ban
   double wa = 1.0, wb = 0.0, wc = 0.0;  // warm start x = wa x + wb x2 + wc x3 (initial test)
   int wn = 0;
   {
-    const int done = sc->done;
+    int done = sc->done;
     if (A.check) cs = check_state(sc, A.it);
     if (A.xs) {
       wa = sc->warm_a;
@@ -2261,6 +2261,17 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int band0, int ban
       hold(nb);
       hold(cs);
       asm volatile("" ::"s"(gam_old), "s"(alpha_old), "s"(wa), "s"(wb), "s"(wc), "s"(wn));
+    }
+    if (kInstance == 1 && red) {
+      // Band 0's workgroup may set `done` in this launch, while others start
+      // late: a workgroup that goes on to the next member takes one decision
+      // for all its waves, or their barriers would no longer pair.  (In a
+      // launch per band a wave that leaves alone ends, and what the others
+      // then write belongs to a solve that has stopped.)
+      __shared__ int s_done;
+      if (threadIdx.x == 0) s_done = done;
+      __syncthreads();
+      done = __builtin_amdgcn_readfirstlane(s_done);
     }
     if (done) return;
   }
