@@ -1366,6 +1366,7 @@ __global__ void __launch_bounds__(kPcgNT) k_pcg_it(PcgArgs A) {
   __shared__ double s_hi[3][kNT];
   __shared__ double s_red[3 * kPcgNW];
   __shared__ double s_tot[3];
+  __shared__ int s_done;
   const Geo& G = A.G;
   const int P = G.P, tid = threadIdx.x;
   const TileRange tr = tile_range(A.nbx * A.nby, blockIdx.x, gridDim.x);
@@ -1414,14 +1415,20 @@ __global__ void __launch_bounds__(kPcgNT) k_pcg_it(PcgArgs A) {
   const double bn = sc->bnorm2, tol = sc->tol;
   const double gam_old = sc->cg_gam[(it + 1) & 1], alpha_old = sc->cg_alpha[(it + 1) & 1];
   asm volatile("" ::"s"(done), "s"(maxit), "s"(bn), "s"(tol), "s"(gam_old), "s"(alpha_old));
-  if (done) return;
   double tot[3];
   part3_sum(pl, gridDim.x, tot);
   if (tid >= kNT) tot[0] = tot[1] = tot[2] = 0.0;
   block_sum<3, kPcgNW>(tot, s_red);
-  if (tid == 0)
+  if (tid == 0) {
     for (int k = 0; k < 3; k++) s_tot[k] = tot[k];
+    s_done = done;
+  }
   __syncthreads();
+  // One decision per workgroup: block 0 of this launch may have set `done`
+  // before a late workgroup started (three fit a CU, so a grid of 1024 is not
+  // resident at once), and waves that left one by one would be missing from
+  // the others' sums.
+  if (s_done) return;
   const double gam = s_tot[0], del = s_tot[1], rho = s_tot[2];
   const double bnorm2 = it == 0 ? rho : bn;
   const double res = bnorm2 > 0 ? sqrt(rho / bnorm2) : 0.0;
