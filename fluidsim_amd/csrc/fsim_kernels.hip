@@ -2280,7 +2280,10 @@ __device__ __forceinline__ void mg_down_body(const MgArgs& A, int band0, int ban
       __syncthreads();
       done = __builtin_amdgcn_readfirstlane(s_done);
     }
-    if (done) return;
+    // (the initial test: band 0 of this launch may already have stopped the
+    // solve, whose warm start the other bands still have to form; only the
+    // assembly's 3, no solve at all, ends it here)
+    if (A.xs ? done == 3 : done) return;
   }
   if (A.xs) {
     // the initial test of MG-PCG.  A warm start is wa x + wb x2 (the init
@@ -3729,9 +3732,7 @@ __global__ void __launch_bounds__(kNT, 3) kb_mg_down(const MgArgs* __restrict__ 
     mg_down_body<1, kCg, false>(ens_arg(t, s, i), b0, b1, nb);
   });
 }
-// The initial cycle's finest level keeps a workgroup per band: its blocks form
-// the warm starts before the convergence test, so none may come so late that
-// it finds the solve already stopped by that test.
+// The initial cycle's finest level, once per solve, keeps a workgroup per band.
 __global__ void __launch_bounds__(kNT, 4) kb_mg_down_init(const MgArgs* __restrict__ t, EnsMap m, EnsSel s) {
   int i, bid, nb;
   if (!ens_slot(m, i, bid, nb)) return;

@@ -47,3 +47,18 @@ def test_members_that_stop_at_different_iterations():
     logs = _compare(cfgs, 8)
     iters = [int(r[7]) for log in logs for r in log if r[6] >= 0]
     assert len(set(iters)) > 4, sorted(set(iters))
+
+
+def test_warm_starts_that_meet_the_tolerance():
+    """Solves that the initial test ends (0 iterations) still form their warm
+    start on every band, in launches of more bands than workgroups fit (1024)."""
+    from fluidsim_amd import configs
+
+    cfgs = configs.config3(24, base_seed=4, lo=150, hi=260, warm=2)
+    assert sum(map(_bands, cfgs)) > 1024
+    for c in cfgs:
+        c["lapl_rtol"] = 1e-2
+    logs = _compare(cfgs, 14)
+    zero = sum(int(r[7] == 0) for log in logs for r in log if r[6] >= 0)
+    print("solves ended by the initial test:", zero)
+    assert zero > 24
