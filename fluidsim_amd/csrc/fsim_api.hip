@@ -2571,6 +2571,7 @@ int eval_staged(double* d, int32_t n, int ni, int no, const double* a, double* o
 template <class L, class LV>
 int eval_any(int32_t n, int ni, int no, const double* a, double* out, L&& launch,
              LV&& launch_inline) {
+  if (!a || !out) return fail(FS_E_ARG, "null argument%s");
   const size_t len = (size_t)(ni + no) * n;
   int dev = -1;
   HIP_OK(hipGetDevice(&dev));
