@@ -2568,14 +2568,16 @@ int eval_staged(double* d, int32_t n, int ni, int no, const double* a, double* o
   HIP_OK(hipMemcpy(out, dO, (size_t)no * n * sizeof(double), hipMemcpyDeviceToHost));
   return 0;
 }
+// may_alloc: what the array does not hold, or a device without one, takes an
+// allocation instead of an error.
 template <class L, class LV>
-int eval_any(int32_t n, int ni, int no, const double* a, double* out, L&& launch,
+int eval_any(int32_t n, int ni, int no, const double* a, double* out, bool may_alloc, L&& launch,
              LV&& launch_inline) {
   if (!a || !out) return fail(FS_E_ARG, "null argument%s");
   const size_t len = (size_t)(ni + no) * n;
   int dev = -1;
   HIP_OK(hipGetDevice(&dev));
-  if (len <= kScratchDoubles && dev < kNoAllocMaxDevices) {
+  if (!may_alloc || (len <= kScratchDoubles && dev < kNoAllocMaxDevices)) {
     // calls in this process are serialised: they share the device's one array
     std::lock_guard<std::mutex> lock(g_noalloc_mu);
     double* d = nullptr;
@@ -2589,11 +2591,12 @@ int eval_any(int32_t n, int ni, int no, const double* a, double* out, L&& launch
   return e;
 }
 
-int eval_flux_common(int32_t n, const double* a, double* out, int dfdph) {
+int eval_flux_common(int32_t n, const double* a, double* out, int dfdph, bool may_alloc = true) {
   FsPhys K;
   fs_phys_init(&K, 10.0, 0.1);
   return eval_any(
-      n, 7, 1, a, out, [&](const double* i, double* o) { launch_eval_flux(K, i, o, n, dfdph, nullptr); },
+      n, 7, 1, a, out, may_alloc,
+      [&](const double* i, double* o) { launch_eval_flux(K, i, o, n, dfdph, nullptr); },
       [&](const EvalInline& v, double* o) { launch_eval_flux_inline(K, v, o, n, dfdph, nullptr); });
 }
 }  // namespace
@@ -2605,7 +2608,8 @@ int fs_eval_fits(double p, int32_t n, const double* T, double* out) {
   FsPhys K;
   fs_phys_init(&K, p, 0.1);
   return eval_any(
-      n, 1, 12, T, out, [&](const double* i, double* o) { launch_eval_fits(K, i, o, n, nullptr); },
+      n, 1, 12, T, out, true,
+      [&](const double* i, double* o) { launch_eval_fits(K, i, o, n, nullptr); },
       [&](const EvalInline& v, double* o) { launch_eval_fits_inline(K, v, o, n, nullptr); });
 }
 
@@ -2619,9 +2623,7 @@ int fs_eval_dfdph(int32_t n, const double* a, double* out) {
 int fs_eval_flux_noalloc(int32_t n, const double* a, double* out, int32_t dfdph) {
   if (n < 0 || n > kNoAllocMaxN)
     return fail(FS_E_ARG, "fs_eval_flux_noalloc: n must lie in 0..%s%d", "", kNoAllocMaxN);
-  if (n == 0) return 0;
-  if (!a || !out) return fail(FS_E_ARG, "null argument%s");
-  return eval_flux_common(n, a, out, dfdph ? 1 : 0);
+  return n == 0 ? 0 : eval_flux_common(n, a, out, dfdph ? 1 : 0, false);
 }
 
 int fs_time_kernel(fs_handle* h, int32_t which, int32_t n, double* avg_ms) {
