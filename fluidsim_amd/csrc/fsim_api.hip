@@ -2946,11 +2946,14 @@ int fs_learn_train(fs_learn* n, int32_t steps, int32_t batch, float lr, uint64_t
                    double* loss) {
   if (!n || steps < 0 || batch <= 0) return fail(FS_E_ARG, "bad argument%s");
   if (n->net.count == 0) return fail(FS_E_ARG, "empty training set%s");
+  const int round = fsl::train_round(&n->net, batch);
+  if (round == 0 && steps > 0)  // before the host holds indices for it
+    return fail(FS_E_HIP, "training step failed (batch too large?)%s");
   std::vector<int> idx;
   std::vector<double> l;
   uint64_t s = seed;
-  for (int k0 = 0; k0 < steps; k0 += fsl::kTrainRound) {
-    const int n_now = std::min(fsl::kTrainRound, steps - k0);
+  for (int k0 = 0; k0 < steps; k0 += round) {
+    const int n_now = std::min(round, steps - k0);
     idx.resize((size_t)n_now * batch);
     for (int& i : idx) {
       uint64_t z = (s += 0x9e3779b97f4a7c15ull);

@@ -24,7 +24,7 @@ constexpr int kPadIn = 16;       // input channels as stored
 constexpr int kOutCh = 16;       // channels feeding the 1x1 output convolution
 constexpr int kAlign = 8;        // network grid sides are multiples of 8 (three poolings)
 
-constexpr int kTrainRound = 64;  // training steps enqueued before the host waits
+constexpr int kTrainRound = 64;  // most training steps enqueued before the host waits
 
 enum InMode { kPlain = 0, kPool = 1, kUpCat = 2 };
 
@@ -92,6 +92,8 @@ int net_apply(Net* net, const MgLevel& L, const double* part, int nb, DevScalars
 int net_store_sample(Net* net, const MgLevel& L, hipStream_t st);
 // Regenerate the BF16 weight copies after the FP32 masters changed.
 void net_refresh(Net* net);
+// Training steps of B samples enqueued before the host waits; 0: B is too large.
+int train_round(const Net* net, int B);
 // Adam steps on the samples idx[step][0..B) of the training set; mean losses.
 int train_steps(Net* net, const int* idx, int steps, int B, float lr, double* loss);
 // Loss and gradient of a host batch (see fs_learn_loss_grad).

@@ -1020,21 +1020,27 @@ int net_store_sample(Net* net, const MgLevel& L, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// As many steps as the loss partials and the indices have room for.
+int train_round(const Net* net, int B) {
+  const int64_t nbl = ((int64_t)B * net->H * net->W + 255) / 256;
+  if (nbl > kLossSlots / 2 || B > kLossSlots) return 0;
+  return std::max(1, std::min(kTrainRound, std::min(kLossSlots / 2 / (int)nbl, kLossSlots / B)));
+}
+
 // Training steps on the batches idx[step][B]; mean losses.  The steps of a round
-// (as many as the loss partials have room for) are enqueued together: their
-// indices go up once and their losses come back once, so that the host waits
-// once per round and not in every step.
+// (train_round) are enqueued together: their indices go up once and their losses
+// come back once, so that the host waits once per round and not in every step.
 int train_steps(Net* net, const int* idx, int steps, int B, float lr, double* loss) {
   Acts& a = net->train;
   hipStream_t st = net->st;
+  const int most = train_round(net, B);
+  if (most == 0) return -1;
   if (a.N != B || a.H != net->H || a.W != net->W) {
     if (acts_alloc(a, B, net->H, net->W)) return -1;
   }
   const int n0 = B * net->H * net->W;
   const int nbl = ceil_div(n0, 256);
-  if (nbl > kLossSlots / 2 || B > kLossSlots) return -1;
   int* d_idx = (int*)(net->lpart + kLossSlots / 2);
-  const int most = std::max(1, std::min(kTrainRound, std::min(kLossSlots / 2 / nbl, kLossSlots / B)));
   std::vector<float> lp;
   for (int k0 = 0; k0 < steps; k0 += most) {
     const int n = std::min(most, steps - k0);
