@@ -2628,6 +2628,14 @@ int fs_eval_flux_noalloc(int32_t n, const double* a, double* out, int32_t dfdph)
 
 int fs_time_kernel(fs_handle* h, int32_t which, int32_t n, double* avg_ms) {
   if (!h || !avg_ms || n <= 0) return fail(FS_E_ARG, "bad argument%s");
+  const bool level_id = (which >= 20 && which < 60);
+  if (!(which >= 1 && which <= 5) && !(which >= 10 && which <= 18) && !level_id)
+    return fail(FS_E_ARG, "unknown kernel id%s");
+  if (level_id && h->mg.size() > 1 && (size_t)(which % 20) >= h->mg_first)
+    return fail(FS_E_ARG, "no tile kernel on that multigrid level%s");
+  if (which >= 13 && h->mg.size() < 2)
+    return fail(FS_E_ARG, "grid too small for a multigrid hierarchy%s");
+  if (which == 15 && !h->net) return fail(FS_E_ARG, "no network attached%s");
   h->warm_ok = false;  // the timed launches overwrite the solver's vectors
   if (sync_scalars(h)) return FS_E_HIP;
   const double tol0 = h->h_sc->tol;
@@ -2670,14 +2678,6 @@ int fs_time_kernel(fs_handle* h, int32_t which, int32_t n, double* avg_ms) {
       launch_pcg_init(ia, h->st);
     }
   };
-  const bool level_id = (which >= 20 && which < 60);
-  if (!(which >= 1 && which <= 5) && !(which >= 10 && which <= 18) && !level_id)
-    return fail(FS_E_ARG, "unknown kernel id%s");
-  if (level_id && h->mg.size() > 1 && (size_t)(which % 20) >= h->mg_first)
-    return fail(FS_E_ARG, "no tile kernel on that multigrid level%s");
-  if (which >= 13 && h->mg.size() < 2)
-    return fail(FS_E_ARG, "grid too small for a multigrid hierarchy%s");
-  if (which == 15 && !h->net) return fail(FS_E_ARG, "no network attached%s");
   if (which == 11) {  // consistent partials for the Jacobi-PCG iterations
     PcgArgs ia = pcg_args(h, 0);
     ia.part_out = h->part(0);
