@@ -93,14 +93,21 @@ def gpu_run(args):
     # per-launch kernel durations on the live state (HIP events on the stream)
     k = {f"stage{s}": d.time_kernel(s, 50) for s in (1, 2, 3, 4, 5)}
     k["assembly"] = d.time_kernel(10, 50)
-    # multigrid-PCG: the down / up kernel of each tile level, the one-workgroup
-    # coarse kernel and one whole iteration
+    # multigrid-PCG: the down and up launches of the tile levels (an up launch
+    # may make the steps of several levels: mg_up0_2 makes those of levels 0 to
+    # 2), the one-workgroup coarse kernel and one whole iteration
+    ups = []  # [first level, last level, ms]
     for lvl in range(16):
         try:
             k[f"mg_down{lvl}"] = d.time_kernel(20 + lvl, 200)
-            k[f"mg_up{lvl}"] = d.time_kernel(40 + lvl, 200)
         except FsError:
             break
+        try:
+            ups.append([lvl, lvl, d.time_kernel(40 + lvl, 200)])
+        except FsError:  # part of the launch of a level above
+            ups[-1][1] = lvl
+    for a, b, ms in ups:
+        k[f"mg_up{a}" if a == b else f"mg_up{a}_{b}"] = ms
     k["mg_coarse"] = d.time_kernel(18, 200)
     k["mg_iteration"] = d.time_kernel(17, 100)
     k["jacobi_pcg_it"] = d.time_kernel(11, 400)
@@ -108,7 +115,7 @@ def gpu_run(args):
 
     copy_gbs = copy_bandwidth(1 << 30, 20)
     return dict(cfg=cfg, elapsed=elapsed, accepted=accepted, attempts=attempts,
-                iters=iters, timers=timers, kernels=k, N=N, s1=s1, copy_gbs=copy_gbs,
+                iters=iters, timers=timers, kernels=k, up_finest=ups[0], N=N, s1=s1, copy_gbs=copy_gbs,
                 poisson=poisson, snap=snap, same=same, stage_tile=d.stage_tile())
 
 
@@ -436,9 +443,13 @@ def main():
     # first-iteration form: down reads r, w, d, cx, cy, u, x, writes p, s, x, r,
     # x1 and the quarter-size coarse residual (12.25 planes; later iterations
     # also read s and p: 14.25); up reads x1, r, d, cx, cy and the coarse
-    # correction, writes u and w = M u (7.25 planes)
+    # correction, writes u and w = M u (7.25 planes; where it also makes the
+    # steps of the levels below, x1, r, d, cx, cy of each in the correction's
+    # place, and the correction of the level below the last)
     ach_d = 12.25 * plane / (kern["mg_down0"] * 1e-3) / 1e9
-    ach_u = 7.25 * plane / (kern["mg_up0"] * 1e-3) / 1e9
+    up_last, up_ms = r["up_finest"][1:]
+    up_planes = 7 + 5 * sum(0.25 ** q for q in range(1, up_last + 1)) + 0.25 ** (up_last + 1)
+    ach_u = up_planes * plane / (up_ms * 1e-3) / 1e9
     timers = r["timers"]
     tot_ms = r["elapsed"] * 1e3
     iters = r["iters"]
@@ -477,7 +488,9 @@ def main():
                      "frac": ach_s / PEAK_HBM_GBS,
                      "traffic": None if stage_traffic is None else stage_traffic,
                      "algorithmic_bytes_per_step": bytes_step},
-        "roofline_poisson": {"kernels": "k_mg_down / k_mg_up, finest level", "bound": "hbm",
+        "roofline_poisson": {"kernels": "down / up launch of the finest level" +
+                                        (f" (up: with the levels down to {up_last})"
+                                         if up_last else ""), "bound": "hbm",
                              "achieved_down": ach_d, "achieved_up": ach_u,
                              "peak": PEAK_HBM_GBS, "unit": "GB/s",
                              "frac_down": ach_d / PEAK_HBM_GBS, "frac_up": ach_u / PEAK_HBM_GBS},

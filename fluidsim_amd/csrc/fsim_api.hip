@@ -749,6 +749,27 @@ int up_depth(const fs_handle* h, size_t l) {
   return (int)std::min<size_t>(2, h->mg_first - 1 - l);
 }
 
+// Whether the launch of a level above makes level l's up step.
+bool up_covered(const fs_handle* h, size_t l) {
+  return (l > 0 && up_depth(h, l - 1) >= 1) || (l > 1 && up_depth(h, l - 2) >= 2);
+}
+
+// The up launch of V-cycle `it` that starts at level l (not a covered one).
+void launch_up(fs_handle* h, size_t l, int it) {
+  const int d = up_depth(h, l);
+  if (d == 0) {
+    launch_mg_up(mg_up_args(h, l, it), h->st);
+    return;
+  }
+  MgDeepArgs a;
+  memset(&a, 0, sizeof(a));
+  static_cast<MgArgs&>(a) = mg_up_args(h, l, it);
+  if (d == 2) a.T = h->mg[l + 2];
+  a.eb = h->mg[l + 1 + d].e;
+  a.Pb = h->mg[l + 1 + d].P;
+  launch_mg_up_deep(a, d, h->st);
+}
+
 // V-cycle `it` of the multigrid-PCG (-1: the initial cycle; it >= 0: one
 // whole CG iteration, its update fused into the finest down kernel).  Only
 // the parity of `it` matters after it = 0.  With `harvest`, the residual
@@ -765,22 +786,8 @@ int launch_vcycle(fs_handle* h, int it, fsl::Net* harvest = nullptr) {
     }
   }
   launch_mg_coarse_cycle(cycle_args(h, it), h->st);
-  for (size_t l = f; l-- > 0;) {
-    // (made by the launch of a level above)
-    if ((l > 0 && up_depth(h, l - 1) >= 1) || (l > 1 && up_depth(h, l - 2) >= 2)) continue;
-    const int d = up_depth(h, l);
-    if (d > 0) {
-      MgDeepArgs a;
-      memset(&a, 0, sizeof(a));
-      static_cast<MgArgs&>(a) = mg_up_args(h, l, it);
-      if (d == 2) a.T = h->mg[l + 2];
-      a.eb = h->mg[l + 1 + d].e;
-      a.Pb = h->mg[l + 1 + d].P;
-      launch_mg_up_deep(a, d, h->st);
-    } else {
-      launch_mg_up(mg_up_args(h, l, it), h->st);
-    }
-  }
+  for (size_t l = f; l-- > 0;)
+    if (!up_covered(h, l)) launch_up(h, l, it);
   return 0;
 }
 
@@ -2633,6 +2640,8 @@ int fs_time_kernel(fs_handle* h, int32_t which, int32_t n, double* avg_ms) {
     return fail(FS_E_ARG, "unknown kernel id%s");
   if (level_id && h->mg.size() > 1 && (size_t)(which % 20) >= h->mg_first)
     return fail(FS_E_ARG, "no tile kernel on that multigrid level%s");
+  if (which >= 40 && level_id && h->mg.size() > 1 && up_covered(h, which - 40))
+    return fail(FS_E_ARG, "that level's up step is part of the launch of a level above%s");
   if (which >= 13 && h->mg.size() < 2)
     return fail(FS_E_ARG, "grid too small for a multigrid hierarchy%s");
   if (which == 15 && !h->net) return fail(FS_E_ARG, "no network attached%s");
@@ -2664,13 +2673,13 @@ int fs_time_kernel(fs_handle* h, int32_t which, int32_t n, double* avg_ms) {
       // same partials it stays a valid update, unlike the recurrence form
       launch_mg_down(mg_down_args(h, 0, 0), h->st);
     } else if (which == 14) {
-      launch_mg_up(mg_up_args(h, 0, 2 + (k & 1)), h->st);
+      launch_up(h, 0, 2 + (k & 1));
     } else if (which == 18) {
       launch_mg_coarse_cycle(cycle_args(h, 2 + (k & 1)), h->st);
     } else if (which >= 20 && which < 40) {
       launch_mg_down(mg_down_args(h, which - 20, 2 + (k & 1)), h->st);
     } else if (which >= 40 && which < 60) {
-      launch_mg_up(mg_up_args(h, which - 40, 2 + (k & 1)), h->st);
+      launch_up(h, which - 40, 2 + (k & 1));
     } else {
       PcgArgs ia = pcg_args(h, 0);
       ia.part_out = h->part(0);

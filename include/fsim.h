@@ -234,7 +234,9 @@ int fs_set_timing(fs_handle* h, int32_t on);
  * level, 16 = one learned flexible-CG iteration, 17 = one multigrid-PCG
  * iteration (sequences of kernels, timed as a whole), 18 = the one-workgroup
  * coarse multigrid kernel, 20 + l / 40 + l = the down / up kernel of tile
- * level l of the multigrid-PCG iteration. */
+ * level l of the multigrid-PCG iteration.  An up launch (14, 40 + l) is the
+ * one that the iteration makes: where it also makes the steps of levels below,
+ * those levels' own ids are refused (FS_E_ARG). */
 int fs_time_kernel(fs_handle* h, int32_t which, int32_t n, double* avg_ms);
 
 /* Device copy bandwidth: `reps` launches of a plain copy kernel moving
