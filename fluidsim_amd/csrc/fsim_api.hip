@@ -354,10 +354,11 @@ hipError_t alloc_pinned(fs_handle* h) {
 
 // One plane between the device and the caller's array (leading dimension ld),
 // piece by piece: the copy of a piece between the pinned memory and the array
-// overlaps the transfer of the next.  A read into a fresh array: 64^2 26 us, 512^2
-// 135 us, 2048^2 2.4 ms, which is the array's page faults; through the
-// runtime's pageable copy and a second host copy 26 us, 209 us, 4.2 ms.  Pieces
-// a quarter the size take 512^2 to 165 us, twice the size 130 us.
+// overlaps the transfer of the next.  A read into a fresh array: 64^2 12 us, 512^2
+// 87 us, 2048^2 2.1 ms, half of it the array's page faults; through the runtime's
+// pageable copy and a second host copy 12 us, 210 us, 4.3 ms (writes 10, 71 and
+// 850 us; 10, 117 and 1800 us).  Pieces half the size take a 2048^2 write to 1010
+// us and a 256^2 one from 24 to 29, twice the size a 512^2 read to 120 us.
 int field_io(fs_handle* h, double* dev, double* host, int32_t ld, bool out) {
   const size_t P = h->P, rows = h->io_cap / P, ny = (size_t)h->by + 2;
   const size_t n = (ny + rows - 1) / rows;

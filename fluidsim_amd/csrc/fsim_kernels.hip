@@ -3567,22 +3567,38 @@ __global__ void k_fill(double* p, double v, size_t n) {
 // pair.  The last workgroup to finish (*done counts them and ends at zero)
 // writes the piece's number to *flag, which the host polls: a second kernel
 // for that took another 5 us a piece.
+// kIoBlocks workgroups with kIoAhead pairs of every thread in flight cover the
+// link's latency; more only crowd it.  Writes of a 512^2 field take 71 us so, 75
+// with 24 workgroups of one pair, 128 with 256 of them, and in four threads at
+// once 49, 55 and 112 us (reads 83, 83, 113 and 46, 45, 76).
+constexpr int kIoBlocks = 16, kIoAhead = 4;
 template <bool kOut>
 __global__ void __launch_bounds__(256) k_io(const double* __restrict__ src,
                                             double* __restrict__ dst, int n, unsigned* done,
                                             uint32_t* flag, uint32_t seq) {
   const int step = (int)gridDim.x * 512;
-  for (int k = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 2; k < n; k += step) {
-    if (k + 1 < n) {
-      if (kOut) {
-        *reinterpret_cast<double2*>(dst + k) = make_double2(src[k], src[k + 1]);
-      } else {
-        const double2 v = *reinterpret_cast<const double2*>(src + k);
-        dst[k] = v.x;
-        dst[k + 1] = v.y;
+  for (int k0 = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 2; k0 < n; k0 += kIoAhead * step) {
+    double2 v[kIoAhead];
+#pragma unroll
+    for (int u = 0; u < kIoAhead; u++) {
+      const int k = k0 + u * step;
+      if (k + 1 < n)
+        v[u] = kOut ? make_double2(src[k], src[k + 1]) : *reinterpret_cast<const double2*>(src + k);
+      else if (k < n) v[u].x = src[k];
+    }
+#pragma unroll
+    for (int u = 0; u < kIoAhead; u++) {
+      const int k = k0 + u * step;
+      if (k + 1 < n) {
+        if (kOut) {
+          *reinterpret_cast<double2*>(dst + k) = v[u];
+        } else {
+          dst[k] = v[u].x;
+          dst[k + 1] = v[u].y;
+        }
+      } else if (k < n) {
+        dst[k] = v[u].x;
       }
-    } else {
-      dst[k] = src[k];
     }
   }
   __threadfence_system();
@@ -3924,7 +3940,8 @@ void launch_io(const double* src, double* dst, int n, bool out, unsigned* done, 
                uint32_t seq, hipStream_t s) {
   const int nb = (n + 511) / 512;
   auto k = out ? k_io<true> : k_io<false>;
-  hipLaunchKernelGGL(k, dim3(nb < 256 ? nb : 256), dim3(256), 0, s, src, dst, n, done, flag, seq);
+  hipLaunchKernelGGL(k, dim3(nb < kIoBlocks ? nb : kIoBlocks), dim3(256), 0, s, src, dst, n, done,
+                     flag, seq);
 }
 void launch_eval_fits_inline(const FsPhys& K, const EvalInline& T, double* out, int n,
                              hipStream_t s) {
