@@ -2542,6 +2542,7 @@ constexpr size_t kNoAllocScratchBytes = (size_t)2 << 20;  // 2 MiB per device
 constexpr size_t kScratchDoubles = kNoAllocScratchBytes / sizeof(double);
 constexpr int32_t kNoAllocMaxN = (int32_t)(kScratchDoubles / 8);
 constexpr int kNoAllocMaxDevices = 64;
+constexpr size_t kWaitDoubles = 1 << 16;  // calls below it wait for the array
 std::mutex g_noalloc_mu;
 double* g_noalloc_ptr[kNoAllocMaxDevices];  // device address of `scratch`, per device
 }  // namespace
@@ -2591,11 +2592,18 @@ int eval_any(int32_t n, int ni, int no, const double* a, double* out, bool may_a
   int dev = -1;
   HIP_OK(hipGetDevice(&dev));
   if (!may_alloc || (len <= kScratchDoubles && dev < kNoAllocMaxDevices)) {
-    // calls in this process are serialised: they share the device's one array
-    std::lock_guard<std::mutex> lock(g_noalloc_mu);
-    double* d = nullptr;
-    if (int e = scratch_ptr(&d)) return e;
-    return eval_staged(d, n, ni, no, a, out, launch, launch_inline);
+    // calls in this process share the device's one array and wait for it; a
+    // large one that may allocate does so if another thread has it (four
+    // threads, per call: 32 000 fluxes 103 us instead of 112, 8000 51 instead of
+    // 54; one flux 27 instead of 17)
+    std::unique_lock<std::mutex> lock(g_noalloc_mu, std::defer_lock);
+    if (!may_alloc || len < kWaitDoubles) lock.lock();
+    else (void)lock.try_lock();
+    if (lock.owns_lock()) {
+      double* d = nullptr;
+      if (int e = scratch_ptr(&d)) return e;
+      return eval_staged(d, n, ni, no, a, out, launch, launch_inline);
+    }
   }
   double* d = nullptr;
   HIP_OK(hipMalloc(&d, len * sizeof(double)));

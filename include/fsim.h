@@ -208,8 +208,9 @@ int fs_eval_dfdph(int32_t n, const double* args7, double* out);
  * loops, harnesses that forbid hipMalloc).  The device staging lives in a
  * fixed 2 MiB array per GPU, held until the process ends, so n is at most
  * 32768 (larger n: FS_E_ARG, nothing launched).  Every call on one GPU
- * shares that array: calls from threads of one process are serialised, and
- * results equal fs_eval_flux / fs_eval_dfdph bitwise. */
+ * shares that array (as do fs_eval_flux, fs_eval_dfdph and fs_eval_fits up to
+ * 2 MiB): calls from threads of one process are serialised, and results equal
+ * fs_eval_flux / fs_eval_dfdph bitwise. */
 int fs_eval_flux_noalloc(int32_t n, const double* args7, double* out, int32_t dfdph);
 
 /* Select the Poisson preconditioner of later fs_lapl_solve calls (0 Jacobi,
