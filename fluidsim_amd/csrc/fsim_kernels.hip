@@ -1537,18 +1537,17 @@ __global__ void __launch_bounds__(kNT) k_pcg_tres(PcgArgs A, int nb) { pcg_tres_
 // A whole Jacobi-PCG solve in one workgroup, for systems whose cells fit its
 // registers: k_pcg_init, the iterations of k_pcg_it, k_pcg_finish and
 // k_pcg_tres in one launch.  Such a system is bound by latency: as a launch per
-// iteration it costs 6-8 us each (3.4 us of kernel, the rest launch and host),
+// iteration it costs 6-9 us each (3.4 us of kernel, the rest launch and host),
 // here an iteration is two barriers, an LDS exchange of u = r / d and three
-// wave reductions, about 1 us.  Measured: a pass of the 40-cell default
-// discharge (40 iterations) 430 -> 117 us.
+// wave reductions, about 1 us in one wave (pcg_small_fits has the others).
+// Measured: a pass of the 40-cell default discharge (40 iterations) 430 -> 117 us.
 //
-// Every value is the one the launches compute, bit for bit: the same
-// expressions, and sums over the same tiles in the same order (a tile's
-// threads by wave trees and then its waves in order, the tiles by one wave's
-// tree).  The tiles are those of the launches, 64 x 8 cells with two cells per
-// thread of 256; in one dimension (kOneD) a tile has one row, so a wave takes
-// a tile of its own.  Thread t holds the cells of tiles (t / 256) + NTH / 256 q
-// (one dimension: t / 64 + NTH / 64 q), q < S.
+// The expressions are those of the launches, and the sums go over the same
+// tiles in the same order (a tile's threads by wave trees and then its waves in
+// order, the tiles by one wave's tree).  The tiles are those of the launches, 64
+// x 8 cells with two cells per thread of 256; in one dimension (kOneD) a tile has
+// one row, so a wave takes a tile of its own.  Thread t holds the cells of tiles
+// (t / 256) + NTH / 256 q (one dimension: t / 64 + NTH / 64 q), q < S.
 template <bool kOneD, int NTH, int S>
 __global__ void __launch_bounds__(NTH) k_pcg_small(PcgArgs A) {
   constexpr int C = kOneD ? S : S * kPcgRows;  // cells per thread
@@ -3851,9 +3850,13 @@ void launch_pcg_finish(const PcgArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_pcg_tres, dim3(1), dim3(kNT), 0, s, a, capped_grid(a.nbx * a.nby));
 }
 // The workgroup shapes of k_pcg_small: the smallest that holds the system's
-// tiles (one dimension: a wave per 64 cells; two: 256 threads per 64 x 8).
+// tiles (one dimension: a wave per 64 cells; two: 256 threads per 64 x 8), while
+// an iteration takes less than as a launch.  One dimension: 1.2 us up to 64
+// cells, 1.4-1.6 to 256, 3.7 to 1024, against 6-9 (four cells per thread, to 4096:
+// 9.1-9.6 against 5.8-6.2); two: 1.5 us for one tile, 4.0 up to four, 5.9-7.2 up to
+// eight, against 6.1-9.
 bool pcg_small_fits(const Geo& G) {
-  if (G.by == 1) return G.bx <= 64 * 64;
+  if (G.by == 1) return G.bx <= 16 * kTX;
   const int nt = ((G.bx + kTX - 1) / kTX) * ((G.by + kPcgTY - 1) / kPcgTY);
   return nt <= 8 && (G.bx + 2) * (G.by + 2) <= kPcgSmallPlane;
 }
@@ -3864,8 +3867,7 @@ void launch_pcg_small(const PcgArgs& a, hipStream_t s) {
   if (a.G.by == 1) {
     if (nt <= 1) PCG_SMALL(true, 64, 1);
     else if (nt <= 4) PCG_SMALL(true, 256, 1);
-    else if (nt <= 16) PCG_SMALL(true, 1024, 1);
-    else PCG_SMALL(true, 1024, 4);
+    else PCG_SMALL(true, 1024, 1);
   } else {
     if (nt <= 1) PCG_SMALL(false, 256, 1);
     else if (nt <= 4) PCG_SMALL(false, 1024, 1);
