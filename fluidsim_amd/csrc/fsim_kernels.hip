@@ -1358,13 +1358,19 @@ __global__ void __launch_bounds__(kNT) k_pcg_init(PcgArgs A) {
 // 65 x 64 to 256^2 cells, 9.85 -> 9.7 at 512^2, 24.5 -> 23.2 at 1024^2.
 // Sums: a thread of the lower four waves adds its cell's terms and those of the
 // cell four rows up, tile by tile, then the waves' trees in order.
-constexpr int kPcgNT = kTX * kPcgTY, kPcgNW = kPcgNT / 64;
-static_assert(kPcgRows == 2 && kPcgNT == 2 * kNT, "two cells per thread of the lower half");
-constexpr int kPcgRing = 2 * kTX + 2 * kPcgTY;  // cells around a tile (no corners)
-__global__ void __launch_bounds__(kPcgNT) k_pcg_it(PcgArgs A) {
-  __shared__ double s_u[kPcgTY + 2][kTX + 2];
-  __shared__ double s_hi[3][kNT];
-  __shared__ double s_red[3 * kPcgNW];
+// TY: the tile's rows, four where the grid has no more: with the upper four waves
+// idle an iteration of 1025 to 8000 cells in one dimension takes 6.0 us instead of
+// 4.7 (a thread per two cells of 256: 5.9), of 2000 x 2 cells 6.0 instead of 4.8.
+static_assert(kPcgRows == 2 && kTX * kPcgTY == 2 * kNT, "two cells per thread of the lower half");
+template <int TY>
+__global__ void __launch_bounds__(kTX * TY) k_pcg_it(PcgArgs A) {
+  constexpr int kThreads = kTX * TY, kWaves = kThreads / 64;
+  constexpr bool kUpper = TY == kPcgTY;    // there are upper four waves
+  constexpr int kRing = 2 * kTX + 2 * TY;  // cells around a tile (no corners)
+  static_assert(TY == kPcgTY || 2 * TY == kPcgTY, "a tile or its lower half");
+  __shared__ double s_u[TY + 2][kTX + 2];
+  __shared__ double s_hi[kUpper ? 3 : 1][kUpper ? kNT : 1];
+  __shared__ double s_red[3 * kWaves];
   __shared__ double s_tot[3];
   __shared__ int s_done;
   const Geo& G = A.G;
@@ -1372,9 +1378,9 @@ __global__ void __launch_bounds__(kPcgNT) k_pcg_it(PcgArgs A) {
   const TileRange tr = tile_range(A.nbx * A.nby, blockIdx.x, gridDim.x);
   const int tx = tid % kTX, ty = tid / kTX;
   // this thread's cell of the ring: below, above, left, right
-  const int q = tid < kPcgRing ? tid : 0;
-  const int rx = q < 2 * kTX ? q % kTX : (q - 2 * kTX) / kPcgTY ? kTX : -1;
-  const int ry = q < 2 * kTX ? (q / kTX ? kPcgTY : -1) : (q - 2 * kTX) % kPcgTY;
+  const int q = tid < kRing ? tid : 0;
+  const int rx = q < 2 * kTX ? q % kTX : (q - 2 * kTX) / TY ? kTX : -1;
+  const int ry = q < 2 * kTX ? (q / kTX ? TY : -1) : (q - 2 * kTX) % TY;
   struct Cell {
     double r, w, s, d;
   };
@@ -1417,8 +1423,8 @@ __global__ void __launch_bounds__(kPcgNT) k_pcg_it(PcgArgs A) {
   asm volatile("" ::"s"(done), "s"(maxit), "s"(bn), "s"(tol), "s"(gam_old), "s"(alpha_old));
   double tot[3];
   part3_sum(pl, gridDim.x, tot);
-  if (tid >= kNT) tot[0] = tot[1] = tot[2] = 0.0;
-  block_sum<3, kPcgNW>(tot, s_red);
+  if (kUpper && tid >= kNT) tot[0] = tot[1] = tot[2] = 0.0;
+  block_sum<3, kWaves>(tot, s_red);
   if (tid == 0) {
     for (int k = 0; k < 3; k++) s_tot[k] = tot[k];
     s_done = done;
@@ -1458,7 +1464,7 @@ __global__ void __launch_bounds__(kPcgNT) k_pcg_it(PcgArgs A) {
     // u_{i+1} (zero outside: r = s = w = 0, d = 1)
     const double sn = c.w + beta * c.s, rn = c.r - alpha * sn, un = rn / c.d;
     s_u[ty + 1][tx + 1] = un;
-    if (tid < kPcgRing) s_u[ry + 1][rx + 1] = (g.r - alpha * (g.w + beta * g.s)) / g.d;
+    if (tid < kRing) s_u[ry + 1][rx + 1] = (g.r - alpha * (g.w + beta * g.s)) / g.d;
     const double pc = c.r / c.d + beta * p;
     __syncthreads();
     double a[3] = {0.0, 0.0, 0.0};
@@ -1475,15 +1481,15 @@ __global__ void __launch_bounds__(kPcgNT) k_pcg_it(PcgArgs A) {
       a[1] = wn * un;
       a[2] = rv * rv;
     }
-    if (tid >= kNT)
+    if (kUpper && tid >= kNT)
 #pragma unroll
       for (int k = 0; k < 3; k++) s_hi[k][tid - kNT] = a[k];
     __syncthreads();
     if (tid < kNT)
 #pragma unroll
-      for (int k = 0; k < 3; k++) acc[k] = acc[k] + a[k] + s_hi[k][tid];
+      for (int k = 0; k < 3; k++) acc[k] = acc[k] + a[k] + (kUpper ? s_hi[k][tid] : 0.0);
   }
-  block_sum<3, kPcgNW>(acc, s_red);
+  block_sum<3, kWaves>(acc, s_red);
   if (tid == 0)
     for (int k = 0; k < 3; k++) A.part_out[3 * blockIdx.x + k] = acc[k];
 }
@@ -3843,7 +3849,10 @@ void launch_pcg_init(const PcgArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_pcg_init, dim3(capped_grid(a.nbx * a.nby)), dim3(kNT), 0, s, a);
 }
 void launch_pcg_it(const PcgArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_pcg_it, dim3(capped_grid(a.nbx * a.nby)), dim3(kPcgNT), 0, s, a);
+  const dim3 g(capped_grid(a.nbx * a.nby));
+  if (a.G.by <= kPcgTY / 2)
+    hipLaunchKernelGGL(k_pcg_it<kPcgTY / 2>, g, dim3(kTX * kPcgTY / 2), 0, s, a);
+  else hipLaunchKernelGGL(k_pcg_it<kPcgTY>, g, dim3(kTX * kPcgTY), 0, s, a);
 }
 void launch_pcg_finish(const PcgArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_pcg_finish, dim3(capped_grid(a.nbx * a.nby)), dim3(kNT), 0, s, a);
@@ -3853,12 +3862,13 @@ void launch_pcg_finish(const PcgArgs& a, hipStream_t s) {
 // tiles (one dimension: a wave per 64 cells; two: 256 threads per 64 x 8), while
 // an iteration takes less than as a launch.  One dimension: 1.2 us up to 64
 // cells, 1.4-1.6 to 256, 3.7 to 1024, against 6-9 (four cells per thread, to 4096:
-// 9.1-9.6 against 5.8-6.2); two: 1.5 us for one tile, 4.0 up to four, 5.9-7.2 up to
-// eight, against 6.1-9.
+// 9.1-9.6 against 4.7); two: 1.5 us for one tile, 4.0 up to four, 6.4-7.2 up to eight
+// against 7.6-8 (grids of at most four rows, whose launches take 5.0 us against 5.9
+// here, up to four).
 bool pcg_small_fits(const Geo& G) {
   if (G.by == 1) return G.bx <= 16 * kTX;
   const int nt = ((G.bx + kTX - 1) / kTX) * ((G.by + kPcgTY - 1) / kPcgTY);
-  return nt <= 8 && (G.bx + 2) * (G.by + 2) <= kPcgSmallPlane;
+  return nt <= (G.by > kPcgTY / 2 ? 8 : 4) && (G.bx + 2) * (G.by + 2) <= kPcgSmallPlane;
 }
 void launch_pcg_small(const PcgArgs& a, hipStream_t s) {
   const int nt = a.nbx * a.nby;
