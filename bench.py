@@ -401,7 +401,7 @@ def main():
         args.no_cpu = True  # a CPU step at 2048^2 takes about a minute; not sampled
         args.no_learned = True
     if args.gpus != 1:
-        print(json.dumps({"error": "this build runs on one GPU: one discharge per device; "
+        print(json.dumps({"error": "the library runs on one GPU: one discharge per device; "
                                    "multi-GPU sharding is a design note only",
                           "n_gpus": args.gpus}))
         sys.exit(2)

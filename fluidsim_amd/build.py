@@ -22,7 +22,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FC = os.environ.get("FC", "/opt/rocm/bin/amdflang")
 
 # -ffp-contract=off keeps the reference's rounding sequence (no FMA contraction);
-# packed FP32 instructions are disabled (they are unreliable on this pool).
+# packed FP32 instructions are disabled (some of their forms have given wrong results).
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]

@@ -525,8 +525,8 @@ int check_status(fs_handle* h) {
 }
 
 // Aggregation hierarchy: halve both axes until the coarsest level has at most
-// 64 cells (solved with its dense inverse).  Coarse planes: d (ghost 1), cx,
-// cy, r, x1, e (ghost 0).
+// kMgBottomMax cells (16, solved with its dense inverse).  Coarse planes: d
+// (ghost 1), cx, cy, r, x1, e (ghost 0).
 size_t mg_lds_first(const fs_handle* h);
 
 int build_mg(fs_handle* h) {
@@ -1124,7 +1124,7 @@ int lapl_solve_impl(fs_handle* h, int* lerr, fs_solve_stats* stats, int mode = 0
     // attached network the learned level gets a zero correction
     if (h->mg.size() < 2)
       return fail(FS_E_ARG,
-                  "learned solver: the grid has no coarse level (<= 64 cells, or 1-D)%s");
+                  "learned solver: the grid has no coarse level (<= 16 cells, or 1-D)%s");
     for (size_t l = lapl_coarse_levels(h); l < learned_level(h); l++)
       launch_mg_coarsen(mg_args(h, l), h->st);
     MgPcgArgs ia = mgpcg_args(h, 1);
@@ -1153,7 +1153,7 @@ int lapl_solve_impl(fs_handle* h, int* lerr, fs_solve_stats* stats, int mode = 0
       if (h->h_sc->done) break;
     }
   } else if (h->p.lapl_solver == 1 && h->mg.size() > 1) {
-    // multigrid-preconditioned PCG (grids of <= 64 cells use Jacobi-PCG)
+    // multigrid-preconditioned PCG (grids of <= 16 cells use Jacobi-PCG)
     int& mg_it = h->mg_it;
     int& mg_chunk = h->mg_chunk;
     if (mode != 2) {
@@ -2802,7 +2802,7 @@ int fs_ensemble_create(int32_t n, const fs_grid_desc* g, const fs_params* p, fs_
     E->m.push_back(h);
     if (h->mg.size() < 2) {
       ens_release(E);
-      return fail(FS_E_ARG, "ensemble member grid of <= 64 cells%s");
+      return fail(FS_E_ARG, "ensemble member grid of <= 16 cells%s");
     }
   }
   // the members' scalars move into one array so that a round reads them with
@@ -2941,7 +2941,7 @@ int fs_learn_samples(const fs_learn* n) { return n ? n->net.count : -1; }
 int fs_learn_harvest(fs_learn* n, fs_handle* h, int32_t* added) {
   if (!n || !h) return fail(FS_E_ARG, "null argument%s");
   if (h->mg.size() < 2)
-    return fail(FS_E_ARG, "the grid has no coarse level (<= 64 cells, or 1-D)%s");
+    return fail(FS_E_ARG, "the grid has no coarse level (<= 16 cells, or 1-D)%s");
   const MgLevel& lc = h->mg[learned_level(h)];
   if (lc.nx > n->net.W || lc.ny > n->net.H)
     return fail(FS_E_ARG, "learned level larger than the training grid%s");

@@ -1742,11 +1742,13 @@ __global__ void __launch_bounds__(NTH) k_pcg_small(PcgArgs A) {
 //   x1 = S r,  r_c = P^T (r - M x1)                                  [down]
 //   x2 = x1 + oc P e_c,  e = x2 + S^T (r - M x2)                     [up]
 // The post-smoother is the adjoint of the pre-smoother, so the cycle is a
-// symmetric positive definite operator and plain CG remains valid.  Levels
-// above 1024 cells are swept in tiles staged in LDS with a halo of four cells
-// (one per half-sweep), one down and one up kernel per level; the remaining
-// levels run inside one workgroup with their iterates in LDS, and the
-// coarsest (<= 64 cells) is solved with a dense inverse.
+// symmetric positive definite operator and plain CG remains valid.  Level 0
+// and those above kMgLdsCells cells (4096) are swept in tiles with a halo of four
+// cells (one per half-sweep), the equations in registers and the iterates in
+// LDS: a down kernel per level, and an up kernel per level or per up to three of
+// them; the remaining levels run inside one workgroup with their iterates in
+// LDS, and the coarsest (at most kMgBottomMax cells, 16) is solved with a dense
+// inverse.
 
 
 // A kernel argument is loaded where it is first used; a kernel that first
@@ -2225,6 +2227,10 @@ __device__ __forceinline__ double uniform(double v) {
 // workgroup, where more waves in flight count) the loads follow the test; the
 // CG form loads its tiles after the reduction, and u, p and x behind the
 // residual's update, which keeps it at 128 VGPRs, four workgroups per CU.
+// kEarly's 191 leave it two, 512 tiles at once: up to there it is the faster,
+// between 513 and 1024 tiles, which it also takes, the other form would be
+// (kernel 15.8 and 13.3 us at 600^2, 19.8 and 16.6 at 1024 x 512; an iteration
+// 56.9 and 53.7, 63.4 and 58.5).
 template <int kInstance, bool kCg, bool kEarly>
 __device__ __forceinline__ void mg_down_body(const MgArgs& A, int band0, int band1, int nb) {
   __shared__ GsX s;

@@ -663,9 +663,11 @@ __global__ void k_nn_store(MgLevel L, int H, int W, float* out) {
 // split: one output tile per wave, the tiles along the grid's y (the network
 // application, and the layers of a batch with at most kSplitPixels pixels);
 // otherwise every tile in each wave.  Measured at batch 16: the 64-channel
-// layers at 8 x 8 (1024 pixels) 22.6 -> 10 us, 48 channels at 16 x 16 9.1 -> 6 us,
-// 32 channels at 32 x 32 (16384 pixels) 8.4 -> 6.8 us; at 64 x 64 the layers
-// have one or three tiles and fill the chip either way.
+// layers at 8 x 8 (1024 pixels) 22.6 -> 10 us, 48 channels at 16 x 16 9.1 -> 6 us;
+// at 64 x 64 the layers have one or three tiles and fill the chip either way.
+// A training step of 64 x 64 samples with the limit at 0, 4096, 16384 and 65536
+// pixels: batch 4 327, 251, 250, 250 us; 8 343, 276, 268, 268; 16 385, 321, 331, 331;
+// 32 510, 473, 474, 487; 64 775, 738, 768, 797.
 constexpr int kSplitPixels = 16384;
 int launch_conv(const ConvArgs& a, hipStream_t st, bool split = false) {
   const int total = a.N * a.H * a.W;

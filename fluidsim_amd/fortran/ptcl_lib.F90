@@ -48,7 +48,7 @@ contains
   end subroutine
 
   ! *** ptcl_step(g, ph, Em) (ptcl_lib.F90:32-97) ***
-  ! Em is the microwave field of em_lib, which this build does not carry: it
+  ! Em is the microwave field of em_lib, which this library does not carry: it
   ! must be zero.
   subroutine ptcl_step(g, ph, Em)
     type(grid), intent(inout) :: g

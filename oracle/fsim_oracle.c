@@ -1,7 +1,7 @@
 /*
  * fsim_oracle.c -- CPU FP64 restatement of the fluidsim plasma-transport path.
  *
- * TEST INFRASTRUCTURE ONLY: the checker for libfsim_hip.so and the timed CPU
+ * TEST INFRASTRUCTURE ONLY: the oracle of libfsim_hip.so's tests and the timed CPU
  * baseline.  Nothing in the product links or loads this file.
  *
  * Every routine follows one reference routine statement by statement, keeping

@@ -1,7 +1,7 @@
 /*
  * fsim_oracle.h -- CPU FP64 restatement of the fluidsim plasma-transport hot path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the checker for the HIP product
+ * TEST INFRASTRUCTURE ONLY.  This library is the oracle of the HIP library's tests
  * (libfsim_hip.so) and the timed CPU baseline.  Only tests/, the smoke() entry
  * and bench.py's cpu_baseline leg may load it.  The product never links it.
  *
