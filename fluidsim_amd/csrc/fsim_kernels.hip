@@ -3734,9 +3734,9 @@ __global__ void __launch_bounds__(1024) kb_mg_coarse_setup(const MgCycleArgs* __
 // 245 us), four of the up kernels.  A workgroup tests a member's state and
 // reduces its partial sums once for all its bands of that member, and what a
 // launch costs follows the members on the list.  Measured on the 256-member
-// sweep (14 327 bands on the finest level): down 245 us, up 150 us with every
-// member iterating (a workgroup per band: 310 and 185 us), 12 and 8 us for the
-// last few members (18 and 13 us), 3 us for none (14 us each).
+// sweep (14 327 bands on the finest level): down 224-256 us, up 137-159 us with
+// every member iterating (a workgroup per band: 310 and 185 us), 12 and 8 us for
+// the last few members (18 and 13 us), 2.4 us for none (14 us each).
 constexpr int kListDown = 3 * 256, kListUp = 4 * 256;
 template <class F>
 __device__ __forceinline__ void ens_bands(const EnsList& l, const EnsMap& m, F body) {
